@@ -1,256 +1,195 @@
 // Grouped dequant-GEMV over the selected experts (kernel family 2) and the
-// fused weighted combine (family 4), one token.
+// fused weighted combine (family 4), one token, any shape the stage takes.
 //
 // Replaces graph B of src/run_moe_stream.cpp:431-438 (per expert:
 // mul_mat(gate), mul_mat(up), mul(silu(g), u), mul_mat(down), concat) plus the
 // shared expert of src/run_qwen35.cpp:658-666, and the host combine at
 // src/run_moe_stream.cpp:447 / src/run_qwen35.cpp:675-676.
 //
-// Both kernels stage the weight bytes they own into LDS with 16-byte loads of
-// the contiguous GGUF byte stream (a run of whole rows of one expert matrix is
-// contiguous), quantise their activation to Q8_K in LDS exactly as the CPU path
-// does, then give each lane one (matrix, row, super-block) integer dot.  The
-// per-block fp32 terms go back through LDS and one lane per row adds them in
-// block order, so g, u and y match the CPU restatement bit for bit given the
-// same activation.
+// Both kernels are bound by the weight stream.  A wave streams 8 rows from
+// memory into registers (rowstream.h), the first blocks' loads issued before
+// the activation's Q8_K blocks are formed in LDS, so the formation and the
+// barrier behind it pass while they fly.  Against copying whole tiles through
+// registers into LDS first (a few loads in flight per CU): 8 of 64 experts of
+// 4096 x 1536 (Q4_K, Q6_K down), gate/up 33.5 -> 15.6 us a launch (56.6 MB,
+// 3.6 TB/s), down 65.2 -> 15.4 us (41.3 MB, 2.7 TB/s).
 #include "kernels.h"
+#include "lds_dma.h"
 #include "qblocks.h"
+#include "rowstream.h"
 #include "wave.h"
 
 namespace hoard {
 
 namespace {
 
-constexpr int kThreads = 256;
-constexpr int kGateUpRows = 16;
-
-__device__ __forceinline__ int block_bytes_dev(int type) { return kquant_block_bytes(type); }
-
-template <class P>
-__device__ __forceinline__ void *align16(P *p) {
-    return reinterpret_cast<void *>((reinterpret_cast<uintptr_t>(p) + 15) & ~(uintptr_t)15);
-}
-
-// LDS bytes reserved for a staged run of `nbytes` starting at any address.
-__host__ __device__ __forceinline__ size_t stage_region(size_t nbytes) {
-    return (nbytes + 32 + 15) & ~(size_t)15;
-}
-
-// Copy [src, src+nbytes) into LDS starting at dst + (src & 15) with aligned
-// 16-byte loads; returns that offset.  Reads up to 15 bytes past the end,
-// which device allocations keep as padding.
-__device__ __forceinline__ int stage_issue(uint8_t *dst, const uint8_t *src, size_t nbytes) {
-    const uintptr_t a = reinterpret_cast<uintptr_t>(src);
-    const uintptr_t a0 = a & ~(uintptr_t)15;
-    const int n16 = (int)((a + nbytes + 15 - a0) >> 4);
-    const uint4 *s = reinterpret_cast<const uint4 *>(a0);
-    uint4 *d = reinterpret_cast<uint4 *>(dst);
-#pragma unroll 8
-    for (int i = threadIdx.x; i < n16; i += kThreads) d[i] = s[i];
-    return (int)(a - a0);
-}
+constexpr int kWaveRows = 8;   // rows a wave streams, one 8-lane group each
+constexpr size_t kMaxLds = 163840 - 2048;  // dynamic LDS of a workgroup, beside the static words
 
 __device__ __forceinline__ size_t row_bytes(int type, int cols) {
     return (size_t)(cols / QK) * (size_t)kquant_block_bytes(type);
 }
 
-__device__ __forceinline__ void terms_dyn(int type, const uint8_t *blk, const Q8Block &x, float &tm,
-                                          float &tn) {
-    switch (type) {
-    case kTypeQ4K: q4k_block_terms(blk, x, tm, tn); break;
-    case kTypeQ5K: q5k_block_terms(blk, x, tm, tn); break;
-    case kTypeQ3K: q3k_block_terms(blk, x, tm, tn); break;
-    default: q6k_block_terms(blk, x, tm, tn); break;
+// Q8_K of blocks first, first + step, ... below end of x into q, by one wave.
+// load() issues the loads of the first K blocks; the rest are loaded one by
+// one as the blocks are formed (behind whatever the wave loaded in between).
+// One quantiser in a loop that shifts the loaded blocks down: unrolled K
+// times it was most of a kernel's code.  x is 4-byte aligned.
+template <int K>
+struct WaveQuant {
+    f32x4_a4 v[K];
+    __device__ __forceinline__ void load(const float *x, int first, int end, int step) {
+#pragma unroll
+        for (int i = 0; i < K; ++i) get(i, x, min(first + i * step, end - 1));
+    }
+    __device__ __forceinline__ void get(int i, const float *x, int b) {
+        v[i] = *reinterpret_cast<const f32x4_a4 *>(x + (size_t)b * QK + 4 * (threadIdx.x & 63));
+    }
+    __device__ __forceinline__ void form(const float *x, Q8L *q, int first, int end, int step) {
+#pragma unroll 1
+        for (int b = first; b < end; b += step) {
+            const float w[4] = {v[0][0], v[0][1], v[0][2], v[0][3]};
+#pragma unroll
+            for (int i = 0; i + 1 < K; ++i) v[i] = v[i + 1];
+            if (b + K * step < end) get(K - 1, x, b + K * step);
+            wave_quantize_q8l_regs(w, q + b);
+        }
+    }
+};
+
+// The dot of the lane group's row (row grp of the 8 at base) with q; prep()
+// runs once the rows' first loads are issued.
+template <int T, class P>
+__device__ __forceinline__ float stream_row_t(const uint8_t *base, const Q8L *q, int nb, P prep) {
+    const int lane = threadIdx.x & 63, t = lane & 7;
+    const uint32_t off = (uint32_t)(lane >> 3) * (uint32_t)(nb * QType<T>::bytes);
+    RowStream<T> rs;
+    rs.begin(base, off, nb, t);
+    prep();
+    return rs.finish(base, off, q, nb, t);
+}
+// T: the type of every matrix the kernel meets, or 0 where they differ (type
+// is the same in every lane of the wave).
+template <int T, class P>
+__device__ __forceinline__ float stream_row(int type, const uint8_t *base, const Q8L *q, int nb, P prep) {
+    if constexpr (T != 0) {
+        return stream_row_t<T>(base, q, nb, prep);
+    } else {
+        switch (type) {
+        case kTypeQ4K: return stream_row_t<kTypeQ4K>(base, q, nb, prep);
+        case kTypeQ5K: return stream_row_t<kTypeQ5K>(base, q, nb, prep);
+        case kTypeQ3K: return stream_row_t<kTypeQ3K>(base, q, nb, prep);
+        default: return stream_row_t<kTypeQ6K>(base, q, nb, prep);
+        }
     }
 }
 
-__device__ __forceinline__ float row_sum_dyn(int type, const float2 *t, int nb) {
-    float acc = 0.0f, accm = 0.0f;
-    for (int b = 0; b < nb; ++b) {
-        acc = acc + t[b].x;
-        accm = accm + t[b].y;
-    }
-    return kquant_has_min(type) ? acc - accm : acc;
-}
-
-__device__ __forceinline__ float silu(float x) { return x / (1.0f + expf(-x)); }
-
 // ---------------------------------------------------------------------------
-// gate/up + SwiGLU.  grid = (rows_max / R, k + has_shared); block = 256; R
-// rows of gate and of up per workgroup (fewer for wide rows, so they fit LDS).
+// gate/up + SwiGLU.  grid = (rows_max / R, k + has_shared, plus a workgroup row
+// for the shared expert's gate); block = 64 * R / 4: R / 8 waves stream the
+// gate rows and R / 8 the up rows.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void gateup_kernel(GateUpArgs a, int R) {
+template <int T>
+__global__ __launch_bounds__(512) void gateup_kernel(GateUpArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
+    __shared__ float gu[64];
+    const int wave = wave_index(), lane = threadIdx.x & 63, t = lane & 7, grp = lane >> 3;
+    const int nw = (int)(blockDim.x >> 6), R = nw / 2 * kWaveRows;
     const int j = blockIdx.y;
     const bool shared = j >= a.k;
-    const MatDesc G = shared ? a.sh_gate : a.gate;
-    const MatDesc U = shared ? a.sh_up : a.up;
-    const int rows = G.rows;
+    if (j > a.k) {
+        // sigmoid gate of the shared expert: f32 dot in the router's lane order
+        if (blockIdx.x == 0 && threadIdx.x < 32) {
+            float acc = 0.0f;
+#pragma unroll 32
+            for (int i = 0; i < a.n_embd; i += 32) acc = fmaf(a.sh_gate_inp[i + lane], a.fx[i + lane], acc);
+            acc = acc + __shfl_xor(acc, 16);
+            acc = row16_ggml_fold(acc);
+            if (lane == 0) a.sgate[0] = 1.0f / (1.0f + expf(-acc));
+        }
+        return;
+    }
+    const bool up = wave >= nw / 2;
+    const MatDesc &W = shared ? (up ? a.sh_up : a.sh_gate) : (up ? a.up : a.gate);
     const int r0 = blockIdx.x * R;
-    if (r0 >= rows) return;
+    if (r0 >= W.rows) return;
     const int nb = a.n_embd / QK;
     float *hout = a.h + (size_t)j * a.hstride + r0;
-
-    if (shared && blockIdx.x == 0 && threadIdx.x < 32) {
-        // sigmoid gate of the shared expert: f32 dot in the router's lane order
-        const int l = threadIdx.x;
-        float acc = 0.0f;
-        for (int i = 0; i < a.n_embd; i += 32) acc = fmaf(a.sh_gate_inp[i + l], a.fx[i + l], acc);
-        acc = acc + __shfl_xor(acc, 16);
-        acc = acc + __shfl_xor(acc, 8);
-        acc = acc + __shfl_xor(acc, 4);
-        acc = acc + __shfl_xor(acc, 1);
-        acc = acc + __shfl_xor(acc, 2);
-        if (l == 0) a.sgate[0] = 1.0f / (1.0f + expf(-acc));
-    }
-
-    const uint8_t *gsrc, *usrc;
-    if (shared) {
-        gsrc = G.base;
-        usrc = U.base;
-    } else {
+    const uint8_t *src = W.base;
+    if (!shared) {
         const int id = a.ids[j];
-        if (id < 0 || id >= G.n_ids) {  // invalid id: poison this expert's rows
+        if (id < 0 || id >= W.n_ids) {  // invalid id: poison this expert's rows
             if (threadIdx.x < R) hout[threadIdx.x] = __builtin_nanf("");
             return;
         }
-        gsrc = G.base + (size_t)id * G.stride;
-        usrc = U.base + (size_t)id * U.stride;
+        src += (size_t)id * W.stride;
     }
-    const size_t rbg = row_bytes(G.type, a.n_embd), rbu = row_bytes(U.type, a.n_embd);
-    gsrc += (size_t)r0 * rbg;
-    usrc += (size_t)r0 * rbu;
-
-    uint8_t *lds_g = smem;
-    uint8_t *lds_u = lds_g + stage_region(R * rbg);
-    Q8Block *qx = reinterpret_cast<Q8Block *>(lds_u + stage_region(R * rbu));
-    float2 *terms = reinterpret_cast<float2 *>(align16(qx + nb));
-
-    const int og = stage_issue(lds_g, gsrc, R * rbg);
-    const int ou = stage_issue(lds_u, usrc, R * rbu);
-
-    const int wave = wave_index();
-    for (int b = wave; b < nb; b += kThreads / 64) wave_quantize_q8k(a.fx + b * QK, &qx[b]);
-    __syncthreads();
-
-    const int per_mat = R * nb;
-    for (int u = threadIdx.x; u < 2 * per_mat; u += kThreads) {
-        const int mat = u / per_mat, rem = u - mat * per_mat;
-        const int row = rem / nb, b = rem - row * nb;
-        float tm, tn;
-        if (mat == 0)
-            terms_dyn(G.type, lds_g + og + row * rbg + b * block_bytes_dev(G.type), qx[b], tm, tn);
-        else
-            terms_dyn(U.type, lds_u + ou + row * rbu + b * block_bytes_dev(U.type), qx[b], tm, tn);
-        terms[u] = make_float2(tm, tn);
-    }
-    __syncthreads();
-
+    Q8L *q8 = reinterpret_cast<Q8L *>(smem);
+    WaveQuant<4> xq;
+    xq.load(a.fx, wave, nb, nw);
+    const int w0 = (up ? wave - nw / 2 : wave) * kWaveRows;  // the wave's first row of the R
+    const float v = stream_row<T>(W.type, src + (size_t)(r0 + w0) * row_bytes(T ? T : W.type, a.n_embd), q8, nb, [&]() {
+        xq.form(a.fx, q8, wave, nb, nw);
+        lds_barrier();
+    });
+    if (t == 0) gu[(up ? R : 0) + w0 + grp] = v;
+    lds_barrier();
     if (threadIdx.x < R) {
-        const int r = threadIdx.x;
-        const float g = row_sum_dyn(G.type, terms + r * nb, nb);
-        const float uu = row_sum_dyn(U.type, terms + per_mat + r * nb, nb);
-        hout[r] = silu(g) * uu;
+        const float g = gu[threadIdx.x], u = gu[R + threadIdx.x];
+        hout[threadIdx.x] = g / (1.0f + expf(-g)) * u;
     }
 }
 
 // ---------------------------------------------------------------------------
-// down + combine.  grid = n_embd / rd; block = 256.
+// down + combine.  grid = n_embd / (8 G) workgroups of G waves a unit (the k
+// experts, then the shared one; several units a wave where they are more than
+// 16 waves): wave u G + s streams rows [8 s, 8 s + 8) of unit u.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void down_combine_kernel(DownArgs a, int rd) {
+template <int T>
+__global__ __launch_bounds__(1024) void down_combine_kernel(DownArgs a, int G) {
     extern __shared__ __align__(16) uint8_t smem[];
-    const int d0 = blockIdx.x * rd;
+    __shared__ float ys[17 * 4 * kWaveRows];
+    __shared__ int bad;
+    const int wave = wave_index(), lane = threadIdx.x & 63, t = lane & 7, grp = lane >> 3;
+    const int nw = (int)(blockDim.x >> 6), R = kWaveRows * G;
+    const int d0 = blockIdx.x * R;
     const int k = a.k;
     const bool has_sh = a.sh_down.base != nullptr;
-    const int nseg = k + (has_sh ? 1 : 0);
+    const int nu = k + (has_sh ? 1 : 0);
     const int nbh = a.down.cols / QK;
-    const int nbs = has_sh ? a.sh_down.cols / QK : 0;
-    const size_t rbd = row_bytes(a.down.type, a.down.cols);
-    const size_t rbs = has_sh ? row_bytes(a.sh_down.type, a.sh_down.cols) : 0;
-    const size_t reg_d = stage_region(rd * rbd), reg_s = has_sh ? stage_region(rd * rbs) : 0;
-
-    uint8_t *lds_w = smem;
-    Q8Block *qh = reinterpret_cast<Q8Block *>(lds_w + k * reg_d + reg_s);
-    const int nq = k * nbh + nbs;
-    float2 *terms = reinterpret_cast<float2 *>(align16(qh + nq));
-    __shared__ int offs[17];
-    __shared__ int bad;
-    __shared__ float wj[16];
-
+    Q8L *q8h = reinterpret_cast<Q8L *>(smem);  // unit u's blocks at u * nbh
     if (threadIdx.x == 0) bad = 0;
-    if (threadIdx.x < k) wj[threadIdx.x] = a.w[threadIdx.x];
-    __syncthreads();
-    for (int s = 0; s < nseg; ++s) {
-        const uint8_t *src;
-        size_t nbytes;
-        uint8_t *dst;
-        if (s < k) {
-            const int id = a.ids[s];
-            if (id < 0 || id >= a.down.n_ids) {
-                if (threadIdx.x == 0) bad = 1;
-                continue;
-            }
-            src = a.down.base + (size_t)id * a.down.stride + (size_t)d0 * rbd;
-            nbytes = rd * rbd;
-            dst = lds_w + s * reg_d;
-        } else {
-            src = a.sh_down.base + (size_t)d0 * rbs;
-            nbytes = rd * rbs;
-            dst = lds_w + k * reg_d;
-        }
-        const int o = stage_issue(dst, src, nbytes);
-        if (threadIdx.x == 0) offs[s] = o;
+    lds_barrier();
+    for (int w = wave; w < nu * G; w += nw) {
+        const int u = w / G, s = w - u * G;
+        const MatDesc &W = u < k ? a.down : a.sh_down;
+        const int nb = W.cols / QK;
+        const float *h = a.h + (size_t)u * a.hstride;
+        const int id = u < k ? a.ids[u] : 0;
+        const bool ok = u >= k || (id >= 0 && id < W.n_ids);
+        if (!ok) bad = 1;
+        Q8L *q = q8h + (size_t)u * nbh;
+        WaveQuant<T == 0 ? 2 : 8> hq;
+        hq.load(h, s, nb, G);
+        const uint8_t *rows = W.base + (size_t)(ok ? id : 0) * W.stride +
+                              (size_t)(d0 + kWaveRows * s) * row_bytes(T ? T : W.type, W.cols);
+        const float y = stream_row<T>(W.type, rows, q, nb, [&]() {
+            hq.form(h, q, s, nb, G);
+            // one wave a unit: its blocks are its own; several: they form them together
+            if (G > 1)
+                lds_barrier();
+            else
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        });
+        if (t == 0) ys[u * R + kWaveRows * s + grp] = y;
     }
-
-    const int wave = wave_index();
-    for (int q = wave; q < nq; q += kThreads / 64) {
-        const int j = q < k * nbh ? q / nbh : k;
-        const int b = q < k * nbh ? q - j * nbh : q - k * nbh;
-        wave_quantize_q8k(a.h + (size_t)j * a.hstride + b * QK, &qh[q]);
-    }
-    __syncthreads();
-    if (bad) {
-        if (threadIdx.x < rd) a.out[d0 + threadIdx.x] = __builtin_nanf("");
-        return;
-    }
-
-    const int routed_units = k * rd * nbh;
-    const int units = routed_units + rd * nbs;
-    for (int u = threadIdx.x; u < units; u += kThreads) {
-        float tm, tn;
-        if (u < routed_units) {
-            const int j = u / (rd * nbh), rem = u - j * rd * nbh;
-            const int row = rem / nbh, b = rem - row * nbh;
-            terms_dyn(a.down.type,
-                      lds_w + j * reg_d + offs[j] + row * rbd + b * block_bytes_dev(a.down.type),
-                      qh[j * nbh + b], tm, tn);
-        } else {
-            const int v = u - routed_units;
-            const int row = v / nbs, b = v - row * nbs;
-            terms_dyn(a.sh_down.type,
-                      lds_w + k * reg_d + offs[k] + row * rbs + b * block_bytes_dev(a.sh_down.type),
-                      qh[k * nbh + b], tm, tn);
-        }
-        terms[u] = make_float2(tm, tn);
-    }
-    __syncthreads();
-
-    if (threadIdx.x < rd) {
-        const int r = threadIdx.x;
+    lds_barrier();
+    if (threadIdx.x < R) {
+        const int r = threadIdx.x, d = d0 + r;
         float acc = 0.0f;
-        for (int j = 0; j < k; ++j) {
-            const float y = row_sum_dyn(a.down.type, terms + (j * rd + r) * nbh, nbh);
-            acc = acc + wj[j] * y;
-        }
-        const int d = d0 + r;
-        float o;
-        if (has_sh) {
-            const float ysh = row_sum_dyn(a.sh_down.type, terms + routed_units + r * nbs, nbs);
-            o = (acc + ysh * a.sgate[0]) + a.res[d];
-        } else {
-            o = acc + a.res[d];
-        }
-        a.out[d] = o;
+        for (int j = 0; j < k; ++j) acc = acc + a.w[j] * ys[j * R + r];
+        float o = has_sh ? (acc + ys[k * R + r] * a.sgate[0]) + a.res[d] : acc + a.res[d];
+        a.out[d] = bad ? __builtin_nanf("") : o;
     }
 }
 
@@ -258,46 +197,46 @@ __global__ __launch_bounds__(kThreads) void down_combine_kernel(DownArgs a, int 
 
 size_t block_bytes(int type) { return (size_t)kquant_block_bytes(type); }
 
-static size_t host_row_bytes(int type, int cols) { return (size_t)(cols / QK) * block_bytes(type); }
-
 hipError_t launch_gateup(const GateUpArgs &a, hipStream_t s) {
-    const int nb = a.n_embd / QK;
-    int rows_max = a.gate.rows;
-    if (a.sh_gate.base) rows_max = rows_max > a.sh_gate.rows ? rows_max : a.sh_gate.rows;
-    // the most rows per workgroup (16 down to 1) whose staged tiles fit 64 KiB of LDS
-    for (int R = kGateUpRows; R >= 1; R >>= 1) {
-        size_t need = stage_region(R * host_row_bytes(a.gate.type, a.n_embd)) +
-                      stage_region(R * host_row_bytes(a.up.type, a.n_embd));
-        if (a.sh_gate.base) {
-            const size_t ns = stage_region(R * host_row_bytes(a.sh_gate.type, a.n_embd)) +
-                              stage_region(R * host_row_bytes(a.sh_up.type, a.n_embd));
-            need = need > ns ? need : ns;
-        }
-        const size_t lds = need + nb * sizeof(Q8Block) + 16 + 2 * (size_t)R * nb * sizeof(float2);
-        if (lds > 65536 || rows_max % R) continue;
-        dim3 grid((unsigned)(rows_max / R), (unsigned)(a.k + (a.sh_gate.base ? 1 : 0)));
-        hipLaunchKernelGGL(gateup_kernel, grid, dim3(kThreads), lds, s, a, R);
-        return hipGetLastError();
-    }
-    return hipErrorInvalidConfiguration;
+    const size_t lds = (size_t)(a.n_embd / QK) * sizeof(Q8L);
+    if (lds > kMaxLds) return hipErrorInvalidConfiguration;
+    const bool sh = a.sh_gate.base != nullptr;
+    const int rows = sh && a.sh_gate.rows > a.gate.rows ? a.sh_gate.rows : a.gate.rows;
+    const int units = a.k + (sh ? 1 : 0);
+    // eight waves share one formation of Q8_K(fx) where that still gives every
+    // CU a workgroup; fewer rows take four, for twice the workgroups
+    const int waves = rows * units >= 8192 ? 8 : 4;
+    const dim3 grid((unsigned)(rows / (4 * waves)), (unsigned)(units + (sh ? 1 : 0)));
+    const int T = a.gate.type;
+    const bool one = a.up.type == T && (!sh || (a.sh_gate.type == T && a.sh_up.type == T));
+    auto *fn = !one             ? gateup_kernel<0>
+               : T == kTypeQ4K ? gateup_kernel<kTypeQ4K>
+               : T == kTypeQ5K ? gateup_kernel<kTypeQ5K>
+               : T == kTypeQ3K ? gateup_kernel<kTypeQ3K>
+                               : gateup_kernel<kTypeQ6K>;
+    hipLaunchKernelGGL(fn, grid, dim3(64 * waves), lds, s, a);
+    return hipGetLastError();
 }
 
 hipError_t launch_down_combine(const DownArgs &a, hipStream_t s) {
     const bool has_sh = a.sh_down.base != nullptr;
-    const int nbh = a.down.cols / QK, nbs = has_sh ? a.sh_down.cols / QK : 0;
-    for (int rd = 8; rd >= 1; rd >>= 1) {
-        if (a.n_embd % rd) continue;
-        const size_t reg_d = stage_region(rd * host_row_bytes(a.down.type, a.down.cols));
-        const size_t reg_s = has_sh ? stage_region(rd * host_row_bytes(a.sh_down.type, a.sh_down.cols)) : 0;
-        const int nq = a.k * nbh + nbs;
-        const size_t lds = a.k * reg_d + reg_s + nq * sizeof(Q8Block) + 16 +
-                           (size_t)(a.k * rd * nbh + rd * nbs) * sizeof(float2);
-        if (lds > 65536) continue;
-        hipLaunchKernelGGL(down_combine_kernel, dim3((unsigned)(a.n_embd / rd)), dim3(kThreads), lds, s,
-                           a, rd);
-        return hipGetLastError();
-    }
-    return hipErrorInvalidConfiguration;
+    const int nu = a.k + (has_sh ? 1 : 0), nbh = a.down.cols / QK, nbs = has_sh ? a.sh_down.cols / QK : 0;
+    const size_t lds = (size_t)(a.k * nbh + nbs) * sizeof(Q8L);
+    if (lds > kMaxLds) return hipErrorInvalidConfiguration;
+    // several waves a unit (up to 16 in all) share the formation of its Q8_K(h),
+    // as long as every CU has a workgroup: 15.5 against 16.1 us at 4096 rows of
+    // 8 units with two
+    int G = 1;
+    while (G < 4 && 2 * G * nu <= 16 && a.n_embd / (kWaveRows * 2 * G) >= 256) G *= 2;
+    const int waves = nu * G < 16 ? nu * G : 16;
+    const int T = a.down.type;
+    auto *fn = has_sh && a.sh_down.type != T ? down_combine_kernel<0>
+               : T == kTypeQ4K               ? down_combine_kernel<kTypeQ4K>
+               : T == kTypeQ5K               ? down_combine_kernel<kTypeQ5K>
+               : T == kTypeQ3K               ? down_combine_kernel<kTypeQ3K>
+                                             : down_combine_kernel<kTypeQ6K>;
+    hipLaunchKernelGGL(fn, dim3((unsigned)(a.n_embd / (kWaveRows * G))), dim3(64 * waves), lds, s, a, G);
+    return hipGetLastError();
 }
 
 }  // namespace hoard

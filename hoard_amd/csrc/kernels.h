@@ -8,7 +8,7 @@
 
 namespace hoard {
 
-// Router tail for M tokens (grid.y = token).  When `xin_is_residual`, fx is
+// Router and its tail for one token (M = 1).  When `xin_is_residual`, fx is
 // rms_norm(xin, eps) and is also written to fx_out; otherwise xin is fx.
 struct RouterArgs {
     const float *xin;      // [M][n]
