@@ -23,7 +23,7 @@ namespace {
 constexpr int kTile = 16;                   // weight rows per MFMA tile
 constexpr int kMaxTok = kBatchedMaxTokens;  // token places per expert group
 constexpr int kCols = 16;                   // token columns per MFMA tile
-constexpr int kMfmaMinTokens = 12;          // smallest expert group computed on MFMA
+constexpr int kMfmaMinTokens = 6;          // smallest expert group computed on MFMA
 constexpr int kXChunk = 1;                  // tokens of Q8_K x staged in LDS at a time
 constexpr int kMaxExperts = 1024;
 static_assert(sizeof(Q8L) == kQ8LBytes, "Q8_K block size shared with the host");
@@ -72,6 +72,10 @@ struct GroupLds {
     int total;
 };
 
+__device__ void group_units(const BatchedArgs &a, GroupLds &g);
+
+// a.unit != 0: the groups go out as sorted pairs and work units, as those of a
+// prefill-sized batch do (a group's mask gives its size and each pair's place).
 __device__ void group_by_expert(const BatchedArgs &a, GroupLds &g, const int *ysrc = nullptr,
                                 const int *bad = nullptr) {
     unsigned *mask = g.mask;
@@ -79,6 +83,7 @@ __device__ void group_by_expert(const BatchedArgs &a, GroupLds &g, const int *ys
     int &wave_total = g.total;
     const int tid = threadIdx.x, nt = blockDim.x, E = a.n_ids, P = a.M * a.k;
     for (int e = tid; e < E; e += nt) mask[e] = 0u;
+    if (a.sh && tid == 0) mask[E] = a.M < 32 ? (1u << a.M) - 1u : ~0u;  // the shared expert: every token
     __syncthreads();
     for (int p = tid; p < P; p += nt) {
         if (!pair_computed(a, ysrc, bad, p)) continue;
@@ -87,6 +92,26 @@ __device__ void group_by_expert(const BatchedArgs &a, GroupLds &g, const int *ys
         atomicOr(&mask[e], 1u << (p / a.k));
     }
     __syncthreads();
+    if (a.unit) {
+        for (int e = tid; e < E + a.sh; e += nt) g.cnt[e] = (unsigned)__popc(mask[e]);
+        __syncthreads();
+        if (tid < 64) group_units(a, g);
+        __syncthreads();
+        const int kk = a.k + a.sh;
+        for (int p = tid; p < a.M * kk; p += nt) {
+            const int t = p / kk, j = p - t * kk;
+            int e = E;
+            if (j < a.k) {
+                if (!pair_computed(a, ysrc, bad, t * a.k + j)) continue;
+                e = __hip_atomic_load(a.sel + t * a.k + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (e < 0 || e >= E) e = 0;
+            }
+            const int pos = g.base[e] + __popc(mask[e] & ((1u << t) - 1u));
+            a.ptok[pos] = t;
+            a.pslot[pos] = j;
+        }
+        return;
+    }
     if (tid < 64) {
         // ascending prefix count of used experts: lane owns a contiguous run of experts
         const int lane = tid, per = (E + 63) / 64, e0 = lane * per;
@@ -155,7 +180,7 @@ __device__ void group_units(const BatchedArgs &a, GroupLds &g) {
         for (int e = e0; e < e0 + per && e < E; ++e) {
             const int c = (int)g.cnt[e];
             cg += c ? 1 : 0;
-            cu += (c + kUnitTokens - 1) / kUnitTokens;
+            cu += (c + a.unit - 1) / a.unit;
             cp += c;
         }
         int ig = cg, iu = cu, ip = cp;
@@ -177,8 +202,8 @@ __device__ void group_units(const BatchedArgs &a, GroupLds &g) {
                 a.uexp[gi] = e;
                 a.ucount[gi] = c;
                 a.goff[gi] = pi;
-                for (int s0 = 0; s0 < c; s0 += kUnitTokens, ++ui)
-                    *reinterpret_cast<int4 *>(a.units + 4 * ui) = make_int4(e, pi + s0, min(kUnitTokens, c - s0), 0);
+                for (int s0 = 0; s0 < c; s0 += a.unit, ++ui)
+                    *reinterpret_cast<int4 *>(a.units + 4 * ui) = make_int4(e, pi + s0, min(a.unit, c - s0), 0);
                 ++gi;
             }
             pi += c;
@@ -198,7 +223,7 @@ __device__ void group_units(const BatchedArgs &a, GroupLds &g) {
 // Grouping of a prefill-sized batch (all threads of one workgroup): the
 // computed (token, slot) pairs sorted by (expert, token) into ptok / pslot, the
 // groups (used experts in ascending order: uexp, ucount, goff) and the work
-// units (at most kUnitTokens pairs of one group each).  pe[p] (in LDS) is the
+// units (at most a.unit pairs of one group each).  pe[p] (in LDS) is the
 // expert of pair p, or -1 for a pair that joins no group.  The order within an
 // expert comes from chunks of at most 32 tokens taken in token order: a pair's
 // place is its expert's running base plus the tokens of its chunk before it
@@ -231,6 +256,16 @@ __device__ void group_large(const BatchedArgs &a, GroupLds &g, const int *pe, in
         for (int e = tid; e < E; e += nt) g.base[e] += __popc(g.mask[e]);
         __syncthreads();
     }
+}
+
+// Q8_K of a block of fx with the sums the expert kernels of this call read.
+__device__ __forceinline__ void quantize_x(const BatchedArgs &a, const float *x, Q8L *out) {
+    if (a.unit && a.gu_type == kTypeQ3K)
+        wave_quantize_q8l<kSums16>(x, out);
+    else if (a.unit)
+        wave_quantize_q8l<kSums32>(x, out);
+    else
+        wave_quantize_q8l(x, out);
 }
 
 template <int R>
@@ -305,7 +340,7 @@ __global__ __launch_bounds__(256) void route_kernel(BatchedArgs a) {
         }
         // Q8_K of fx: workgroup i of a token group quantises blocks i, i + gridDim.x, ...
         // of its tokens, so every block is formed whatever the expert count (grid width)
-        for (int b = blockIdx.x; b < nb; b += gridDim.x) wave_quantize_q8l(x + b * QK, q8(a.q8x) + (size_t)t * nb + b);
+        for (int b = blockIdx.x; b < nb; b += gridDim.x) quantize_x(a, x + b * QK, q8(a.q8x) + (size_t)t * nb + b);
     }
     // Completion protocol without cache-flushing fences: the logits and the
     // tails' sel / wsel are stored at device scope (through to memory, past
@@ -491,7 +526,7 @@ __global__ __launch_bounds__(640) void route_tails_kernel(BatchedArgs a) {
         if (lane < kk) a.pexp[(size_t)t * kk + lane] = lane < a.k ? e : a.n_ids;
     } else if (wave <= nb) {
         const int b = wave - 1;
-        wave_quantize_q8l(a.fx + (size_t)t * kRouteN + b * QK, q8(a.q8x) + (size_t)t * nb + b);
+        quantize_x(a, a.fx + (size_t)t * kRouteN + b * QK, q8(a.q8x) + (size_t)t * nb + b);
     } else if (a.sh) {
         const float v = router_order_dot(a.sh_gate_inp, a.fx + (size_t)t * kRouteN);
         if (lane == 0) a.sgl[t] = v;
@@ -523,7 +558,7 @@ __global__ __launch_bounds__(512) void prep_ids_large_kernel(BatchedArgs a) {
         }
         if (lane == 0) a.bad[t] = bad ? 1 : 0;
     }
-    if (wave < nb) wave_quantize_q8l(a.fx + (size_t)t * kRouteN + wave * QK, q8(a.q8x) + (size_t)t * nb + wave);
+    if (wave < nb) quantize_x(a, a.fx + (size_t)t * kRouteN + wave * QK, q8(a.q8x) + (size_t)t * nb + wave);
     if (a.sh && wave == 1) {
         const float v = router_order_dot(a.sh_gate_inp, a.fx + (size_t)t * kRouteN);
         if (lane == 0) a.sgl[t] = v;
@@ -611,7 +646,7 @@ __global__ __launch_bounds__(512) void prep_ids_kernel(BatchedArgs a) {
     if ((int)blockIdx.x < a.M) {
         const int t = blockIdx.x;
         for (int b = wave; b < nb; b += 8)
-            wave_quantize_q8l(a.fx + (size_t)t * kRouteN + b * QK, q8(a.q8x) + (size_t)t * nb + b);
+            quantize_x(a, a.fx + (size_t)t * kRouteN + b * QK, q8(a.q8x) + (size_t)t * nb + b);
         if (a.sh && wave == 0) {
             const float v = router_order_dot(a.sh_gate_inp, a.fx + (size_t)t * kRouteN);
             if ((threadIdx.x & 63) == 0) a.sgl[t] = v;
@@ -905,6 +940,11 @@ namespace {
 // The launches after the grouping: gate/up, Q8_K(h), down, combine.
 hipError_t launch_groups(const BatchedArgs &a, hipStream_t s) {
     const int nbh = a.n_ff / QK;
+    if (a.unit) {
+        if (hipError_t e = launch_prefill_groups(a, s); e != hipSuccess) return e;
+        hipLaunchKernelGGL(combine_kernel, dim3((a.n_embd + 255) / 256, a.M), dim3(256), 0, s, a);
+        return hipGetLastError();
+    }
     const int umax = (a.n_ids < a.M * a.k ? a.n_ids : a.M * a.k) + a.sh;
     if (a.gu_type == kTypeQ3K)
         hipLaunchKernelGGL((gateup_kernel<kTypeQ3K, 8>), dim3(a.n_ff / 8, umax), dim3(128), 0, s, a);
@@ -933,14 +973,52 @@ bool args_ok(const BatchedArgs &a) {
            (a.gu_type == kTypeQ4K || a.gu_type == kTypeQ3K) &&
            a.k + a.sh <= kMaxK && a.n_ids >= 1 && a.n_ids + a.sh <= kMaxExperts && a.E + a.sh <= kMaxExperts &&
            (!a.sh || (a.sh == 1 && a.sh_gate && a.sh_up && a.sh_down && a.sh_gate_inp && a.sgl)) &&
-           (a.M <= kMaxTok || (a.goff && a.ptok && a.pslot && a.pexp && a.units && a.n_units && a.max_units >= 1));
+           (a.M <= kMaxTok || (a.goff && a.ptok && a.pslot && a.pexp && a.units && a.n_units));
 }
 
 }  // namespace
 
+// Whether a batch runs as sorted pairs in work units of one expert (16, 32 or
+// 64 pairs each), and the unit size; 0: the per-token dots of expert groups.
+//
+// Above 32 tokens always units, of the smallest size that holds most experts'
+// pairs: small units keep more weights in flight, larger ones read an expert's
+// weights once for more pairs.  Mean pairs an expert against us/layer with
+// units of 16 / 32 / 64: 4 (256 experts, M = 128) 151 / 158 / 179, 8 (128
+// experts, M = 128) 124 / 129 / 128, 10 (512 experts, M = 512) 336 / 336 / 349,
+// 16 (64 experts, M = 128) 102 / 97 / 104, 32 (64 experts, M = 256) 146 / 131 /
+// 125.
+//
+// Up to 32 tokens the dots of most groups' one or two tokens cost less than
+// folding their weights for 16 MFMA columns, except where the row type makes
+// the dot dear: with P pairs over n experts, Q3_K gate/up from P = 1.25 n (64
+// experts: M = 8 67 against 69, M = 10 79 / 75, M = 32 175 / 92 us/layer with
+// units), Q4_K down from 0.75 n (M = 4 40.0 / 41.2, M = 6 46.2 / 45.8, M = 32
+// 119 / 71), Q5_K down beside Q4_K gate/up from n / 8 (256 experts and a shared
+// one: M = 3 36.6 / 36.5, M = 4 42.6 / 41.7, M = 8 52.6 / 50.9, M = 16 71 / 71,
+// M = 32 112 / 104), and any type from 2 n (128 experts: M = 24 92 / 97, M = 32
+// 108 / 103).
+static int unit_pairs(const BatchedArgs &a) {
+    const int P = a.M * a.k, n = a.n_ids;
+    if (a.M <= kMaxTok) {
+        const bool units = P >= 2 * n || (a.gu_type == kTypeQ3K ? 4 * P >= 5 * n
+                                          : a.d_type == kTypeQ4K ? 4 * P >= 3 * n
+                                                                 : a.d_type == kTypeQ5K && 8 * P >= n);
+        return units ? kUnitTokensMin : 0;
+    }
+    return P <= 11 * n ? kUnitTokensMin : P <= 21 * n ? 2 * kUnitTokensMin : kUnitTokens;
+}
+static BatchedArgs with_units(const BatchedArgs &a) {
+    BatchedArgs r = a;
+    r.unit = unit_pairs(a);
+    if (r.unit) r.max_units = prefill_max_units(a.M, a.k + a.sh, a.n_ids + a.sh, r.unit);
+    return r;
+}
+
 // Batches of up to 32 tokens group by expert with 32 token places per group;
 // larger ones sort the pairs and run the prefill units (prefill.hip).
-hipError_t launch_batched(const BatchedArgs &a, hipStream_t s) {
+hipError_t launch_batched(const BatchedArgs &args, hipStream_t s) {
+    const BatchedArgs a = with_units(args);
     if (!args_ok(a) || a.ysrc || a.n_ids != a.E || (a.M + kRouteTok - 1) / kRouteTok > kBatchedCounters - 1)
         return hipErrorInvalidValue;
     if (a.M > kMaxTok) {
@@ -966,7 +1044,8 @@ hipError_t launch_batched(const BatchedArgs &a, hipStream_t s) {
     return launch_groups(a, s);
 }
 
-hipError_t launch_batched_ids(const BatchedArgs &a, hipStream_t s) {
+hipError_t launch_batched_ids(const BatchedArgs &args, hipStream_t s) {
+    const BatchedArgs a = with_units(args);
     if (!args_ok(a) || !a.ysrc || !a.bad) return hipErrorInvalidValue;
     if (a.M > kMaxTok) {
         hipLaunchKernelGGL(prep_ids_large_kernel, dim3(a.M), dim3(512), 0, s, a);

@@ -93,7 +93,8 @@ struct BatchedArgs {
                             // (its first occurrence of the same id), else null
     int *bad;               // [M] caller ids only: 1 for a token with an id outside [0, n_ids), else null
     // prefill-sized batches (M > kBatchedMaxTokens): the pairs sorted by (expert, token)
-    // and cut into work units of at most kUnitTokens pairs of one expert
+    // and cut into work units of at most `unit` pairs of one expert
+    int unit;               // 16, 32 or 64 (kUnitTokens)
     int *goff;              // [umax] first sorted position of each group
     int *ptok, *pslot;      // [M*k] token and slot of each sorted pair
     int *pexp;              // [M*k] expert of each pair for the grouping, -1 for one that joins none
@@ -122,7 +123,8 @@ __device__ __forceinline__ const uint8_t *batched_down(const BatchedArgs &a, int
 }
 constexpr int kBatchedMaxTokens = 32;         // the verify-sized path: per-token dots or MFMA per group
 constexpr int kBatchedMaxTokensLarge = 512;   // the prefill-sized path: sorted pairs, MFMA units
-constexpr int kUnitTokens = 64;               // pairs of one expert per prefill work unit
+constexpr int kUnitTokens = 64;               // most pairs of one expert per prefill work unit
+constexpr int kUnitTokensMin = 16;            // the smallest unit size
 constexpr int kBatchedCounters = 160;         // route completion counters: one per 4 tokens, and the tails'
 constexpr size_t kQ8LBytes = 304;
 hipError_t launch_batched(const BatchedArgs &a, hipStream_t s);
@@ -139,10 +141,11 @@ size_t noalloc_scratch_bytes();
 // The expert products and combine of a prefill-sized batch after its grouping
 // (prefill.hip): gate/up + SwiGLU, Q8_K(h), down, ordered combine.
 hipError_t launch_prefill_groups(const BatchedArgs &a, hipStream_t s);
-// Upper bound of the prefill work units for M*k pairs over n_ids groups.
-inline int prefill_max_units(int M, int k, int n_ids) {
+// Upper bound of the work units of `unit` pairs for M*k pairs over n_ids
+// groups: a group of c pairs takes at most (c + unit - 1) / unit of them.
+inline int prefill_max_units(int M, int k, int n_ids, int unit) {
     const int P = M * k, umax = n_ids < P ? n_ids : P;
-    return umax + (P + kUnitTokens - 1) / kUnitTokens;
+    return (P + umax * (unit - 1)) / unit;
 }
 
 // Persistent stacked decode (one cooperative launch per token).

@@ -209,25 +209,4 @@ __device__ __forceinline__ void tile_q6k(const uint8_t *T, size_t rb, const Q8L 
     for (int i = 0; i < 4; ++i) out[i] = acc[i];
 }
 
-// One super-block b of a 16-row Q4_K tile (row r at W + r*rb) against the
-// token column whose operands are x (the fields q4_load fills); adds its fp32
-// block terms to acc / accm in block order.
-__device__ __forceinline__ void q4_tile_block(const uint8_t *W, size_t rb, int b, const Q6X &x, float acc[4],
-                                              float accm[4]) {
-    Q4Ops o;
-    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
-    const uint8_t *blk_r = W + (size_t)r * rb + (size_t)b * kQ4KBytes;
-#pragma unroll
-    for (int jc = 0; jc < 4; ++jc) o.qa[jc] = *reinterpret_cast<const uint2 *>(blk_r + 16 + 32 * jc + 8 * q);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        o.hd[i] = *reinterpret_cast<const uint4 *>(W + (size_t)(4 * q + i) * rb + (size_t)b * kQ4KBytes);
-#pragma unroll
-    for (int s = 0; s < 8; ++s) o.xb[s] = x.xb[s];
-    o.b0 = x.b0;
-    o.b1 = x.b1;
-    o.xd = x.xd;
-    q4_compute(o, acc, accm);
-}
-
 }  // namespace hoard

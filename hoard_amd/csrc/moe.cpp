@@ -1183,7 +1183,7 @@ BatchedLayout batched_layout(const hoard_moe_cfg &c, int T) {
     L.Ts = std::min(T, hoard::kBatchedMaxTokens);
     L.umax_s = std::min(E, L.Ts * k);
     L.umax = std::min(E, T * k);
-    L.max_units = hoard::prefill_max_units(T, k, E);
+    L.max_units = hoard::prefill_max_units(T, k, E, hoard::kUnitTokensMin);  // the most of any unit size
     const size_t pairs_s = (size_t)L.umax_s * hoard::kBatchedMaxTokens, pairs = (size_t)T * k;
     L.q8x = (size_t)T * nb * hoard::kQ8LBytes;
     L.q8h = std::max(pairs_s, pairs) * nbh * hoard::kQ8LBytes;
@@ -1237,7 +1237,6 @@ void bind_batched(hoard::BatchedArgs &a, const BatchedLayout &L, uint8_t *q8x, u
     a.units = ints + L.o_units;
     a.q8hd = reinterpret_cast<float *>(ints + L.o_q8hd);
     a.n_units = ints + L.o_nunits;
-    a.max_units = hoard::prefill_max_units(a.M, a.k + a.sh, a.n_ids + a.sh);
     a.sgl = reinterpret_cast<float *>(ints + L.o_sgl);
     a.hist = hist;
     a.counters = counters;

@@ -6,7 +6,7 @@
 //
 // batched.hip routes the tokens (or takes the caller's ids), forms Q8_K(fx)
 // and sorts the (token, slot) pairs by (expert, token) into work units of at
-// most kUnitTokens pairs of one expert.  Here, per unit:
+// most 16, 32 or 64 pairs of one expert.  Here, per unit:
 //   gate/up  32 rows of gate and of up per workgroup (16 rows of one matrix per
 //            wave) against the unit's tokens on v_mfma_i32_16x16x64_i8, 16
 //            token columns per MFMA, the sub-block scales folded into the
@@ -15,14 +15,11 @@
 //   Q8_K(h)  per pair;
 //   down     64 rows per workgroup, the tile staged in LDS in one burst;
 //            y goes to its (token, slot) place;
-// Q3_K gate/up rows (pf_gateup_q3_kernel) and Q4_K / Q5_K down rows run one
-// MFMA per sub-block or scale group with the scales applied per (row, token)
-// (mfma.h); Q4_K gate/up and Q6_K down rows fold the scales into the operand.
 //   combine  per token, slots in order, plus the residual.
 // Every expert's weights are read once per unit (once per call for a group of
-// at most kUnitTokens tokens); each (row, token) value is formed from the
-// per-token path's integer sub-block sums in its fp32 order (mfma.h), so every
-// token's result is the single-token path's bit for bit.
+// one unit's pairs); each (row, token) value is formed from the per-token
+// path's integer sub-block sums in its fp32 order, so every token's result is
+// the single-token path's bit for bit.
 #include "kernels.h"
 #include "lds_dma.h"
 #include "mfma.h"
@@ -37,8 +34,6 @@ namespace {
 constexpr int kWaveRows = 16;  // rows per wave: one MFMA tile
 constexpr int kGuRows = 32;    // gate (and up) rows per workgroup: two 16-row tiles
 constexpr int kDnRows = 64;    // down rows per workgroup
-constexpr int kChunks = kUnitTokens / 16;  // 16-token MFMA chunks per unit
-static_assert(kChunks == 4, "four token chunks per unit");
 
 __device__ __forceinline__ const Q8L *q8c(const uint8_t *p) { return reinterpret_cast<const Q8L *>(p); }
 
@@ -55,6 +50,9 @@ __device__ __forceinline__ bool load_unit(const BatchedArgs &a, int unit, Unit &
     w.n = r.z;
     return w.n > 0;
 }
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ v4i mfma_16x16x64(v4i a, v4i b, v4i c) {
     return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
@@ -75,27 +73,49 @@ __device__ __forceinline__ v4i mfma_16x16x64(v4i a, v4i b, v4i c) {
 // hi = q * (sc >> 3) and lo = q * (sc & 7), each <= 105, with
 // sc * q = 8 hi + lo; a nibble times a factor below 8 never carries into the
 // next byte, so a whole word multiplies at once.  The min term
-// sum_s m_s * (sum of sub-block s's activation quants) is a third MFMA with
-// m_s broadcast over the step.  The three chains give exactly the per-token
-// path's integer sums isum = 8 D_hi + D_lo and msum = D_min.  Each 16-bit half
-// of a word of four nibbles multiplies at once (v_pk_mul_lo_u16, full rate,
-// where a 32-bit multiply is quarter rate).
+// sum_s m_s S_s (S_s the sum of sub-block s's activation quants) is one
+// v_mfma_f32_16x16x32_f16 (min_operand below).  The chains give exactly the
+// per-token path's integer sums isum = 8 D_hi + D_lo and msum = D_min.  Each
+// 16-bit half of a word of four nibbles multiplies at once (v_pk_mul_lo_u16,
+// full rate, where a 32-bit multiply is quarter rate).
 struct Q4Fold {
     v4i hi[4], lo[4];
-    v4i mn[2];            // the min of sub-block 2 g + h in every byte (steps of nibble half h)
+    v8h mn;
     float d[4], dmin[4];  // factors of the four rows whose results the lane receives
 };
 
+// The min term of a super-block as one fp16 MFMA.  Every part of a sub-block's
+// sum S_s that the activation block stores (kSums32) and every
+// min (6 bits) is an exact fp16, and the fp32 sum of 16 products stays below
+// 8 * 63 * 4064 < 2^24, so msum comes out exact: K index 8 g + s holds the even
+// parts (g = 0) and the low bits (g = 1) of the sums against m_s, and m = 0 at
+// g = 2, 3, whose lanes read the sums again.  It replaces four int8 steps with
+// m_s broadcast (12 -> 9 MFMAs per chunk step, and a conversion less per row).
+// mn[0] / mn[1]: the mins of sub-blocks 0..3 / 4..7, a byte each.
+__device__ __forceinline__ v8h min_operand(const uint32_t mn[2]) {
+    const bool low = (threadIdx.x & 63) < 32;  // g = 0, 1
+    typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+    const v2h k1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
+    v2h r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        // 0x6400 | m is 1024 + m; bytes 2 (i % 2) and 2 (i % 2) + 1 of the word, each below 0x64
+        const uint32_t w = low ? mn[i >> 1] : 0u;
+        r[i] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, w, (i & 1) ? 0x04030402u : 0x04010400u)) - k1024;
+    }
+    return v8h{r[0][0], r[0][1], r[1][0], r[1][1], r[2][0], r[2][1], r[3][0], r[3][1]};
+}
+__device__ __forceinline__ v4f mfma_f16(v8h a, v8h b) {
+    const v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, z, 0, 0, 0);
+}
+
+typedef short v2s16 __attribute__((ext_vector_type(2)));
 typedef unsigned short v2u16 __attribute__((ext_vector_type(2)));
-// Bytes of w (each <= 15) times f (<= 7), byte by byte: no product carries.
+// Bytes of w times f, byte by byte, where no product passes 255: none carries.
 __device__ __forceinline__ int nib_mul(uint32_t w, uint32_t f) {
     const v2u16 m = {(unsigned short)f, (unsigned short)f};
     return (int)__builtin_bit_cast(uint32_t, __builtin_bit_cast(v2u16, w) * m);
-}
-
-// Byte i of w in all four bytes (one v_perm_b32).
-__device__ __forceinline__ int splat_byte_of(uint32_t w, int i) {
-    return (int)__builtin_amdgcn_perm(w, w, 0x01010101u * (uint32_t)i);
 }
 
 // The lane's raw bytes of one super-block of a 16-row tile: its row's header
@@ -123,11 +143,7 @@ __device__ __forceinline__ void q4_fold(const Q4Raw &raw, Q4Fold &o) {
     // the scales and mins of sub-blocks 2 g (low nibbles) and 2 g + 1 (high)
     const int s0 = 2 * g;
     const uint32_t sc0 = (uint32_t)byte_of(sc[s0 >> 2], s0 & 3), sc1 = (uint32_t)byte_of(sc[s0 >> 2], (s0 & 3) + 1);
-    const int mw = (int)mn[s0 >> 2];
-    const int m0 = (int)__builtin_amdgcn_perm(mw, mw, 0x01010101u * (uint32_t)(s0 & 3));
-    const int m1 = (int)__builtin_amdgcn_perm(mw, mw, 0x01010101u * (uint32_t)((s0 & 3) + 1));
-    o.mn[0] = v4i{m0, m0, m0, m0};
-    o.mn[1] = v4i{m1, m1, m1, m1};
+    o.mn = min_operand(mn);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const uint4 qv = raw.qv[j >> 1];
@@ -146,144 +162,44 @@ __device__ __forceinline__ void q4_fold(const Q4Raw &raw, Q4Fold &o) {
     }
 }
 
-// One super-block of the folded tile against the lane's token column (its Q8_K
-// block x): the integer sums from the three MFMA chains, then the per-token
-// path's fp32 block terms added in order.  Step j's B operand: activation
-// quants 64 g + 16 (j / 2) + 32 (j % 2) .. + 15.
-template <class X>
-__device__ __forceinline__ void q4_fold_step(const Q4Fold &w, const X &x, float acc[4], float accm[4]) {
-    const int g = (threadIdx.x & 63) >> 4;
-    v4i dh = {0, 0, 0, 0}, dl = {0, 0, 0, 0}, dn = {0, 0, 0, 0};
+// The lane's operands of one token's activation block: four 16-byte pieces of
+// its quants (which ones depends on the fold), its sums (types with a min
+// term) and its scale.
+struct XOps {
+    v4i x[4];
+    v8h bs;
+    float xd;
+};
+
+// acc / accm of the lane's four rows for one super-block: the integer sums
+// from the MFMA chains, then the per-token path's fp32 block terms in order.
+__device__ __forceinline__ void q4_fold_step(const Q4Fold &w, const XOps &x, float acc[4], float accm[4]) {
+    v4i dh = {0, 0, 0, 0}, dl = {0, 0, 0, 0};
+    const v4f dn = mfma_f16(w.mn, x.bs);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const v4i xv = *reinterpret_cast<const v4i *>(&x.qs[16 * g + 4 * (j >> 1) + 8 * (j & 1)]);
-        dh = mfma_16x16x64(w.hi[j], xv, dh);
-        dl = mfma_16x16x64(w.lo[j], xv, dl);
-        dn = mfma_16x16x64(w.mn[j & 1], xv, dn);
+        dh = mfma_16x16x64(w.hi[j], x.x[j], dh);
+        dl = mfma_16x16x64(w.lo[j], x.x[j], dl);
     }
-    const float xd = x.d;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int isum = 8 * dh[i] + dl[i];
-        const float dd = w.d[i] * xd;
-        const float dm = w.dmin[i] * xd;
+        const float dd = w.d[i] * x.xd;
+        const float dm = w.dmin[i] * x.xd;
         acc[i] = acc[i] + dd * (float)isum;
-        accm[i] = accm[i] + dm * (float)dn[i];
+        accm[i] = accm[i] + dm * dn[i];
     }
 }
-
-// -- gate/up + SwiGLU ------------------------------------------------------------
-// grid (n_ff / 32, max units), block 256: wave w takes rows [32 x + 16 (w % 2), +16)
-// of gate (w < 2) or up (w >= 2) of the unit's expert against every token of the
-// unit.  Per super-block the workgroup copies the Q8_K blocks of the unit's
-// token chunks into LDS (one buffer ahead) while each wave holds the next
-// super-block of its rows in registers; the gate waves hand their values to the
-// up waves through LDS, which form h and store it to hbuf[sorted pair][row].
-// Three workgroups share a CU (43 KB of LDS each).  The kernel is compiled to
-// the 128 registers of four waves a SIMD all the same: that schedule measured
-// 1 % faster for the layer than the 146-register one at three waves (a fourth
-// workgroup a CU, with the gate values over an x buffer, spilled and measured
-// 12 % slower).
-// The part of a Q8_K block the folded gate/up tiles read: the quants and the
-// scale (granules 0-15 and 18 of the block; its 16-element sums are not read).
-struct Q8S {
-    int32_t qs[64];
-    float d;
-    int32_t pad[3];
-};
-static_assert(sizeof(Q8S) == 272 && offsetof(Q8L, d) == 288, "Q8S: 17 granules, d from granule 18 of Q8L");
-constexpr int kXGran = (int)sizeof(Q8S) / 16;                          // 16-byte granules staged per token
-constexpr int kXChunksPerBlock = (kUnitTokens * kXGran + 63) / 64;     // 1 KB copies per unit block
-
-template <int NB>
-__global__ __launch_bounds__(256, 4) void pf_gateup_kernel(BatchedArgs a) {
-    __shared__ __align__(16) Q8S xs[2][kUnitTokens];  // the unit's Q8_K block b (two buffers)
-    __shared__ float gx[2][kChunks][4][64];            // gate values: [row tile][chunk][row i][lane]
-    Unit w;
-    if (!load_unit(a, blockIdx.y, w)) return;
-    const int wave = wave_index(), lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
-    const int m = wave >> 1, rt = wave & 1;
-    const int row0 = blockIdx.x * kGuRows + rt * kWaveRows;
-    constexpr size_t rb = (size_t)NB * kQ4KBytes;
-    const uint8_t *W = (m ? batched_up(a, w.e) : batched_gate(a, w.e)) + (size_t)row0 * rb;
-    const int nch = (w.n + 15) >> 4;
-    // this lane's granules of the x copy: chunks wave, wave + 4, ...; only the
-    // unit's tokens are copied (the MFMA columns of the places past them read
-    // whatever the buffer holds, and their results are not stored)
-    constexpr int kXJ = (kXChunksPerBlock + 3) / 4;
-    const int ngran = w.n * kXGran;
-    // byte offsets into q8x (it holds at most 512 tokens' blocks): half the
-    // registers of pointers
-    uint32_t xoff[kXJ];
+// Step j of a Q4_K fold takes activation quants 64 g + 16 (j / 2) + 32 (j % 2) .. + 15.
+template <class X>
+__device__ __forceinline__ void q4_load_x(const X &x, XOps &o) {
+    const int g = (threadIdx.x & 63) >> 4;
 #pragma unroll
-    for (int j = 0; j < kXJ; ++j) {
-        const int p = 64 * (wave + 4 * j) + lane, tt = min(p / kXGran, kUnitTokens - 1), o = p % kXGran;
-        xoff[j] = (uint32_t)a.ptok[w.p0 + min(tt, w.n - 1)] * (uint32_t)(NB * sizeof(Q8L)) + 16u * (o < 16 ? o : 18);
-    }
-    auto stage_x = [&](int b, int buf) {
-#pragma unroll
-        for (int j = 0; j < kXJ; ++j) {
-            const int ck = wave + 4 * j;
-            if (64 * ck < ngran && 64 * ck + lane < ngran)
-                dma_lanes(reinterpret_cast<uint8_t *>(&xs[buf][0]) + 1024 * ck,
-                          a.q8x + (xoff[j] + (uint32_t)(b * sizeof(Q8L))));
-        }
-    };
-    float acc[kChunks][4], accm[kChunks][4];
-#pragma unroll
-    for (int ch = 0; ch < kChunks; ++ch)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[ch][i] = accm[ch][i] = 0.0f;
-    Q4Raw raw;
-    q4_raw_load(W, rb, 0, raw);
-    stage_x(0, 0);
-#pragma unroll 1
-    for (int b = 0; b < NB; ++b) {
-        // Other waves read the x chunks this wave copied: the compiler does not
-        // see the copies, so the wave waits for its own before the barrier (it
-        // waits for the raw weight loads of block b there anyway).
-        lds_dma_wait();
-        __syncthreads();  // every wave's copies of x(b) landed, and x(b - 1) is read
-        Q4Fold t;
-        q4_fold(raw, t);
-        // the fold is done before the next loads issue
-        asm volatile("" ::"v"(t.hi[0]), "v"(t.hi[1]), "v"(t.hi[2]), "v"(t.hi[3]), "v"(t.lo[0]), "v"(t.lo[1]),
-                     "v"(t.lo[2]), "v"(t.lo[3])
-                     : "memory");
-        // the next super-block's activation copies issue before its weight
-        // loads (both are waited for at the next super-block; copies first
-        // measured 3 % faster for the layer at 512 tokens)
-        if (b + 1 < NB) {
-            stage_x(b + 1, (b + 1) & 1);
-            q4_raw_load(W, rb, b + 1, raw);
-        }
-        const Q8S *xb = xs[b & 1];
-#pragma unroll
-        for (int ch = 0; ch < kChunks; ++ch)
-            if (ch < nch) q4_fold_step(t, xb[ch * 16 + c], acc[ch], accm[ch]);
-    }
-    if (m == 0) {
-#pragma unroll
-        for (int ch = 0; ch < kChunks; ++ch)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) gx[rt][ch][i][lane] = acc[ch][i] - accm[ch][i];
-    }
-    __syncthreads();
-    if (m == 0) return;
-#pragma unroll
-    for (int ch = 0; ch < kChunks; ++ch) {
-        const int idx = ch * 16 + c;
-        if (ch < nch && idx < w.n) {
-            float hv[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float g = gx[rt][ch][i][lane], uu = acc[ch][i] - accm[ch][i];
-                hv[i] = g / (1.0f + expf(-g)) * uu;
-            }
-            *reinterpret_cast<float4 *>(a.hbuf + (size_t)(w.p0 + idx) * a.n_ff + row0 + 4 * q) =
-                make_float4(hv[0], hv[1], hv[2], hv[3]);
-        }
-    }
+    for (int j = 0; j < 4; ++j) o.x[j] = *reinterpret_cast<const v4i *>(&x.qs[16 * g + 4 * (j >> 1) + 8 * (j & 1)]);
+}
+template <class X>
+__device__ __forceinline__ v8h load_sums(const X &x) {
+    return reinterpret_cast<const v8h *>(x.bsums)[((threadIdx.x & 63) >> 4) & 1];
 }
 
 // -- Q8_K of h per sorted pair --------------------------------------------------
@@ -292,60 +208,23 @@ __global__ __launch_bounds__(256) void pf_quant_h_kernel(BatchedArgs a) {
     const int pos = blockIdx.x, b = wave_index();
     const int nbh = a.n_ff / QK;
     if (b >= nbh) return;
-    const float d = wave_quantize_q8l(a.hbuf + (size_t)pos * a.n_ff + (size_t)b * QK,
+    const float d = wave_quantize_q8l<kSums32>(a.hbuf + (size_t)pos * a.n_ff + (size_t)b * QK,
                                       reinterpret_cast<Q8L *>(a.q8h) + (size_t)pos * nbh + b);
     // the scales again, four to a pair: the down kernels copy a unit's in one 16-byte load a lane
     if ((threadIdx.x & 63) == 0) a.q8hd[(size_t)pos * 4 + b] = d;
 }
 
-// -- down: 64 rows of the unit's expert, y to its (token, slot) place -----------
-// grid (n_embd / 64, max units), block 256, for Q4_K down rows (OLMoE).  The
-// 64-row tile is copied into LDS in one burst; wave w takes rows [16 w, +16) of it.
-template <int NBH>
-__global__ __launch_bounds__(256) void pf_down_q4_kernel(BatchedArgs a) {
-    constexpr int kRowBytes = NBH * kQ4KBytes;
-    constexpr int kTileBytes = kDnRows * kRowBytes;
-    static_assert(kTileBytes % 16 == 0, "the tile copies in 16-byte units");
-    __shared__ __align__(16) uint8_t tile[kTileBytes];
-    Unit w;
-    if (!load_unit(a, blockIdx.y, w)) return;
-    const int wave = wave_index(), lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
-    const int rt0 = blockIdx.x * kDnRows;
-    // each wave copies its own 16 rows and waits for them alone
-    constexpr int kWaveBytes = kWaveRows * kRowBytes;
-    static_assert(kWaveBytes % 16 == 0, "a wave's rows copy in 16-byte units");
-    uint8_t *T = tile + wave * kWaveBytes;
-    dma_wave_copy_nt(T, batched_down(a, w.e) + (size_t)(rt0 + wave * kWaveRows) * kRowBytes, kWaveBytes);
-    lds_dma_wait();
-    const int nch = (w.n + 15) >> 4;
-    const Q8L *q8h = reinterpret_cast<const Q8L *>(a.q8h);
-    // (chunk, block) steps with the next step's activation operands loaded
-    // while the current one computes
-    auto xq_of = [&](int ch) { return q8h + (size_t)(w.p0 + min(ch * 16 + c, w.n - 1)) * NBH; };
-    Q6X cur, nxt;
-    q6_load_x(xq_of(0), 0, cur);
-    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f}, accm[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    const int steps = nch * NBH;
-#pragma unroll 1
-    for (int st = 0; st < steps; ++st) {
-        const int ch = st / NBH, b = st - ch * NBH;
-        if (st + 1 < steps) q6_load_x(xq_of((st + 1) / NBH), (st + 1) % NBH, nxt);
-        q4_tile_block(T, kRowBytes, b, cur, acc, accm);
-        if (b == NBH - 1) {
-            const int idx = ch * 16 + c;
-            if (idx < w.n) {
-                const int pos = w.p0 + idx, t = a.ptok[pos], j = a.pslot[pos];
-                float v[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) v[i] = acc[i] - accm[i];
-                *reinterpret_cast<float4 *>(a.ybuf + ((size_t)t * (a.k + a.sh) + j) * a.n_embd + rt0 + wave * kWaveRows +
-                                            4 * q) = make_float4(v[0], v[1], v[2], v[3]);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[i] = accm[i] = 0.0f;
-        }
-        cur = nxt;
-    }
+// Bytes 0, 2 and 1, 3 of w in the 16-bit halves of two words, and back.
+__device__ __forceinline__ void bytes_to_halves(uint32_t w, uint32_t &w02, uint32_t &w13) {
+    w02 = __builtin_amdgcn_perm(0u, w, 0x0c020c00u);
+    w13 = __builtin_amdgcn_perm(0u, w, 0x0c030c01u);
+}
+__device__ __forceinline__ int halves_to_bytes(uint32_t w02, uint32_t w13) {
+    return (int)__builtin_amdgcn_perm(w13, w02, 0x06020400u);
+}
+// The high bytes of the halves.
+__device__ __forceinline__ int high_bytes(uint32_t w02, uint32_t w13) {
+    return (int)__builtin_amdgcn_perm(w13, w02, 0x07030501u);
 }
 
 // -- down, Q6_K rows folded for v_mfma_i32_16x16x64_i8 --------------------------
@@ -355,15 +234,15 @@ __global__ __launch_bounds__(256) void pf_down_q4_kernel(BatchedArgs a) {
 // bits 4 (jc % 2) + 2 (g / 2) .. + 1 of qh bytes 128 + 32 (jc / 2) + 16 (g % 2) ..
 // + 15 on top, and which share one group scale, sc = scales[4 jc + g].  The
 // per-token path forms isum = sum_g sc_g * sum_{e in g} (q_e - 32) x_e.  Here
-// w = sc * q (-8064 <= w <= 8001) is split as w = 64 hi + lo with lo = w & 63 in
-// [0, 63] and hi = w >> 6 in [-126, 125], both int8, and the zero point comes from a third MFMA with
-// sc broadcast over the lane's 16 elements (the token's group sums):
-// isum = 64 D_hi + D_lo - 32 D_sc, exactly.  A super-block of the tile is
-// folded once and used for every token chunk of the unit.
+// w = sc * (q - 32) = sc * q - 32 sc (one 16-bit multiply-add; -4064 <= w <=
+// 4096) is split as w = 256 hi + lo with lo its low byte read as int8 and
+// hi = (w + 128) >> 8 in [-16, 16]: isum = 256 D_hi + D_lo, exactly, and both
+// parts are bytes of 16-bit words as they stand.  A super-block of the tile is
+// folded once and used for every token chunk of the unit.  (With the zero
+// point as a third MFMA chain, sc broadcast, a step took 12 MFMAs for these 8.)
 struct Q6Fold {
     v4i hi[4], lo[4];
-    uint32_t sc;  // byte jc: the group scale of the lane's elements of chunk jc
-    float d[4];   // factors of the four rows whose results the lane receives
+    float d[4];  // factors of the four rows whose results the lane receives
 };
 
 // 16 bytes at a 2-byte aligned LDS address, as four words.
@@ -382,6 +261,8 @@ __device__ __forceinline__ void q6_fold(const uint8_t *T, size_t rb, int b, Q6Fo
         const int sc = (int)(int8_t)blk[192 + 4 * jc + g];
         const uint32_t nsh = 4u * (uint32_t)(jc & 1), hsh = 4u * (uint32_t)(jc & 1) + 2u * (uint32_t)(g >> 1);
         const uint32_t sc16 = ((uint32_t)sc & 0xffffu) * 0x00010001u;  // sc in both 16-bit halves
+        typedef short v2s __attribute__((ext_vector_type(2)));
+        const v2s s2 = __builtin_bit_cast(v2s, sc16), z2 = {(short)(-32 * sc), (short)(-32 * sc)};
         const uint32_t qlw[4] = {ql.x, ql.y, ql.z, ql.w}, qhw[4] = {qh.x, qh.y, qh.z, qh.w};
         int hw[4], lw[4];
 #pragma unroll
@@ -390,22 +271,13 @@ __device__ __forceinline__ void q6_fold(const uint8_t *T, size_t rb, int b, Q6Fo
             // bytes 0, 2 and 1, 3 in 16-bit halves; w = sc * q in each half
             const uint32_t w02 = __builtin_amdgcn_perm(0u, q, 0x0c020c00u) ;
             const uint32_t w13 = __builtin_amdgcn_perm(0u, q, 0x0c030c01u);
-            typedef short v2s __attribute__((ext_vector_type(2)));
-            const v2s s2 = __builtin_bit_cast(v2s, sc16);
-            const v2s a02 = __builtin_bit_cast(v2s, w02) * s2, a13 = __builtin_bit_cast(v2s, w13) * s2;
-            // hi = w >> 6 (arithmetic: floor(w / 64)), lo = w & 63 = w - 64 hi
-            const v2s h02 = a02 >> (v2s){6, 6}, h13 = a13 >> (v2s){6, 6};
-            const v2s l02 = a02 & (v2s){63, 63}, l13 = a13 & (v2s){63, 63};
-            // back to bytes: result byte 2i from the 02 half i, byte 2i + 1 from the 13 half i
-            hw[k] = (int)__builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, h13), __builtin_bit_cast(uint32_t, h02),
-                                               0x06020400u);
-            lw[k] = (int)__builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, l13), __builtin_bit_cast(uint32_t, l02),
-                                               0x06020400u);
+            const v2s a02 = __builtin_bit_cast(v2s, w02) * s2 + z2, a13 = __builtin_bit_cast(v2s, w13) * s2 + z2;
+            const v2s r = {128, 128};
+            lw[k] = halves_to_bytes(__builtin_bit_cast(uint32_t, a02), __builtin_bit_cast(uint32_t, a13));
+            hw[k] = high_bytes(__builtin_bit_cast(uint32_t, a02 + r), __builtin_bit_cast(uint32_t, a13 + r));
         }
         o.hi[jc] = v4i{hw[0], hw[1], hw[2], hw[3]};
         o.lo[jc] = v4i{lw[0], lw[1], lw[2], lw[3]};
-        if (jc == 0) o.sc = 0u;
-        o.sc |= ((uint32_t)sc & 0xffu) << (8 * jc);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -414,104 +286,16 @@ __device__ __forceinline__ void q6_fold(const uint8_t *T, size_t rb, int b, Q6Fo
     }
 }
 
-// The lane's B operands of one token's Q8_K block: qs bytes 64 jc + 16 g .. + 15.
-struct Q6XB {
-    v4i x[4];
-    float xd;
-};
-__device__ __forceinline__ void q6_load_xb(const Q8L &x, Q6XB &o) {
-    const int g = (threadIdx.x & 63) >> 4;
-#pragma unroll
-    for (int jc = 0; jc < 4; ++jc) o.x[jc] = *reinterpret_cast<const v4i *>(&x.qs[16 * jc + 4 * g]);
-    o.xd = x.d;
-}
-// The quants alone, the scale coming from elsewhere.
-__device__ __forceinline__ void q6_load_xq(const Q8L &x, Q6XB &o) {
+// The quants of one token's block as the Q3_K, Q5_K and Q6_K folds take them:
+// step jc elements 64 jc + 16 g .. + 15.
+template <class X>
+__device__ __forceinline__ void q6_load_x(const X &x, XOps &o) {
     const int g = (threadIdx.x & 63) >> 4;
 #pragma unroll
     for (int jc = 0; jc < 4; ++jc) o.x[jc] = *reinterpret_cast<const v4i *>(&x.qs[16 * jc + 4 * g]);
 }
 
-__device__ __forceinline__ void q6_fold_step(const Q6Fold &w, const Q6XB &x, float acc[4]) {
-    v4i dh = {0, 0, 0, 0}, dl = {0, 0, 0, 0}, ds = {0, 0, 0, 0};
-#pragma unroll
-    for (int jc = 0; jc < 4; ++jc) {
-        dh = mfma_16x16x64(w.hi[jc], x.x[jc], dh);
-        dl = mfma_16x16x64(w.lo[jc], x.x[jc], dl);
-        const int s4 = splat_byte_of(w.sc, jc);
-        ds = mfma_16x16x64(v4i{s4, s4, s4, s4}, x.x[jc], ds);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int isum = 64 * dh[i] + dl[i] - 32 * ds[i];
-        acc[i] = acc[i] + (w.d[i] * x.xd) * (float)isum;
-    }
-}
-
-typedef short v2s16 __attribute__((ext_vector_type(2)));
-typedef unsigned short v2u16b __attribute__((ext_vector_type(2)));
-
-// Bytes 0, 2 and 1, 3 of w in the 16-bit halves of two words, and back.
-__device__ __forceinline__ void bytes_to_halves(uint32_t w, uint32_t &w02, uint32_t &w13) {
-    w02 = __builtin_amdgcn_perm(0u, w, 0x0c020c00u);
-    w13 = __builtin_amdgcn_perm(0u, w, 0x0c030c01u);
-}
-__device__ __forceinline__ int halves_to_bytes(uint32_t w02, uint32_t w13) {
-    return (int)__builtin_amdgcn_perm(w13, w02, 0x06020400u);
-}
-
-// Q3_K super-block b of a 16-row tile in LDS (row r at T + r*rb; 110-byte
-// blocks, only 2-byte aligned), folded for v_mfma_i32_16x16x64_i8.  Lane group
-// g of chunk jc supplies elements 64 jc + 16 g .. + 15 of its row: 32-element
-// range 2 jc + g / 2 (half n = jc / 2, quarter j = 2 (jc & 1) + g / 2),
-// positions l = 16 (g & 1) .. + 15, one 16-element scale group G = 4 jc + g.
-// Its quants are q3 = q2 + 4 h - 4 (q2: bits 2 j .. 2 j + 1 of qs[32 n + l];
-// h: bit 4 n + j of hmask[l]) and w = (sc_G - 32) * q3 lies in [-124, 128]; it
-// is split as w = 64 hi + lo with lo = w & 63 and hi = w >> 6 in [-2, 2], both
-// int8, so isum = 64 D_hi + D_lo is the per-token path's integer sum exactly.
-struct Q3Fold {
-    v4i hi[4], lo[4];
-    float d[4];  // factors of the four rows whose results the lane receives
-};
-
-__device__ __forceinline__ void q3_fold(const uint8_t *T, size_t rb, int b, Q3Fold &o) {
-    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    const uint8_t *blk = T + (size_t)r * rb + (size_t)b * kQ3KBytes;
-    const uint4 hm = lds_u128_a2(blk + 16 * (g & 1));  // hmask[l], l = 16 (g & 1) .. + 15
-    const uint2 s01 = lds_u64_a2(blk + 96);
-    const uint32_t s2 = lds_u32(blk + 104);
-    const uint32_t hmw[4] = {hm.x, hm.y, hm.z, hm.w};
-#pragma unroll
-    for (int jc = 0; jc < 4; ++jc) {
-        const int n = jc >> 1, j = 2 * (jc & 1) + (g >> 1);
-        const uint4 qv = lds_u128_a2(blk + 32 + 32 * n + 16 * (g & 1));
-        const int sc = q3k_scale(4 * jc + g, s01.x, s01.y, s2);
-        const v2s16 scv = {(short)sc, (short)sc};
-        const uint32_t qw[4] = {qv.x, qv.y, qv.z, qv.w};
-        int hw[4], lw[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const uint32_t q = ((qw[k] >> (2 * j)) & 0x03030303u) | (((hmw[k] >> (4 * n + j)) & 0x01010101u) << 2);
-            uint32_t q02, q13;
-            bytes_to_halves(q, q02, q13);
-            const v2s16 w02 = (__builtin_bit_cast(v2s16, q02) - (v2s16){4, 4}) * scv;
-            const v2s16 w13 = (__builtin_bit_cast(v2s16, q13) - (v2s16){4, 4}) * scv;
-            hw[k] = halves_to_bytes(__builtin_bit_cast(uint32_t, w02 >> (v2s16){6, 6}),
-                                    __builtin_bit_cast(uint32_t, w13 >> (v2s16){6, 6}));
-            lw[k] = halves_to_bytes(__builtin_bit_cast(uint32_t, w02 & (v2s16){63, 63}),
-                                    __builtin_bit_cast(uint32_t, w13 & (v2s16){63, 63}));
-        }
-        o.hi[jc] = v4i{hw[0], hw[1], hw[2], hw[3]};
-        o.lo[jc] = v4i{lw[0], lw[1], lw[2], lw[3]};
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint8_t *blk_i = T + (size_t)(4 * g + i) * rb + (size_t)b * kQ3KBytes;
-        o.d[i] = half_bits_to_float((uint32_t)blk_i[108] | ((uint32_t)blk_i[109] << 8));
-    }
-}
-
-__device__ __forceinline__ void q3_fold_step(const Q3Fold &w, const Q6XB &x, float acc[4]) {
+__device__ __forceinline__ void fold_step(const Q6Fold &w, const XOps &x, float acc[4], float *) {
     v4i dh = {0, 0, 0, 0}, dl = {0, 0, 0, 0};
 #pragma unroll
     for (int jc = 0; jc < 4; ++jc) {
@@ -520,7 +304,118 @@ __device__ __forceinline__ void q3_fold_step(const Q3Fold &w, const Q6XB &x, flo
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int isum = 64 * dh[i] + dl[i];
+        const int isum = 256 * dh[i] + dl[i];
+        acc[i] = acc[i] + (w.d[i] * x.xd) * (float)isum;
+    }
+}
+
+// Q3_K super-block b of a 16-row tile in LDS (row r at T + r*rb; 110-byte
+// blocks, only 2-byte aligned), folded for v_mfma_i32_16x16x64_i8.  Lane group
+// g of chunk jc supplies elements 64 jc + 16 g .. + 15 of its row: 32-element
+// range 2 jc + g / 2 (half n = jc / 2, quarter j = 2 (jc & 1) + g / 2),
+// positions l = 16 (g & 1) .. + 15, one 16-element scale group G = 4 jc + g.
+// Its quants are q3 = q - 4, q = q2 + 4 h (q2: bits 2 j .. 2 j + 1 of
+// qs[32 n + l]; h: bit 4 n + j of hmask[l]), its scale sc_G is in [-32, 31].
+// sc_G * q3 reaches 128, but w = sc_G * (q3 + 1) lies in [-128, 124], an int8, so
+// one MFMA chain forms sum w x, and what the 1 adds comes off through an fp16
+// MFMA over the 16-element sums T_G (exact: at most 2032):
+// isum = D_w - sum_G sc_G T_G.  Five MFMAs a chunk step and 16 registers, where
+// sc * q3 split in two int8 parts takes eight and 32.
+struct Q3Fold {
+    v4i w[4];
+    v8h sc;      // -sc of the groups of the lane's K range (zero at g = 2, 3)
+    float d[4];  // factors of the four rows whose results the lane receives
+};
+// The lane's raw bytes of the block: its half of hmask, its half of the qs of
+// both 128-element halves, its row's scales and factor.
+struct Q3Raw {
+    uint4 hm, qv[2];
+    uint32_t s[3], d;
+};
+__device__ __forceinline__ void q3_raw_lds(const uint8_t *T, size_t rb, int b, Q3Raw &o) {
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const uint8_t *blk = T + (size_t)r * rb + (size_t)b * kQ3KBytes;
+    o.hm = lds_u128_a2(blk + 16 * (g & 1));
+    o.qv[0] = lds_u128_a2(blk + 32 + 16 * (g & 1));
+    o.qv[1] = lds_u128_a2(blk + 64 + 16 * (g & 1));
+    const uint2 s01 = lds_u64_a2(blk + 96);
+    o.s[0] = s01.x;
+    o.s[1] = s01.y;
+    o.s[2] = lds_u32(blk + 104);
+    o.d = (uint32_t)blk[108] | ((uint32_t)blk[109] << 8);
+}
+// The same from memory, which takes 2-byte aligned loads of any width.
+__device__ __forceinline__ void raw_load(const uint8_t *W, size_t rb, int b, Q3Raw &o) {
+    typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+    typedef uint32_t v3u __attribute__((ext_vector_type(3)));
+    typedef v4u v4u_a2 __attribute__((aligned(2)));
+    typedef v3u v3u_a2 __attribute__((aligned(2)));
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const uint8_t *blk = W + (size_t)r * rb + (size_t)b * kQ3KBytes;
+    const v4u h = *reinterpret_cast<const v4u_a2 *>(blk + 16 * (g & 1));
+    const v4u q0 = *reinterpret_cast<const v4u_a2 *>(blk + 32 + 16 * (g & 1));
+    const v4u q1 = *reinterpret_cast<const v4u_a2 *>(blk + 64 + 16 * (g & 1));
+    const v3u sc = *reinterpret_cast<const v3u_a2 *>(blk + 96);
+    o.hm = make_uint4(h[0], h[1], h[2], h[3]);
+    o.qv[0] = make_uint4(q0[0], q0[1], q0[2], q0[3]);
+    o.qv[1] = make_uint4(q1[0], q1[1], q1[2], q1[3]);
+    o.s[0] = sc[0];
+    o.s[1] = sc[1];
+    o.s[2] = sc[2];
+    o.d = *reinterpret_cast<const uint16_t *>(blk + 108);
+}
+
+__device__ __forceinline__ void fold(const Q3Raw &raw, Q3Fold &o) {
+    const uint32_t g = (threadIdx.x & 63) >> 4, gh = g >> 1;
+    // scale bytes g of the three words: groups g, 4 + g, 8 + g, 12 + g
+    const uint32_t b0 = raw.s[0] >> (8 * g), b1 = raw.s[1] >> (8 * g), b2 = raw.s[2] >> (8 * g);
+    const uint32_t s6[4] = {(b0 & 15u) | ((b2 & 3u) << 4), (b1 & 15u) | ((b2 & 12u) << 2),
+                            ((b0 >> 4) & 15u) | (b2 & 48u), ((b1 >> 4) & 15u) | ((b2 >> 2) & 48u)};
+    const uint32_t hm[4] = {raw.hm.x >> gh, raw.hm.y >> gh, raw.hm.z >> gh, raw.hm.w >> gh};
+#pragma unroll
+    for (int jc = 0; jc < 4; ++jc) {
+        const int n = jc >> 1, cq = 4 * (jc & 1), ch = 4 * n + 2 * (jc & 1);  // after the lane's own shifts
+        const uint4 &qv = raw.qv[n];
+        const uint32_t qw[4] = {qv.x >> (2 * gh), qv.y >> (2 * gh), qv.z >> (2 * gh), qv.w >> (2 * gh)};
+        const int sc = (int)s6[jc] - 32;
+        const v2s16 scv = {(short)sc, (short)sc}, z = {(short)(-3 * sc), (short)(-3 * sc)};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t h = ch < 2 ? hm[k] << (2 - ch) : hm[k] >> (ch - 2);  // the bit at bit 2 of each byte
+            const uint32_t q = ((qw[k] >> cq) & 0x03030303u) | (h & 0x04040404u);
+            uint32_t q02, q13;
+            bytes_to_halves(q, q02, q13);
+            o.w[jc][k] = halves_to_bytes(__builtin_bit_cast(uint32_t, __builtin_bit_cast(v2s16, q02) * scv + z),
+                                         __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2s16, q13) * scv + z));
+        }
+    }
+    // the scales of groups 8 g .. 8 g + 7 (g = 0, 1) as fp16: 0x6400 | s is 1024 + s
+    typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+    const uint32_t sh = 4u * (g & 1u);
+    uint32_t w0 = ((raw.s[0] >> sh) & 0x0f0f0f0fu) | (((raw.s[2] >> sh) & 0x03030303u) << 4);
+    uint32_t w1 = ((raw.s[1] >> sh) & 0x0f0f0f0fu) | (((raw.s[2] >> sh) & 0x0c0c0c0cu) << 2);
+    w0 = g < 2 ? w0 : 0x20202020u;  // sc = 0
+    w1 = g < 2 ? w1 : 0x20202020u;
+    const v2h k1056 = {(_Float16)1056.0f, (_Float16)1056.0f};
+    v2h r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t w = i < 2 ? w0 : w1;
+        r[i] = k1056 - __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, w, (i & 1) ? 0x04030402u : 0x04010400u));
+    }
+    o.sc = v8h{r[0][0], r[0][1], r[1][0], r[1][1], r[2][0], r[2][1], r[3][0], r[3][1]};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o.d[i] = half_bits_to_float((uint32_t)__shfl((int)raw.d, 4 * (int)g + i));
+}
+
+__device__ __forceinline__ void fold_step(const Q3Fold &w, const XOps &x, float acc[4], float *) {
+    v4i dw = {0, 0, 0, 0};
+    const v4f dt = mfma_f16(w.sc, x.bs);
+#pragma unroll
+    for (int jc = 0; jc < 4; ++jc) dw = mfma_16x16x64(w.w[jc], x.x[jc], dw);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int isum = dw[i] + (int)dt[i];
         acc[i] = acc[i] + (w.d[i] * x.xd) * (float)isum;
     }
 }
@@ -529,12 +424,14 @@ __device__ __forceinline__ void q3_fold_step(const Q3Fold &w, const Q6XB &x, flo
 // d, dmin, Q4_K-packed scales and mins, qh[32], qs[128]), folded as the Q4_K
 // gate/up tile is: lane group g of chunk jc takes nibble g / 2 of qs bytes
 // 32 jc + 16 (g & 1) .. + 15 with bit 2 jc + g / 2 of qh[l] on top (q5 in
-// [0, 31]), sub-block s = 2 jc + g / 2.  w = sc_s * q5 <= 1953 is split as
-// w = 64 hi + lo (lo = w & 63, hi = w >> 6 <= 30); the min term is a third MFMA
-// with m_s broadcast over its sub-block: isum = 64 D_hi + D_lo, msum = D_min.
+// [0, 31]), sub-block s = 2 jc + g / 2.  sc_s is taken two bits at a time, so
+// that q5 * part (at most 93) stays a byte of a word multiply:
+// isum = 16 D_2 + 4 D_1 + D_0; the min term is Q4_K's fp16 MFMA.  (Two chains
+// of a product formed in 16-bit halves cost 5 vector instructions more per
+// word of four quants.)
 struct Q5Fold {
-    v4i hi[4], lo[4];
-    uint32_t mn;          // byte jc: the min of the lane's sub-block in chunk jc
+    v4i p[3][4];
+    v8h mn;
     float d[4], dmin[4];  // factors of the four rows whose results the lane receives
 };
 
@@ -547,30 +444,21 @@ __device__ __forceinline__ void q5_fold(const uint8_t *T, size_t rb, int b, Q5Fo
     q4k_scales_packed(hd, sc, mn);
     const uint32_t qhw[4] = {qh.x, qh.y, qh.z, qh.w};
     const uint32_t nsh = 4u * (uint32_t)(g >> 1), bsh = 8u * (uint32_t)(g >> 1);
-    o.mn = 0u;
+    o.mn = min_operand(mn);
 #pragma unroll
     for (int jc = 0; jc < 4; ++jc) {
         const int s = 2 * jc + (g >> 1);
         const uint32_t sh = 16u * (uint32_t)(jc & 1) + bsh;  // byte 2 (jc & 1) + g / 2 of word jc / 2
-        const uint32_t scs = (sc[jc >> 1] >> sh) & 0xffu, mns = (mn[jc >> 1] >> sh) & 0xffu;
-        const v2u16b scv = {(unsigned short)scs, (unsigned short)scs};
+        const uint32_t scs = (sc[jc >> 1] >> sh) & 0xffu;
         const uint4 qv = *reinterpret_cast<const uint4 *>(blk + 48 + 32 * jc + 16 * (g & 1));
         const uint32_t qw[4] = {qv.x, qv.y, qv.z, qv.w};
-        int hw[4], lw[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const uint32_t q = ((qw[k] >> nsh) & 0x0f0f0f0fu) | (((qhw[k] >> s) & 0x01010101u) << 4);
-            uint32_t q02, q13;
-            bytes_to_halves(q, q02, q13);
-            const v2u16b w02 = __builtin_bit_cast(v2u16b, q02) * scv, w13 = __builtin_bit_cast(v2u16b, q13) * scv;
-            hw[k] = halves_to_bytes(__builtin_bit_cast(uint32_t, w02 >> (v2u16b){6, 6}),
-                                    __builtin_bit_cast(uint32_t, w13 >> (v2u16b){6, 6}));
-            lw[k] = halves_to_bytes(__builtin_bit_cast(uint32_t, w02 & (v2u16b){63, 63}),
-                                    __builtin_bit_cast(uint32_t, w13 & (v2u16b){63, 63}));
+            o.p[0][jc][k] = nib_mul(q, scs & 3u);
+            o.p[1][jc][k] = nib_mul(q, (scs >> 2) & 3u);
+            o.p[2][jc][k] = nib_mul(q, scs >> 4);
         }
-        o.hi[jc] = v4i{hw[0], hw[1], hw[2], hw[3]};
-        o.lo[jc] = v4i{lw[0], lw[1], lw[2], lw[3]};
-        o.mn |= mns << (8 * jc);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -580,275 +468,416 @@ __device__ __forceinline__ void q5_fold(const uint8_t *T, size_t rb, int b, Q5Fo
     }
 }
 
-__device__ __forceinline__ void q5_fold_step(const Q5Fold &w, const Q6XB &x, float acc[4], float accm[4]) {
-    v4i dh = {0, 0, 0, 0}, dl = {0, 0, 0, 0}, dn = {0, 0, 0, 0};
+__device__ __forceinline__ void fold_step(const Q5Fold &w, const XOps &x, float acc[4], float accm[4]) {
+    v4i d0 = {0, 0, 0, 0}, d1 = {0, 0, 0, 0}, d2 = {0, 0, 0, 0};
+    const v4f dn = mfma_f16(w.mn, x.bs);
 #pragma unroll
     for (int jc = 0; jc < 4; ++jc) {
-        dh = mfma_16x16x64(w.hi[jc], x.x[jc], dh);
-        dl = mfma_16x16x64(w.lo[jc], x.x[jc], dl);
-        const int m4 = splat_byte_of(w.mn, jc);
-        dn = mfma_16x16x64(v4i{m4, m4, m4, m4}, x.x[jc], dn);
+        d0 = mfma_16x16x64(w.p[0][jc], x.x[jc], d0);
+        d1 = mfma_16x16x64(w.p[1][jc], x.x[jc], d1);
+        d2 = mfma_16x16x64(w.p[2][jc], x.x[jc], d2);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int isum = 64 * dh[i] + dl[i];
+        const int isum = 4 * (4 * d2[i] + d1[i]) + d0[i];
         const float dd = w.d[i] * x.xd;
         const float dm = w.dmin[i] * x.xd;
         acc[i] = acc[i] + dd * (float)isum;
-        accm[i] = accm[i] + dm * (float)dn[i];
+        accm[i] = accm[i] + dm * dn[i];
     }
 }
 
-// -- gate/up + SwiGLU for Q3_K rows (OLMoE in its Q3_K_M form) --------------------
+// The fold of a type's super-block from a tile in LDS, and its operands.
+template <int T>
+struct Tile;
+template <>
+struct Tile<kTypeQ4K> {
+    using Fold = Q4Fold;
+    static __device__ __forceinline__ void fold(const uint8_t *t, size_t rb, int b, Fold &o) {
+        Q4Raw raw;
+        q4_raw_load(t, rb, b, raw);
+        q4_fold(raw, o);
+    }
+    static __device__ __forceinline__ void load_x(const Q8L &x, XOps &o) {
+        q4_load_x(x, o);
+        o.bs = load_sums(x);
+    }
+    static __device__ __forceinline__ void step(const Fold &w, const XOps &x, float acc[4], float accm[4]) {
+        q4_fold_step(w, x, acc, accm);
+    }
+};
+template <>
+struct Tile<kTypeQ5K> {
+    using Fold = Q5Fold;
+    static __device__ __forceinline__ void fold(const uint8_t *t, size_t rb, int b, Fold &o) { q5_fold(t, rb, b, o); }
+    static __device__ __forceinline__ void load_x(const Q8L &x, XOps &o) {
+        q6_load_x(x, o);
+        o.bs = load_sums(x);
+    }
+    static __device__ __forceinline__ void step(const Fold &w, const XOps &x, float acc[4], float accm[4]) {
+        fold_step(w, x, acc, accm);
+    }
+};
+template <>
+struct Tile<kTypeQ6K> {
+    using Fold = Q6Fold;
+    static __device__ __forceinline__ void fold(const uint8_t *t, size_t rb, int b, Fold &o) { q6_fold(t, rb, b, o); }
+    static __device__ __forceinline__ void load_x(const Q8L &x, XOps &o) { q6_load_x(x, o); }
+    static __device__ __forceinline__ void step(const Fold &w, const XOps &x, float acc[4], float accm[4]) {
+        fold_step(w, x, acc, accm);
+    }
+};
+
+// The gate/up row types: a lane's raw bytes of a super-block of a 16-row tile
+// from memory, its fold, the fold's operands and step.  pin(): the fold is done
+// before the loads that follow (or their registers are copied every step).
+template <int TG>
+struct GateUp;
+template <>
+struct GateUp<kTypeQ4K> {
+    using Raw = Q4Raw;
+    using Fold = Q4Fold;
+    static constexpr int kDepth = 3;
+    static __device__ __forceinline__ void load(const uint8_t *W, size_t rb, int b, Raw &o) { q4_raw_load(W, rb, b, o); }
+    static __device__ __forceinline__ void fold(const Raw &r, Fold &o) { q4_fold(r, o); }
+    template <class X>
+    static __device__ __forceinline__ void load_x(const X &x, XOps &o) {
+        q4_load_x(x, o);
+    }
+    static __device__ __forceinline__ void step(const Fold &w, const XOps &x, float acc[4], float accm[4]) {
+        q4_fold_step(w, x, acc, accm);
+    }
+    static __device__ __forceinline__ void pin(const Fold &f) {
+        asm volatile("" ::"v"(f.hi[0]), "v"(f.hi[1]), "v"(f.hi[2]), "v"(f.hi[3]), "v"(f.lo[0]), "v"(f.lo[1]),
+                     "v"(f.lo[2]), "v"(f.lo[3])
+                     : "memory");
+    }
+};
+template <>
+struct GateUp<kTypeQ3K> {
+    using Raw = Q3Raw;
+    using Fold = Q3Fold;
+    static constexpr int kDepth = 3;
+    static __device__ __forceinline__ void load(const uint8_t *W, size_t rb, int b, Raw &o) { raw_load(W, rb, b, o); }
+    static __device__ __forceinline__ void fold(const Raw &r, Fold &o) { hoard::fold(r, o); }
+    template <class X>
+    static __device__ __forceinline__ void load_x(const X &x, XOps &o) {
+        q6_load_x(x, o);
+    }
+    static __device__ __forceinline__ void step(const Fold &w, const XOps &x, float acc[4], float accm[4]) {
+        fold_step(w, x, acc, accm);
+    }
+    static __device__ __forceinline__ void pin(const Fold &f) {
+        asm volatile("" ::"v"(f.w[0]), "v"(f.w[1]), "v"(f.w[2]), "v"(f.w[3]), "v"(f.sc) : "memory");
+    }
+};
+// -- gate/up + SwiGLU ------------------------------------------------------------
 // grid (n_ff / 32, max units), block 256: wave w takes rows [32 x + 16 (w % 2), +16)
-// of gate (w < 2) or up (w >= 2).  The 32 rows of each matrix are copied into
-// LDS in one burst (110-byte blocks, 2-byte aligned, read with alignbyte); per
-// super-block each wave folds its rows once (q3_fold) and runs them against
-// every token chunk of the unit.  The gate waves hand their values to the up
-// waves through LDS, which form h.
-template <int NB>
-__global__ __launch_bounds__(256, 2) void pf_gateup_q3_kernel(BatchedArgs a) {
-    constexpr int kRowBytes = NB * kQ3KBytes;
-    constexpr int kTileBytes = 2 * kWaveRows * kRowBytes;  // 32 rows of one matrix
-    static_assert(kRowBytes % 16 == 0, "Q3_K rows of 8 blocks are 880 bytes: tiles start 16-byte aligned");
-    __shared__ __align__(16) uint8_t tile[2][kTileBytes];
-    __shared__ float gx[2][kChunks][4][64];  // gate values: [row tile][chunk][row i][lane]
-    __shared__ float xds[4][kUnitTokens * NB];  // each wave's copy of the tokens' Q8_K block scales
+// of gate (w < 2) or up (w >= 2) of the unit's expert against every token of the
+// unit.  Per super-block the workgroup copies the Q8_K blocks of the unit's
+// token chunks into LDS (one buffer ahead) while each wave holds the next
+// super-block of its rows in registers; the gate waves hand their values to the
+// up waves through LDS, which form h and store it to hbuf[sorted pair][row].
+// Four chunks: three workgroups share a CU (47 KB of LDS each).  Bound by its
+// vector and matrix instructions, which share a SIMD's issue, and the weight
+// stream together: Qwen3-30B at 512 tokens 89 us a launch (226 MB).  Q3_K rows
+// took 174 us at 512 tokens of 64 experts with a tile in LDS and every wave
+// loading its tokens' blocks, 120 here.
+// CH: the 16-token chunks of a unit (units of 16 CH pairs).
+constexpr int kXGran = (int)sizeof(Q8L) / 16;  // 16-byte granules staged per token
+
+template <int TG, int NB, int CH>
+__global__ __launch_bounds__(256, CH == 4 ? 3 : 4) void pf_gateup_kernel(BatchedArgs a) {
+    using S = GateUp<TG>;
+    constexpr int kTok = 16 * CH;
+    constexpr int kXChunksPerBlock = (kTok * kXGran + 63) / 64;  // 1 KB copies per unit block
+    __shared__ __align__(16) Q8L xs[2][kTok];  // the unit's Q8_K block b (two buffers)
+    __shared__ float gx[2][CH][4][64];         // gate values: [row tile][chunk][row i][lane]
     Unit w;
     if (!load_unit(a, blockIdx.y, w)) return;
     const int wave = wave_index(), lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
     const int m = wave >> 1, rt = wave & 1;
-    const int row0 = blockIdx.x * 2 * kWaveRows;
-    // the lane's token of each chunk, read once, while the tile lands
-    int tok[kChunks];
-#pragma unroll
-    for (int ch = 0; ch < kChunks; ++ch) tok[ch] = a.ptok[w.p0 + min(ch * 16 + c, w.n - 1)];
-    // each wave copies its own 16 rows and waits for them alone
-    constexpr int kWaveBytes = kWaveRows * kRowBytes;
-    uint8_t *T = tile[m] + rt * kWaveBytes;
-    dma_wave_copy_nt(T, (m ? batched_up(a, w.e) : batched_gate(a, w.e)) + (size_t)(row0 + rt * kWaveRows) * kRowBytes,
-                     kWaveBytes);
-    // the block scales of the unit's token places, place-major, into the wave's
-    // LDS copy (NB 4-byte copies a lane; the lane's place comes from the lane
-    // that read its token): a 4-byte load of a scale with every chunk's quants
-    // in the loop cost more
-    static_assert(NB == 8, "eight blocks a token: a copy covers eight places");
-    const Q8L *q8xs = reinterpret_cast<const Q8L *>(a.q8x);
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-        const int tk = __shfl(tok[j >> 1], 8 * (j & 1) + (lane >> 3));
-        dma_lanes4(reinterpret_cast<uint8_t *>(&xds[wave][64 * j]),
-                   reinterpret_cast<const uint8_t *>(&q8xs[(size_t)tk * NB + (lane & 7)].d));
-    }
-    lds_dma_wait();
+    const int row0 = blockIdx.x * kGuRows + rt * kWaveRows;
+    constexpr size_t rb = (size_t)NB * QType<TG>::bytes;
+    const uint8_t *W = (m ? batched_up(a, w.e) : batched_gate(a, w.e)) + (size_t)row0 * rb;
     const int nch = (w.n + 15) >> 4;
-    const Q8L *q8x = reinterpret_cast<const Q8L *>(a.q8x);
-    auto x_of = [&](int ch, int b) -> const Q8L & { return q8x[(size_t)tok[ch] * NB + b]; };
-    auto load_x = [&](int ch, int b, Q6XB &o) {
-        q6_load_xq(x_of(ch, b), o);
-        o.xd = xds[wave][(ch * 16 + c) * NB + b];
+    // this lane's granules of the x copy: chunks wave, wave + 4, ...; only the
+    // unit's tokens are copied (the MFMA columns of the places past them read
+    // whatever the buffer holds, and their results are not stored)
+    constexpr int kXJ = (kXChunksPerBlock + 3) / 4;
+    const int ngran = w.n * kXGran;
+    // byte offsets into q8x (it holds at most 512 tokens' blocks): half the
+    // registers of pointers
+    uint32_t xoff[kXJ];
+#pragma unroll
+    for (int j = 0; j < kXJ; ++j) {
+        const int p = 64 * (wave + 4 * j) + lane, tt = min(p / kXGran, kTok - 1), o = p % kXGran;
+        xoff[j] = (uint32_t)a.ptok[w.p0 + min(tt, w.n - 1)] * (uint32_t)(NB * sizeof(Q8L)) + 16u * o;
+    }
+    auto stage_x = [&](int b, int buf) {
+#pragma unroll
+        for (int j = 0; j < kXJ; ++j) {
+            const int ck = wave + 4 * j;
+            if (64 * ck < ngran && 64 * ck + lane < ngran)
+                dma_lanes(reinterpret_cast<uint8_t *>(&xs[buf][0]) + 1024 * ck,
+                          a.q8x + (xoff[j] + (uint32_t)(b * sizeof(Q8L))));
+        }
     };
-    float acc[kChunks][4];
+    float acc[CH][4], accm[CH][4];
 #pragma unroll
-    for (int ch = 0; ch < kChunks; ++ch)
+    for (int ch = 0; ch < CH; ++ch)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[ch][i] = 0.0f;
+        for (int i = 0; i < 4; ++i) acc[ch][i] = accm[ch][i] = 0.0f;
+    typename S::Raw raw;
+    S::load(W, rb, 0, raw);
+    stage_x(0, 0);
 #pragma unroll 1
     for (int b = 0; b < NB; ++b) {
-        // every chunk's activation operands in flight before the fold, which covers them
-        Q6XB xc[kChunks];
+        // Other waves read the x chunks this wave copied: the compiler does not
+        // see the copies, so the wave waits for its own before the barrier (it
+        // waits for the raw weight loads of block b there anyway).
+        lds_dma_wait();
+        __syncthreads();  // every wave's copies of x(b) landed, and x(b - 1) is read
+        typename S::Fold t;
+        S::fold(raw, t);
+        S::pin(t);
+        // the next super-block's activation copies issue before its weight
+        // loads (both are waited for at the next super-block; copies first
+        // measured 3 % faster for the layer at 512 tokens)
+        if (b + 1 < NB) {
+            stage_x(b + 1, (b + 1) & 1);
+            S::load(W, rb, b + 1, raw);
+        }
+        const Q8L *xb = xs[b & 1];
 #pragma unroll
-        for (int ch = 0; ch < kChunks; ++ch)
-            if (ch < nch) load_x(ch, b, xc[ch]);
-        Q3Fold f;
-        q3_fold(T, kRowBytes, b, f);
-#pragma unroll
-        for (int ch = 0; ch < kChunks; ++ch)
-            if (ch < nch) q3_fold_step(f, xc[ch], acc[ch]);
+        for (int ch = 0; ch < CH; ++ch)
+            if (ch < nch) {
+                const Q8L &x = xb[ch * 16 + c];
+                XOps xo;
+                S::load_x(x, xo);
+                xo.bs = load_sums(x);
+                xo.xd = x.d;
+                S::step(t, xo, acc[ch], accm[ch]);
+            }
     }
     if (m == 0) {
 #pragma unroll
-        for (int ch = 0; ch < kChunks; ++ch)
+        for (int ch = 0; ch < CH; ++ch)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) gx[rt][ch][i][lane] = acc[ch][i];
+            for (int i = 0; i < 4; ++i) gx[rt][ch][i][lane] = acc[ch][i] - accm[ch][i];
     }
     __syncthreads();
     if (m == 0) return;
 #pragma unroll
-    for (int ch = 0; ch < kChunks; ++ch) {
+    for (int ch = 0; ch < CH; ++ch) {
         const int idx = ch * 16 + c;
         if (ch < nch && idx < w.n) {
             float hv[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float g = gx[rt][ch][i][lane], uu = acc[ch][i];
+                const float g = gx[rt][ch][i][lane], uu = acc[ch][i] - accm[ch][i];
                 hv[i] = g / (1.0f + expf(-g)) * uu;
             }
-            *reinterpret_cast<float4 *>(a.hbuf + (size_t)(w.p0 + idx) * a.n_ff + row0 + rt * kWaveRows + 4 * q) =
+            *reinterpret_cast<float4 *>(a.hbuf + (size_t)(w.p0 + idx) * a.n_ff + row0 + 4 * q) =
                 make_float4(hv[0], hv[1], hv[2], hv[3]);
         }
     }
 }
 
-// grid (n_embd / 64, max units), block 256: as pf_down_q4_kernel for Q6_K rows,
-// super-block major: each super-block of the wave's 16 rows is folded once,
-// then run against every token chunk of the unit, the next chunk's activation
-// operands in flight meanwhile.  Three workgroups per CU (166 VGPRs).
-template <int NBH>
-__global__ __launch_bounds__(256, 3) void pf_down_q6_kernel(BatchedArgs a) {
-    constexpr int kRowBytes = NBH * kQ6KBytes;
-    constexpr int kTileBytes = kDnRows * kRowBytes;
-    static_assert(kTileBytes % 16 == 0, "the tile copies in 16-byte units");
-    __shared__ __align__(16) uint8_t tile[kTileBytes];
-    __shared__ int yrow[kUnitTokens];  // y row (token * slots + slot) of each of the unit's pairs
-    __shared__ __align__(16) float xds[4][kUnitTokens][4];  // each wave's copy of the pairs' Q8_K(h) scales
+// -- gate/up + SwiGLU for units of at most 16 pairs ------------------------------
+// grid (n_ff / 32, max units), block 256, waves as above.  With one token chunk
+// a wave's registers leave room for kDepth super-blocks of raw weights in
+// flight, and all of the unit's activation blocks fit LDS at once (39 KB, four
+// workgroups a CU): one barrier after they land, then every wave streams its
+// rows from memory at its own pace.  Qwen3.5 at 131 tokens (302 MB): 85 -> 72 us
+// a launch against units of 64; Q3_K at 27
+// tokens 75 (per-token dots) -> 54.
+// The quants and scale of a Q8_K block in LDS (17 granules: 16 tokens' reads
+// of one place fall into different banks).
+struct Q8S {
+    int32_t qs[64];
+    float d;
+    int32_t pad[3];
+};
+static_assert(sizeof(Q8S) == 272 && offsetof(Q8L, d) == 288 && offsetof(Q8L, bsums) == 256, "Q8S from Q8L");
+
+template <int TG, int NB>
+__global__ __launch_bounds__(256, 4) void pf_gateup16_kernel(BatchedArgs a) {
+    using S = GateUp<TG>;
+    constexpr int D = S::kDepth, kGran = (int)sizeof(Q8S) / 16, kCopies = (16 * kGran + 63) / 64;
+    static_assert(NB % 4 == 0 && NB >= D, "a wave copies NB / 4 blocks of every token");
+    __shared__ __align__(16) Q8S xs[NB][16];
+    __shared__ __align__(16) v8h sums[NB][32];
     Unit w;
     if (!load_unit(a, blockIdx.y, w)) return;
     const int wave = wave_index(), lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
-    const int rt0 = blockIdx.x * kDnRows;
-    const int nch = (w.n + 15) >> 4;
-    const Q8L *q8h = reinterpret_cast<const Q8L *>(a.q8h);
-    auto x_of = [&](int ch, int b) -> const Q8L & {
-        return q8h[(size_t)(w.p0 + min(ch * 16 + c, w.n - 1)) * NBH + b];
-    };
-    // the pairs' block scales come from the wave's LDS copy, copied with the
-    // tile: a 4-byte load of a scale with every chunk's quants cost more
-    auto load_x = [&](int ch, int b, Q6XB &o) {
-        q6_load_xq(x_of(ch, b), o);
-        o.xd = xds[wave][min(ch * 16 + c, kUnitTokens - 1)][b];
-    };
-    // Chunk ch of a super-block takes its activation operands from x[ch % 2]:
-    // chunk 0's are loaded before the fold, each later chunk's while the one
-    // before it computes.
-    static_assert(kChunks == 4, "four chunks, two operand sets");
-    Q6XB x0, x1;
-    // the pairs' places, read while the tile lands
-    const int tid = threadIdx.x;
-    const int pt = tid < w.n ? a.ptok[w.p0 + tid] : 0, ps = tid < w.n ? a.pslot[w.p0 + tid] : 0;
-    // each wave copies its own 16 rows and waits for them alone: no barrier
-    // between the copies and the folds
-    constexpr int kWaveBytes = kWaveRows * kRowBytes;
-    static_assert(kWaveBytes % 16 == 0, "a wave's rows copy in 16-byte units");
-    uint8_t *T = tile + wave * kWaveBytes;
-    dma_lanes(reinterpret_cast<uint8_t *>(&xds[wave][0][0]),
-              reinterpret_cast<const uint8_t *>(a.q8hd + (size_t)(w.p0 + min(lane, w.n - 1)) * 4));
-    dma_wave_copy_nt(T, batched_down(a, w.e) + (size_t)(rt0 + wave * kWaveRows) * kRowBytes, kWaveBytes);
+    const int m = wave >> 1, rt = wave & 1;
+    const int row0 = blockIdx.x * kGuRows + rt * kWaveRows;
+    constexpr size_t rb = (size_t)NB * QType<TG>::bytes;
+    const uint8_t *W = (m ? batched_up(a, w.e) : batched_gate(a, w.e)) + (size_t)row0 * rb;
+    // the tokens of this lane's granules, then the first weights, then the copies
+    int tk[kCopies + 1];
+#pragma unroll
+    for (int j = 0; j <= kCopies; ++j) {
+        const int tt = j < kCopies ? (64 * j + lane) / kGran : lane >> 1;
+        tk[j] = a.ptok[w.p0 + min(tt, w.n - 1)];
+    }
+    asm volatile("" ::: "memory");
+    typename S::Raw raw[D];
+#pragma unroll
+    for (int i = 0; i < D; ++i) S::load(W, rb, i, raw[i]);
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < NB / 4; ++i) {
+        const int b = wave * (NB / 4) + i;
+        const uint32_t blk = (uint32_t)(b * (int)sizeof(Q8L));
+#pragma unroll
+        for (int j = 0; j < kCopies; ++j) {
+            const int p = 64 * j + lane, o = p % kGran;
+            if (64 * j < w.n * kGran && p < w.n * kGran)
+                dma_lanes(reinterpret_cast<uint8_t *>(&xs[b][0]) + 1024 * j,
+                          a.q8x + ((uint32_t)tk[j] * (uint32_t)(NB * sizeof(Q8L)) + blk + 16u * (o < 16 ? o : 18)));
+        }
+        if (lane < 2 * w.n)
+            dma_lanes(reinterpret_cast<uint8_t *>(&sums[b][0]),
+                      a.q8x + ((uint32_t)tk[kCopies] * (uint32_t)(NB * sizeof(Q8L)) + blk + 256u + 16u * (lane & 1)));
+    }
     lds_dma_wait();
-    if (tid < w.n) yrow[tid] = pt * (a.k + a.sh) + ps;
-    float acc[kChunks][4];
+    __syncthreads();
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f}, accm[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int ch = 0; ch < kChunks; ++ch)
+    for (int b = 0; b < NB; ++b) {
+        typename S::Fold f;
+        S::fold(raw[b % D], f);
+        S::pin(f);  // the fold is done before its registers are loaded again
+        if (b + D < NB) S::load(W, rb, b + D, raw[b % D]);
+        const Q8S &x = xs[b][c];
+        XOps xo;
+        xo.xd = x.d;
+        xo.bs = sums[b][2 * c + (q & 1)];
+        S::load_x(x, xo);
+        S::step(f, xo, acc, accm);
+    }
+    // the gate waves hand their values to the up waves over the activations
+    __syncthreads();
+    float *gx = reinterpret_cast<float *>(&xs[0][0]) + (size_t)rt * 256;
+    if (m == 0) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[ch][i] = 0.0f;
+        for (int i = 0; i < 4; ++i) gx[64 * i + lane] = acc[i] - accm[i];
+    }
+    __syncthreads();
+    if (m == 0 || c >= w.n) return;
+    float hv[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float g = gx[64 * i + lane], uu = acc[i] - accm[i];
+        hv[i] = g / (1.0f + expf(-g)) * uu;
+    }
+    *reinterpret_cast<float4 *>(a.hbuf + (size_t)(w.p0 + c) * a.n_ff + row0 + 4 * q) =
+        make_float4(hv[0], hv[1], hv[2], hv[3]);
+}
+
+// -- down: 64 rows of the unit's expert, y to its (token, slot) place -----------
+// grid (n_embd / 64, max units), block 256.  Each wave copies its own 16 rows
+// into LDS in one burst and waits for them alone (no barrier before the folds);
+// each super-block of them is folded once, then run against every token chunk
+// of the unit (CH of 16 pairs).  TS: the shared expert's row type beside
+// routed rows of type TD (Qwen3.5: Q6_K beside Q5_K), in the same launch.
+// With four chunks, Q6_K keeps two operand sets (chunk ch's loaded while the one
+// before it computes, three workgroups a CU); Q4_K and Q5_K load every chunk's
+// before the fold, which covers them, and one chunk always is.
+template <int T, int NBH, int CH>
+__device__ __forceinline__ void down_rows16(const uint8_t *tile, int nch, const Q8L *x0, const int (&xi)[CH],
+                                            const float (*xds)[4], float (&acc)[CH][4], float (&accm)[CH][4]) {
+    using K = Tile<T>;
+    const int c = threadIdx.x & 15;
+    auto load_x = [&](int ch, int b, XOps &o) {
+        K::load_x(x0[(size_t)xi[ch] * NBH + b], o);
+        o.xd = xds[ch * 16 + c][b];
+    };
 #pragma unroll 1
     for (int b = 0; b < NBH; ++b) {
-        load_x(0, b, x0);
-        Q6Fold f;
-        q6_fold(T, kRowBytes, b, f);
-        if (nch > 1) load_x(1, b, x1);
-        q6_fold_step(f, x0, acc[0]);
-        if (nch > 1) {
-            if (nch > 2) load_x(2, b, x0);
-            q6_fold_step(f, x1, acc[1]);
-            if (nch > 2) {
-                if (nch > 3) load_x(3, b, x1);
-                q6_fold_step(f, x0, acc[2]);
-                if (nch > 3) q6_fold_step(f, x1, acc[3]);
+        typename K::Fold f;
+        if constexpr (T == kTypeQ6K && CH == 4) {
+            XOps xa, xb;
+            load_x(0, b, xa);
+            K::fold(tile, NBH * QType<T>::bytes, b, f);
+            if (nch > 1) load_x(1, b, xb);
+            K::step(f, xa, acc[0], accm[0]);
+            if (nch > 1) {
+                if (nch > 2) load_x(2, b, xa);
+                K::step(f, xb, acc[1], accm[1]);
+                if (nch > 2) {
+                    if (nch > 3) load_x(3, b, xb);
+                    K::step(f, xa, acc[2], accm[2]);
+                    if (nch > 3) K::step(f, xb, acc[3], accm[3]);
+                }
             }
-        }
-    }
-    __syncthreads();  // yrow is written
+        } else {
+            XOps xc[CH];
 #pragma unroll
-    for (int ch = 0; ch < kChunks; ++ch) {
-        const int idx = ch * 16 + c;
-        if (ch < nch && idx < w.n) {
-            *reinterpret_cast<float4 *>(a.ybuf + (size_t)yrow[idx] * a.n_embd + rt0 + wave * kWaveRows + 4 * q) =
-                make_float4(acc[ch][0], acc[ch][1], acc[ch][2], acc[ch][3]);
+            for (int ch = 0; ch < CH; ++ch)
+                if (ch < nch) load_x(ch, b, xc[ch]);
+            K::fold(tile, NBH * QType<T>::bytes, b, f);
+#pragma unroll
+            for (int ch = 0; ch < CH; ++ch)
+                if (ch < nch) K::step(f, xc[ch], acc[ch], accm[ch]);
         }
     }
 }
 
-// grid (n_embd / 64, max units), block 256: Q5_K down rows folded as the Q6_K
-// ones are (each super-block of the wave's 16 rows folded once, then run against
-// every token chunk of the unit); TS = Q6_K: the shared expert's Q6_K rows
-// beside them (Qwen3.5), a unit of which takes the Q6_K fold.
-template <int NBH, int TS>
-__global__ __launch_bounds__(256, 2) void pf_down_q5_kernel(BatchedArgs a) {
-    constexpr int kRowBytesD = NBH * kQ5KBytes, kRowBytesS = NBH * QType<TS>::bytes;
+template <int TD, int NBH, int TS, int CH>
+constexpr int kDownWaves = CH == 1 ? 4 : (CH == 2 || TD == kTypeQ6K) ? 3 : 2;  // waves a SIMD (register bound)
+
+template <int TD, int NBH, int TS, int CH>
+__global__ __launch_bounds__(256, (kDownWaves<TD, NBH, TS, CH>)) void pf_down_kernel(BatchedArgs a) {
+    constexpr int kRowBytesD = NBH * QType<TD>::bytes, kRowBytesS = NBH * QType<TS>::bytes;
     constexpr int kTileBytes = kDnRows * (kRowBytesD > kRowBytesS ? kRowBytesD : kRowBytesS);
-    static_assert(TS == kTypeQ5K || TS == kTypeQ6K, "the shared expert's down rows are Q5_K or Q6_K");
+    static_assert(kWaveRows * kRowBytesD % 16 == 0 && kWaveRows * kRowBytesS % 16 == 0, "16-byte copies");
     __shared__ __align__(16) uint8_t tile[kTileBytes];
-    __shared__ int yrow[kUnitTokens];  // y row (token * slots + slot) of each of the unit's pairs
-    __shared__ __align__(16) float xds[4][kUnitTokens][4];  // each wave's copy of the pairs' Q8_K(h) scales
+    __shared__ int yrow[16 * CH];  // y row (token * slots + slot) of each of the unit's pairs
+    __shared__ __align__(16) float xds[4][16 * CH][4];  // each wave's copy of the pairs' Q8_K(h) scales
     Unit w;
     if (!load_unit(a, blockIdx.y, w)) return;
-    const bool shx = TS != kTypeQ5K && a.sh && w.e == a.n_ids;  // the shared expert's Q6_K rows
-    const int rbytes = shx ? kRowBytesS : kRowBytesD;
+    const bool shx = TS != TD && a.sh && w.e == a.n_ids;  // the shared expert's rows
     const int wave = wave_index(), lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
     const int rt0 = blockIdx.x * kDnRows;
     // the pairs' places, read while the tile lands
     const int tid = threadIdx.x;
     const int pt = tid < w.n ? a.ptok[w.p0 + tid] : 0, ps = tid < w.n ? a.pslot[w.p0 + tid] : 0;
-    // each wave copies its own 16 rows and waits for them alone
-    const int wbytes = kWaveRows * rbytes;  // a multiple of 16 for both row types
+    const int wbytes = kWaveRows * (shx ? kRowBytesS : kRowBytesD);
     uint8_t *T = tile + wave * wbytes;
-    dma_lanes(reinterpret_cast<uint8_t *>(&xds[wave][0][0]),
-              reinterpret_cast<const uint8_t *>(a.q8hd + (size_t)(w.p0 + min(lane, w.n - 1)) * 4));
-    dma_wave_copy_nt(T, batched_down(a, w.e) + (size_t)(rt0 + wave * kWaveRows) * rbytes, wbytes);
+    // the pairs' block scales with the tile: a 4-byte load of a scale with every
+    // chunk's quants cost more
+    if (CH == 4 || lane < 16 * CH)
+        dma_lanes(reinterpret_cast<uint8_t *>(&xds[wave][0][0]),
+                  reinterpret_cast<const uint8_t *>(a.q8hd + (size_t)(w.p0 + min(lane, w.n - 1)) * 4));
+    dma_wave_copy_nt(T, batched_down(a, w.e) + (size_t)(rt0 + wave * kWaveRows) * (wbytes / kWaveRows), wbytes);
     lds_dma_wait();
     if (tid < w.n) yrow[tid] = pt * (a.k + a.sh) + ps;
     const int nch = (w.n + 15) >> 4;
-    const Q8L *q8h = reinterpret_cast<const Q8L *>(a.q8h);
-    auto x_of = [&](int ch, int b) -> const Q8L & {
-        return q8h[(size_t)(w.p0 + min(ch * 16 + c, w.n - 1)) * NBH + b];
-    };
-    // the quants from memory, the pairs' block scales from the wave's LDS copy
-    auto load_x = [&](int ch, int b, Q6XB &o) {
-        q6_load_xq(x_of(ch, b), o);
-        o.xd = xds[wave][min(ch * 16 + c, kUnitTokens - 1)][b];
-    };
-    float acc[kChunks][4], accm[kChunks][4];
+    const Q8L *x0 = reinterpret_cast<const Q8L *>(a.q8h) + (size_t)w.p0 * NBH;
+    int xi[CH];  // the lane's pair of each chunk (places past the last repeat it)
 #pragma unroll
-    for (int ch = 0; ch < kChunks; ++ch)
+    for (int ch = 0; ch < CH; ++ch) xi[ch] = min(ch * 16 + c, w.n - 1);
+    float acc[CH][4], accm[CH][4];
+#pragma unroll
+    for (int ch = 0; ch < CH; ++ch)
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[ch][i] = accm[ch][i] = 0.0f;
-    if (shx) {
-        if constexpr (TS == kTypeQ6K) {
-#pragma unroll 1
-            for (int b = 0; b < NBH; ++b) {
-                Q6XB xc[kChunks];
-#pragma unroll
-                for (int ch = 0; ch < kChunks; ++ch)
-                    if (ch < nch) load_x(ch, b, xc[ch]);
-                Q6Fold f;
-                q6_fold(T, kRowBytesS, b, f);
-#pragma unroll
-                for (int ch = 0; ch < kChunks; ++ch)
-                    if (ch < nch) q6_fold_step(f, xc[ch], acc[ch]);
-            }
-        }
-    } else {
-#pragma unroll 1
-        for (int b = 0; b < NBH; ++b) {
-            Q6XB xc[kChunks];
-#pragma unroll
-            for (int ch = 0; ch < kChunks; ++ch)
-                if (ch < nch) load_x(ch, b, xc[ch]);
-            Q5Fold f;
-            q5_fold(T, kRowBytesD, b, f);
-#pragma unroll
-            for (int ch = 0; ch < kChunks; ++ch)
-                if (ch < nch) q5_fold_step(f, xc[ch], acc[ch], accm[ch]);
-        }
-    }
+    if (TS != TD && shx)
+        down_rows16<TS, NBH, CH>(T, nch, x0, xi, xds[wave], acc, accm);
+    else
+        down_rows16<TD, NBH, CH>(T, nch, x0, xi, xds[wave], acc, accm);
     __syncthreads();  // yrow is written
 #pragma unroll
-    for (int ch = 0; ch < kChunks; ++ch) {
+    for (int ch = 0; ch < CH; ++ch) {
         const int idx = ch * 16 + c;
         if (ch < nch && idx < w.n) {
+            // accm stays 0 for rows without a min term
             *reinterpret_cast<float4 *>(a.ybuf + (size_t)yrow[idx] * a.n_embd + rt0 + wave * kWaveRows + 4 * q) =
                 make_float4(acc[ch][0] - accm[ch][0], acc[ch][1] - accm[ch][1], acc[ch][2] - accm[ch][2],
-                            acc[ch][3] - accm[ch][3]);  // accm stays 0 for Q6_K rows
+                            acc[ch][3] - accm[ch][3]);
         }
     }
 }
@@ -904,36 +933,56 @@ __global__ __launch_bounds__(256) void pf_combine_kernel(BatchedArgs a) {
 
 }  // namespace
 
-hipError_t launch_prefill_groups(const BatchedArgs &a, hipStream_t s) {
+namespace {
+
+template <int CH>
+hipError_t launch_units(const BatchedArgs &a, hipStream_t s) {
     const int nbh = a.n_ff / QK;
-    if (a.n_embd != 2048 || a.n_ff % kGuRows || a.n_embd % kDnRows || nbh > 4 || a.max_units < 1)
+    const dim3 gg(a.n_ff / kGuRows, a.max_units);
+    if (a.gu_type == kTypeQ4K) {
+        if constexpr (CH == 1)
+            hipLaunchKernelGGL((pf_gateup16_kernel<kTypeQ4K, 8>), gg, dim3(256), 0, s, a);
+        else
+            hipLaunchKernelGGL((pf_gateup_kernel<kTypeQ4K, 8, CH>), gg, dim3(256), 0, s, a);
+    } else if (a.gu_type == kTypeQ3K) {
+        if constexpr (CH == 1)
+            hipLaunchKernelGGL((pf_gateup16_kernel<kTypeQ3K, 8>), gg, dim3(256), 0, s, a);
+        else
+            hipLaunchKernelGGL((pf_gateup_kernel<kTypeQ3K, 8, CH>), gg, dim3(256), 0, s, a);
+    } else {
         return hipErrorInvalidValue;
-    if (a.gu_type == kTypeQ4K)
-        hipLaunchKernelGGL(pf_gateup_kernel<8>, dim3(a.n_ff / kGuRows, a.max_units), dim3(256), 0, s, a);
-    else if (a.gu_type == kTypeQ3K)
-        hipLaunchKernelGGL(pf_gateup_q3_kernel<8>, dim3(a.n_ff / kGuRows, a.max_units), dim3(256), 0, s, a);
-    else
-        return hipErrorInvalidValue;
+    }
     hipLaunchKernelGGL(pf_quant_h_kernel, dim3(a.M * (a.k + a.sh)), dim3(64 * nbh), 0, s, a);
     const dim3 dg(a.n_embd / kDnRows, a.max_units);
     const int sd = a.sh ? a.sh_d_type : a.d_type;
 // one kernel instance per (routed down type, super-blocks per row, shared down type)
-#define HOARD_DOWN(T, N, TS, K)                                          \
-    if (a.d_type == T && nbh == N && sd == TS) {                         \
-        hipLaunchKernelGGL((K), dg, dim3(256), 0, s, a);                 \
+#define HOARD_DOWN(T, N, TS)                                                          \
+    if (a.d_type == T && nbh == N && sd == TS) {                                      \
+        hipLaunchKernelGGL((pf_down_kernel<T, N, TS, CH>), dg, dim3(256), 0, s, a);   \
     } else
-    HOARD_DOWN(kTypeQ6K, 3, kTypeQ6K, pf_down_q6_kernel<3>)
-    HOARD_DOWN(kTypeQ6K, 2, kTypeQ6K, pf_down_q6_kernel<2>)
-    HOARD_DOWN(kTypeQ6K, 4, kTypeQ6K, pf_down_q6_kernel<4>)
-    HOARD_DOWN(kTypeQ4K, 4, kTypeQ4K, pf_down_q4_kernel<4>)
-    HOARD_DOWN(kTypeQ4K, 3, kTypeQ4K, pf_down_q4_kernel<3>)
-    HOARD_DOWN(kTypeQ4K, 2, kTypeQ4K, pf_down_q4_kernel<2>)
-    HOARD_DOWN(kTypeQ5K, 4, kTypeQ5K, (pf_down_q5_kernel<4, kTypeQ5K>))
-    HOARD_DOWN(kTypeQ5K, 2, kTypeQ5K, (pf_down_q5_kernel<2, kTypeQ5K>))
-    HOARD_DOWN(kTypeQ5K, 2, kTypeQ6K, (pf_down_q5_kernel<2, kTypeQ6K>)) {
+    HOARD_DOWN(kTypeQ6K, 3, kTypeQ6K)
+    HOARD_DOWN(kTypeQ6K, 2, kTypeQ6K)
+    HOARD_DOWN(kTypeQ6K, 4, kTypeQ6K)
+    HOARD_DOWN(kTypeQ4K, 4, kTypeQ4K)
+    HOARD_DOWN(kTypeQ4K, 3, kTypeQ4K)
+    HOARD_DOWN(kTypeQ4K, 2, kTypeQ4K)
+    HOARD_DOWN(kTypeQ5K, 4, kTypeQ5K)
+    HOARD_DOWN(kTypeQ5K, 2, kTypeQ5K)
+    HOARD_DOWN(kTypeQ5K, 2, kTypeQ6K) {
         return hipErrorInvalidValue;
     }
 #undef HOARD_DOWN
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_prefill_groups(const BatchedArgs &a, hipStream_t s) {
+    if (a.n_embd != 2048 || a.n_ff % kGuRows || a.n_embd % kDnRows || a.n_ff / QK > 4 || a.max_units < 1)
+        return hipErrorInvalidValue;
+    const hipError_t e = a.unit == 16 ? launch_units<1>(a, s) : a.unit == 32 ? launch_units<2>(a, s)
+                         : a.unit == kUnitTokens ? launch_units<4>(a, s) : hipErrorInvalidValue;
+    if (e != hipSuccess || a.M <= kBatchedMaxTokens) return e;  // (a small batch's combine follows the caller)
     hipLaunchKernelGGL(pf_combine_kernel, dim3((a.n_embd + 1023) / 1024, a.M), dim3(256), 0, s, a);
     return hipGetLastError();
 }

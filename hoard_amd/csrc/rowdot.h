@@ -25,13 +25,21 @@ static_assert(sizeof(Q8L) == 304, "Q8L is 19 x 16 bytes");
 // Wave quantisation of 256 floats to Q8_K (ggml quantize_row_q8_K semantics:
 // largest |x| with its sign, first index on ties; iscale = -127/max;
 // q = min(127, nearest_int(iscale*x)); d = 1/iscale; all-zero block -> 0).
+// What the place of the block's 16-element sums holds: the sums as int16 (the
+// per-token dots), or the exact fp16 forms the MFMA units read: the sums S_s
+// of the eight 32-element sub-blocks, halves 0..7 with bit 0 cleared (even and
+// at most 4064 in magnitude) and halves 8..15 that bit (kSums32, types with a
+// min term); or the sixteen 16-element sums (at most 2032; kSums16, Q3_K).
+constexpr int kSumsInt = 0, kSums32 = 1, kSums16 = 2;
+template <int Sums = kSumsInt>
 __device__ __forceinline__ float wave_quantize_q8l_regs(const float v[4], Q8L *out);
 // Returns the block's scale d (in every lane).
+template <int Sums = kSumsInt>
 __device__ __forceinline__ float wave_quantize_q8l(const float *x, Q8L *out) {
     const int lane = threadIdx.x & 63;
     const float4 v4 = *reinterpret_cast<const float4 *>(x + 4 * lane);
     const float v[4] = {v4.x, v4.y, v4.z, v4.w};
-    return wave_quantize_q8l_regs(v, out);
+    return wave_quantize_q8l_regs<Sums>(v, out);
 }
 
 // One Q4_K row of nb super-blocks (16-byte aligned in LDS) dotted with x.
@@ -569,6 +577,7 @@ __device__ __forceinline__ unsigned wave_max_bits(unsigned u) {
 // patterns cleared to 0 first), which orders them as the values would be, so
 // the wave max is an integer max and the element that holds it is found with
 // one compare per element, one ballot and one read of its lane.
+template <int Sums>
 __device__ __forceinline__ float wave_quantize_q8l_regs(const float v[4], Q8L *out) {
     const int lane = threadIdx.x & 63;
     unsigned b[4];
@@ -599,8 +608,18 @@ __device__ __forceinline__ float wave_quantize_q8l_regs(const float v[4], Q8L *o
         packed |= ((uint32_t)(q & 0xff)) << (8 * i);
     }
     out->qs[lane] = (int32_t)packed;
-    s = group4_sum(s);
-    if ((lane & 3) == 0) out->bsums[lane >> 2] = (int16_t)s;
+    _Float16 *hs = reinterpret_cast<_Float16 *>(out->bsums);
+    if constexpr (Sums == kSums32) {
+        s = group8_sum(s);
+        if ((lane & 7) == 0) hs[lane >> 3] = (_Float16)(s & ~1);
+        if ((lane & 7) == 1) hs[8 + (lane >> 3)] = (_Float16)(s & 1);
+    } else if constexpr (Sums == kSums16) {
+        s = group4_sum(s);
+        if ((lane & 3) == 0) hs[lane >> 2] = (_Float16)s;
+    } else {
+        s = group4_sum(s);
+        if ((lane & 3) == 0) out->bsums[lane >> 2] = (int16_t)s;
+    }
     const float d = 1.0f / iscale;
     if (lane == 0) out->d = d;
     return d;
