@@ -21,6 +21,7 @@ struct RouterArgs {
     unsigned *counters;    // [M], zero on entry, left zero on exit
     int32_t *sel;          // [M][k]
     float *wsel;           // [M][k]
+    int32_t *sel_host;     // [k] the selection again, in pinned host memory (null: not wanted)
 };
 hipError_t launch_router(const RouterArgs &a, hipStream_t s);
 
@@ -253,6 +254,20 @@ hipError_t launch_layer_route(const RouterArgs &a, hipStream_t s);
 bool layer_ffn_ok(const GateUpArgs &g, const DownArgs &d);
 hipError_t launch_layer_gateup(const GateUpArgs &g, hipStream_t s);
 hipError_t launch_layer_down(const DownArgs &d, hipStream_t s);
+
+// A slot pool's step on the compute stream: expert records copied from pinned
+// host memory into their slots, and the slot ids of the selection (pool.hip).
+constexpr int kMaxSlotIds = 16;
+struct SlotFill {
+    const uint8_t *src[kMaxSlotIds];  // pinned host records, 16-byte aligned
+    uint8_t *dst[kMaxSlotIds];        // their slots
+    size_t bytes;                     // per record, a multiple of 16
+    int n;                            // records to copy
+    int32_t slot[kMaxSlotIds];        // the selection's slots
+    int32_t *slot_dev;                // [n_ids]
+    int n_ids;
+};
+hipError_t launch_slot_fill(const SlotFill &a, hipStream_t s);
 
 size_t block_bytes(int type);
 

@@ -300,7 +300,7 @@ struct KernelMark {
 };
 
 int run_route(hoard_moe *h, const Layer &L, const float *xin, int is_residual, float eps, int32_t *sel,
-              float *w, hipStream_t s) {
+              float *w, hipStream_t s, int32_t *sel_host = nullptr) {
     const hoard_moe_cfg &c = h->cfg;
     hoard::RouterArgs a{};
     a.xin = xin;
@@ -317,6 +317,7 @@ int run_route(hoard_moe *h, const Layer &L, const float *xin, int is_residual, f
     a.counters = h->counters;
     a.sel = sel;
     a.wsel = w;
+    a.sel_host = sel_host;
     const bool fast = h->layer_kernels && hoard::layer_route_ok(a) &&
                       ((reinterpret_cast<uintptr_t>(xin) | reinterpret_cast<uintptr_t>(L.router)) & 15) == 0;
     KernelMark mark(h, HOARD_KERNEL_ROUTER, s);
@@ -464,7 +465,7 @@ void pool_abandon(hoard_moe *h, int layer, const hipStream_t *up) {
 }
 
 int pool_ensure(hoard_moe *h, int layer, const int32_t *sel, int n, bool sequential, int32_t *slot_host,
-                int32_t *slot_dev, hipStream_t s, hipStream_t cs) {
+                int32_t *slot_dev, hipStream_t s, hipStream_t cs, bool fill = false) {
     const hoard_moe_cfg &c = h->cfg;
     Layer &L = h->layers[layer];
     for (int j = 0; j < n; ++j)
@@ -491,6 +492,33 @@ int pool_ensure(hoard_moe *h, int layer, const int32_t *sel, int n, bool sequent
             return fail(HOARD_ERR_HIP, "%s: %s", #expr, hipGetErrorString(e_));                  \
         }                                                                                        \
     } while (0)
+    // fill: an on-demand layer, on the compute stream itself: one kernel copies
+    // the records and writes the slot ids, in stream order after the last FFN
+    // that read the slots (an event wait where that ran on another stream)
+    if (fill) {
+        hipStream_t up[kUpStreams];
+        for (int i = 0; i < kUpStreams; ++i) up[i] = s;
+        hoard::SlotFill f{};
+        f.bytes = L.gstride;
+        f.slot_dev = slot_dev;
+        f.n_ids = n;
+        for (int j = 0; j < n; ++j) {
+            f.slot[j] = slots[j];
+            h->stats.reqs += 1;
+            if (!miss[j]) {
+                h->stats.hits += 1;
+                continue;
+            }
+            if (h->fail_upload > 0 && --h->fail_upload == 0) POOL_TRY(hipErrorOutOfMemory);
+            f.src[f.n] = L.host_experts + (size_t)sel[j] * f.bytes;
+            f.dst[f.n++] = L.slots + (size_t)slots[j] * f.bytes;
+            h->stats.misses += 1;
+            h->stats.bytes_h2d += f.bytes;
+        }
+        if (f.n && L.used) POOL_TRY(hipStreamWaitEvent(s, L.last_use, 0));
+        POOL_TRY(hoard::launch_slot_fill(f, s));
+        return HOARD_OK;
+    }
     // misses are dealt round-robin to the caller's copy stream and the internal
     // ones; each first waits until the last FFN reading this layer's slots is done
     hipStream_t up[kUpStreams];
@@ -576,12 +604,14 @@ int pool_mark_use(hoard_moe *h, int layer, hipStream_t s) {
     return HOARD_OK;
 }
 
-// On-demand pool step after a device-side route: the selection is read back
-// (the reference's D2H of sel, :367), then the slots are ensured.
-int pool_after_route(hoard_moe *h, int layer, const int32_t *sel_dev, int32_t *slot_dev, hipStream_t s) {
-    HIP_TRY(hipMemcpyAsync(h->pin_sel, sel_dev, sizeof(int32_t) * h->cfg.n_used, hipMemcpyDeviceToHost, s));
+// On-demand pool step after a device-side route, which left the selection in
+// pinned host memory (the reference's D2H of sel, :367): once the stream has
+// reached it the slots are ensured.
+int pool_after_route(hoard_moe *h, int layer, int32_t *slot_dev, hipStream_t s) {
     HIP_TRY(hipStreamSynchronize(s));
-    return pool_ensure(h, layer, h->pin_sel, h->cfg.n_used, false, nullptr, slot_dev, s, s);
+    // the storage tier's entries are fenced per copy and keep the copy streams
+    const bool fill = !h->store && (h->layers[layer].gstride % 16) == 0;
+    return pool_ensure(h, layer, h->pin_sel, h->cfg.n_used, false, nullptr, slot_dev, s, s, fill);
 }
 
 // The one-launch decodes need 8 XCDs x 32 CUs (one workgroup per CU).  The
@@ -741,11 +771,11 @@ int decode_layers(hoard_moe *h, int l0, int l1, float *x_dev, float eps, hipStre
         rc = run_layer_fused(h, L, x_dev, 1, eps, x_dev, x_dev, h->sel, h->wsel, s, &fused);
         if (rc) return rc;
         if (fused) continue;
-        rc = run_route(h, L, x_dev, 1, eps, h->sel, h->wsel, s);
+        rc = run_route(h, L, x_dev, 1, eps, h->sel, h->wsel, s, h->pin_sel);
         if (rc) return rc;
         const int32_t *ids = h->sel;
         if (h->cfg.pool_k > 0) {
-            rc = pool_after_route(h, l, h->sel, h->slot_ids, s);
+            rc = pool_after_route(h, l, h->slot_ids, s);
             if (rc) return rc;
             ids = h->slot_ids;
         }
@@ -1089,11 +1119,11 @@ int hoard_moe_layer(hoard_moe *h, int layer, const float *fx_dev, const float *r
     bool fused = false;
     rc = run_layer_fused(h, L, fx_dev, 0, 0.0f, res_dev, out_dev, sel, w, s, &fused);
     if (rc || fused) return rc;
-    rc = run_route(h, L, fx_dev, 0, 0.0f, sel, w, s);
+    rc = run_route(h, L, fx_dev, 0, 0.0f, sel, w, s, h->pin_sel);
     if (rc) return rc;
     const int32_t *ids = sel;
     if (h->cfg.pool_k > 0) {
-        rc = pool_after_route(h, layer, sel, h->slot_ids, s);
+        rc = pool_after_route(h, layer, h->slot_ids, s);
         if (rc) return rc;
         ids = h->slot_ids;
     }

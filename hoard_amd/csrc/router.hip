@@ -85,7 +85,10 @@ __global__ __launch_bounds__(64 * kRows) void router_kernel(RouterArgs a) {
         last = __hip_atomic_fetch_add(&a.counters[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
     __syncthreads();
     if (!last) return;
-    if (wave == 0) router_tail<true>(a.logits, E, a.k, a.renorm, a.sel, a.wsel, 0);
+    if (wave == 0) {
+        const int id = router_tail<true>(a.logits, E, a.k, a.renorm, a.sel, a.wsel, 0);
+        if (a.sel_host && lane < a.k) a.sel_host[lane] = id;
+    }
     if (threadIdx.x == 0) __hip_atomic_store(&a.counters[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
