@@ -1,30 +1,28 @@
-// Batched expert stage for M tokens (speculative verify / small prefill):
-// tokens are grouped by expert so every selected expert's weights are read
-// once per call, and the expert products run on int8 MFMA.
+// Batched expert stage for M tokens (speculative verify / prefill): routing,
+// grouping by expert into work units, so that every selected expert's weights
+// are read once per unit, and the expert products of small units.
 //
 // Counterpart of ggml_mul_mat_id over the slot pool with per-token ids
 // (src/run_specloop.cpp:126-139; all-resident form src/run_m1.cpp:97-108)
 // followed by the weighted sum over the selected experts.
 //
-// The MFMA tiles and why they give the per-token path's bits are in mfma.h.
-// Batches of more than 32 tokens take the sorted-pair path of prefill.hip after
-// the routing and grouping here.
+// Units of a few pairs run here on per-token dots; larger ones on the int8
+// MFMA kernels of prefill.hip.
 #include "kernels.h"
 #include "lds_dma.h"
 #include "mfma.h"
 #include "qblocks.h"
 #include "rowdot.h"
+#include "rowstream.h"
 #include "router_tail.h"
 
 namespace hoard {
 
 namespace {
 
-constexpr int kTile = 16;                   // weight rows per MFMA tile
-constexpr int kMaxTok = kBatchedMaxTokens;  // token places per expert group
-constexpr int kCols = 16;                   // token columns per MFMA tile
-constexpr int kMfmaMinTokens = 6;          // smallest expert group computed on MFMA
-constexpr int kXChunk = 1;                  // tokens of Q8_K x staged in LDS at a time
+constexpr int kMaxTok = kBatchedMaxTokens;  // tokens of a verify-sized batch
+constexpr int kRowSets = 2;  // row sets of 8 a wave takes of the down rows (four of the shortest rows measured slower)
+static_assert(kDotTokens == 4 && kMaxTok <= 256, "a unit's tokens are the bytes of one word");
 constexpr int kMaxExperts = 1024;
 static_assert(sizeof(Q8L) == kQ8LBytes, "Q8_K block size shared with the host");
 
@@ -66,111 +64,55 @@ __device__ __forceinline__ bool pair_computed(const BatchedArgs &a, const int *y
 // buffers, which are free by then.
 struct GroupLds {
     unsigned mask[kMaxExperts];  // tokens (of a chunk) selecting each expert
-    int uidx[kMaxExperts];       // group of each expert
     unsigned cnt[kMaxExperts];   // pairs per expert
     int base[kMaxExperts];       // next sorted position of each expert
+    int ubase[kMaxExperts];      // first unit of each expert
     int total;
 };
 
 __device__ void group_units(const BatchedArgs &a, GroupLds &g);
 
-// a.unit != 0: the groups go out as sorted pairs and work units, as those of a
-// prefill-sized batch do (a group's mask gives its size and each pair's place).
-__device__ void group_by_expert(const BatchedArgs &a, GroupLds &g, const int *ysrc = nullptr,
+// Grouping of a batch of at most 32 tokens (all threads of the workgroup): a
+// group's mask gives its size and each pair's place.  sel: the pairs' selected
+// experts, in LDS.  Units of kDotTokens pairs carry their tokens in the record.
+__device__ void group_by_expert(const BatchedArgs &a, GroupLds &g, const int *sel, const int *ysrc = nullptr,
                                 const int *bad = nullptr) {
     unsigned *mask = g.mask;
-    int *uidx = g.uidx;
-    int &wave_total = g.total;
     const int tid = threadIdx.x, nt = blockDim.x, E = a.n_ids, P = a.M * a.k;
     for (int e = tid; e < E; e += nt) mask[e] = 0u;
     if (a.sh && tid == 0) mask[E] = a.M < 32 ? (1u << a.M) - 1u : ~0u;  // the shared expert: every token
     __syncthreads();
-    for (int p = tid; p < P; p += nt) {
-        if (!pair_computed(a, ysrc, bad, p)) continue;
-        int e = __hip_atomic_load(a.sel + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (e < 0 || e >= E) e = 0;  // out-of-range selections count as expert 0
-        atomicOr(&mask[e], 1u << (p / a.k));
-    }
+    // out-of-range selections count as expert 0
+    auto expert = [&](int p) { return sel[p] < 0 || sel[p] >= E ? 0 : sel[p]; };
+    for (int p = tid; p < P; p += nt)
+        if (pair_computed(a, ysrc, bad, p)) atomicOr(&mask[expert(p)], 1u << (p / a.k));
     __syncthreads();
-    if (a.unit) {
-        for (int e = tid; e < E + a.sh; e += nt) g.cnt[e] = (unsigned)__popc(mask[e]);
-        __syncthreads();
-        if (tid < 64) group_units(a, g);
-        __syncthreads();
-        const int kk = a.k + a.sh;
-        for (int p = tid; p < a.M * kk; p += nt) {
-            const int t = p / kk, j = p - t * kk;
-            int e = E;
-            if (j < a.k) {
-                if (!pair_computed(a, ysrc, bad, t * a.k + j)) continue;
-                e = __hip_atomic_load(a.sel + t * a.k + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (e < 0 || e >= E) e = 0;
-            }
-            const int pos = g.base[e] + __popc(mask[e] & ((1u << t) - 1u));
-            a.ptok[pos] = t;
-            a.pslot[pos] = j;
-        }
-        return;
-    }
-    if (tid < 64) {
-        // ascending prefix count of used experts: lane owns a contiguous run of experts
-        const int lane = tid, per = (E + 63) / 64, e0 = lane * per;
-        int cnt = 0;
-        for (int e = e0; e < e0 + per && e < E; ++e) cnt += mask[e] ? 1 : 0;
-        int incl = cnt;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int o = __shfl_up(incl, off);
-            if (lane >= off) incl += o;
-        }
-        int u = incl - cnt;
-        for (int e = e0; e < e0 + per && e < E; ++e) {
-            const unsigned m = mask[e];
-            a.hist[e] = (unsigned)__popc(m);
-            if (m) {
-                uidx[e] = u;
-                a.uexp[u] = e;
-                a.ucount[u] = __popc(m);
-                ++u;
-            }
-        }
-        if (lane == 63) wave_total = incl;
-    }
+    for (int e = tid; e < E + a.sh; e += nt) g.cnt[e] = (unsigned)__popc(mask[e]);
     __syncthreads();
-    for (int p = tid; p < P; p += nt) {
-        if (!pair_computed(a, ysrc, bad, p)) continue;
-        const int t = p / a.k, j = p % a.k;
-        int e = __hip_atomic_load(a.sel + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (e < 0 || e >= E) e = 0;
-        const int g = uidx[e], c = __popc(mask[e] & ((1u << t) - 1u));
-        a.utok[g * kMaxTok + c] = t;
-        a.uslot[g * kMaxTok + c] = j;
-    }
-    if (a.sh) {
-        // the shared expert: group n_unique (after the routed groups), every
-        // token, slot k
-        const int g = wave_total;
-        for (int t = tid; t < a.M; t += nt) {
-            a.utok[g * kMaxTok + t] = t;
-            a.uslot[g * kMaxTok + t] = a.k;
+    if (tid < 64) group_units(a, g);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the records are written before their token bytes
+    __syncthreads();
+    const int kk = a.k + a.sh;
+    for (int p = tid; p < a.M * kk; p += nt) {
+        const int t = p / kk, j = p - t * kk;
+        int e = E;
+        if (j < a.k) {
+            if (!pair_computed(a, ysrc, bad, t * a.k + j)) continue;
+            e = expert(t * a.k + j);
         }
-        if (tid == 0) {
-            a.uexp[g] = a.n_ids;
-            a.ucount[g] = a.M;
-        }
+        const int c = __popc(mask[e] & ((1u << t) - 1u));
+        a.ptok[g.base[e] + c] = t;
+        a.pslot[g.base[e] + c] = j;
+        if (a.unit == kDotTokens)
+            reinterpret_cast<uint8_t *>(a.units + 4 * (g.ubase[e] + c / kDotTokens) + 3)[c % kDotTokens] = (uint8_t)t;
     }
-    if (tid == 0) a.n_unique[0] = wave_total;
-    // the grid's group places past the used ones hold no expert, so a
-    // workgroup learns from its place alone whether it has work
-    const int umax = min(E, P) + a.sh;
-    for (int g = wave_total + a.sh + tid; g < umax; g += nt) a.uexp[g] = -1;
 }
 
 // Groups and units in ascending expert order from the per-expert pair counts
-// g.cnt (wave 0 of the grouping workgroup): uexp / ucount / goff / hist, the
-// unit records {expert, first sorted pair, pairs} (every place past the last
-// unit zeroed), n_unique / n_units, and g.base[e], the first sorted place of
-// expert e.
+// g.cnt (wave 0 of the grouping workgroup): hist, the unit records {expert,
+// first sorted pair, pairs, 0} (every place past the last unit zeroed),
+// n_unique / n_units, and g.base[e] / g.ubase[e], the first sorted place and
+// the first unit of expert e.
 __device__ void group_units(const BatchedArgs &a, GroupLds &g) {
     const int tid = threadIdx.x, E = a.n_ids + a.sh;
     {
@@ -193,18 +135,15 @@ __device__ void group_units(const BatchedArgs &a, GroupLds &g) {
                 ip += op;
             }
         }
-        int gi = ig - cg, ui = iu - cu, pi = ip - cp;
+        int ui = iu - cu, pi = ip - cp;
         for (int e = e0; e < e0 + per && e < E; ++e) {
             const int c = (int)g.cnt[e];
             a.hist[e] = (unsigned)c;
             g.base[e] = pi;
+            g.ubase[e] = ui;
             if (c) {
-                a.uexp[gi] = e;
-                a.ucount[gi] = c;
-                a.goff[gi] = pi;
                 for (int s0 = 0; s0 < c; s0 += a.unit, ++ui)
                     *reinterpret_cast<int4 *>(a.units + 4 * ui) = make_int4(e, pi + s0, min(a.unit, c - s0), 0);
-                ++gi;
             }
             pi += c;
         }
@@ -222,7 +161,7 @@ __device__ void group_units(const BatchedArgs &a, GroupLds &g) {
 
 // Grouping of a prefill-sized batch (all threads of one workgroup): the
 // computed (token, slot) pairs sorted by (expert, token) into ptok / pslot, the
-// groups (used experts in ascending order: uexp, ucount, goff) and the work
+// groups (used experts in ascending order) and the work
 // units (at most a.unit pairs of one group each).  pe[p] (in LDS) is the
 // expert of pair p, or -1 for a pair that joins no group.  The order within an
 // expert comes from chunks of at most 32 tokens taken in token order: a pair's
@@ -260,9 +199,9 @@ __device__ void group_large(const BatchedArgs &a, GroupLds &g, const int *pe, in
 
 // Q8_K of a block of fx with the sums the expert kernels of this call read.
 __device__ __forceinline__ void quantize_x(const BatchedArgs &a, const float *x, Q8L *out) {
-    if (a.unit && a.gu_type == kTypeQ3K)
+    if (a.unit != kDotTokens && a.gu_type == kTypeQ3K)
         wave_quantize_q8l<kSums16>(x, out);
-    else if (a.unit)
+    else if (a.unit != kDotTokens)
         wave_quantize_q8l<kSums32>(x, out);
     else
         wave_quantize_q8l(x, out);
@@ -354,25 +293,33 @@ __global__ __launch_bounds__(256) void route_kernel(BatchedArgs a) {
                gridDim.x - 1;
     __syncthreads();
     if (!last) return;
+    // the selections of every token, in LDS over the staging buffers, which are free
+    static_assert(sizeof(GroupLds) <= sizeof(xl) && sizeof(int) * kMaxTok * kMaxK <= sizeof(wl), "grouping LDS");
+    int *sel_s = reinterpret_cast<int *>(&wl[0][0]);
+    const bool one = gridDim.y == 1;  // one token group: this workgroup holds every selection
     for (int tt = wave; tt < kRouteTok; tt += 4) {
         const int tok = tg * kRouteTok + tt;
-        if (tok < a.M) router_tail<true>(a.logits, E, a.k, a.renorm, a.sel, a.wsel, tok);
+        if (tok < a.M) {
+            const int id = router_tail<true>(a.logits, E, a.k, a.renorm, a.sel, a.wsel, tok);
+            if (one && lane < a.k) sel_s[tok * a.k + lane] = id;
+        }
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        __hip_atomic_store(&a.counters[tg], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        last = __hip_atomic_fetch_add(&a.counters[kBatchedCounters - 1], 1u, __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT) == gridDim.y - 1;
+    if (threadIdx.x == 0) __hip_atomic_store(&a.counters[tg], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!one) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (threadIdx.x == 0)
+            last = __hip_atomic_fetch_add(&a.counters[kBatchedCounters - 1], 1u, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT) == gridDim.y - 1;
+        __syncthreads();
+        if (!last) return;
+        for (int p = threadIdx.x; p < a.M * a.k; p += blockDim.x)
+            sel_s[p] = __hip_atomic_load(a.sel + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (threadIdx.x == 0)
+            __hip_atomic_store(&a.counters[kBatchedCounters - 1], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
-    if (!last) return;
-    // the staging buffers are free: the grouping's LDS goes over them
-    static_assert(sizeof(GroupLds) <= sizeof(xl), "grouping LDS fits the token staging");
-    GroupLds &g = *reinterpret_cast<GroupLds *>(&xl[0][0]);
-    group_by_expert(a, g);
-    if (threadIdx.x == 0)
-        __hip_atomic_store(&a.counters[kBatchedCounters - 1], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    group_by_expert(a, *reinterpret_cast<GroupLds *>(&xl[0][0]), sel_s);
 }
 
 // -- prefill-sized routing: tiled router GEMM, then tails, then the grouping -----
@@ -655,41 +602,45 @@ __global__ __launch_bounds__(512) void prep_ids_kernel(BatchedArgs a) {
     }
     __shared__ int bad_s[kMaxTok];
     __shared__ int ysrc_s[kMaxTok * kMaxK];
+    __shared__ int sel_s[kMaxTok * kMaxK];
     __shared__ GroupLds g;
     const int tid = threadIdx.x, P = a.M * a.k;
     for (int t = tid; t < a.M; t += blockDim.x) bad_s[t] = 0;
+    for (int p = tid; p < P; p += blockDim.x) sel_s[p] = a.sel[p];
     __syncthreads();
     for (int p = tid; p < P; p += blockDim.x) {
         const int t = p / a.k, j = p % a.k;
-        const int e = a.sel[p];
+        const int e = sel_s[p];
         if (e < 0 || e >= a.n_ids) bad_s[t] = 1;
         int first = j;
         for (int i = j - 1; i >= 0; --i)
-            if (a.sel[t * a.k + i] == e) first = i;
+            if (sel_s[t * a.k + i] == e) first = i;
         ysrc_s[p] = first;
         a.ysrc[p] = first;  // for the combine launch
     }
     __syncthreads();
     for (int t = tid; t < a.M; t += blockDim.x) a.bad[t] = bad_s[t];
-    group_by_expert(a, g, ysrc_s, bad_s);
+    group_by_expert(a, g, sel_s, ysrc_s, bad_s);
 }
 
-// Expert groups are computed two ways.  A group of fewer than kMfmaMinTokens
-// tokens runs token by token with the per-token row dot, whose cost grows with
-// the group; a larger group runs on MFMA, whose cost is that of 16 token
-// columns whatever the group's size (two passes over the LDS tile above 16
-// tokens).  Both give the per-token path's bits.
-// Weight tiles are contiguous rows of the expert and are copied into LDS in
-// one burst.
-
-// A group's expert and size, read together (u < the grid's umax keeps them in
-// bounds; the grouping leaves expert -1 at every place past the used groups):
-// one latency.  Testing both keeps the compiler from moving their loads after
-// the test (a group always has an expert >= 0 and a token).
-__device__ __forceinline__ bool load_group(const BatchedArgs &a, int u, int &e, int &m) {
-    e = a.uexp[u];
-    m = min(a.ucount[u], kMaxTok);
-    return (e >= 0) & (m >= 1);
+// Few tokens an expert: units of at most kDotTokens pairs computed token by
+// token with the per-token row dots, which give the single-token path's bits.
+// A larger group is cut into several units (its weights are then read again,
+// from the caches), so that no workgroup is left with a long chain of tokens: a
+// shared expert's group of 8 tokens in one piece set the launches' time
+// (Qwen3-Next at M = 8: 75.4 us/layer, 58.7 as it is now).
+struct DotUnit {
+    int e, p0, n;
+    uint32_t tok;  // the pairs' tokens, a byte each
+};
+// One memory latency; a place past the last unit holds no pairs.
+__device__ __forceinline__ bool load_dot_unit(const BatchedArgs &a, int unit, DotUnit &w) {
+    const int4 r = *reinterpret_cast<const int4 *>(a.units + 4 * unit);
+    w.e = r.x;
+    w.p0 = r.y;
+    w.n = min(r.z, kDotTokens);
+    w.tok = (uint32_t)r.w;
+    return w.n > 0;
 }
 
 // Gather the Q8_K row (nb blocks) of token tt into LDS at xs, 16-byte granules
@@ -705,9 +656,10 @@ __device__ __forceinline__ void gather_token(uint8_t *xs, const uint8_t *q8base,
 }
 
 // -- gate/up: 8 rows of gate (wave 0) and up (wave 1) of one expert ----------
-// Per-token dot: one 8-lane group per row, lane t holding the token's Q8_K
-// block t.  MFMA (Q4_K groups of kMfmaMinTokens or more): the 8 rows fill a
-// 16-row tile twice.  Q3_K groups of any size run token by token.
+// One 8-lane group per row, lane t holding the token's Q8_K block t; the weight
+// tile is contiguous rows, copied into LDS in one burst.  x goes into LDS with
+// the tile, a token at a time (a vector load issued during the compute would
+// queue behind the tile copies of the other workgroups on this CU).
 template <int TGU, int NB>
 __global__ __launch_bounds__(128, 3) void gateup_kernel(BatchedArgs a) {
     static_assert(NB == 8, "one 8-lane group per row, one lane per super-block");
@@ -716,182 +668,102 @@ __global__ __launch_bounds__(128, 3) void gateup_kernel(BatchedArgs a) {
     constexpr int kRowBytes = NB * QType<TGU>::bytes;
     constexpr int kTileBytes = kRows * kRowBytes;
     static_assert(kTileBytes % 16 == 0, "the tile copies in 16-byte units");
-    const int u = blockIdx.y;
-    const int *tok = a.utok + u * kMaxTok;
-    // the group's first four tokens are read with its size and expert (the
-    // group's places are in the buffer whatever they turn out to be): one
-    // latency, not two
-    static_assert(kMaxTok % 4 == 0, "a group's token places are 16-byte aligned");
-    const int4 tok4 = *reinterpret_cast<const int4 *>(tok);
-    int e, m;
-    const bool has = load_group(a, u, e, m);
-    asm volatile("" ::"s"(tok4.x), "s"(tok4.y), "s"(tok4.z), "s"(tok4.w));  // loaded before the test, not after
-    if (!has) return;
+    DotUnit w;
+    if (!load_dot_unit(a, blockIdx.y, w)) return;
     __shared__ __align__(16) uint8_t wt[2][kTileBytes];
-    __shared__ __align__(16) uint8_t xs[kXChunk * NB * sizeof(Q8L)];
-    __shared__ float gu[2][kRows][kCols];  // gate and up values of 16 token columns
+    __shared__ __align__(16) uint8_t xs[NB * sizeof(Q8L)];
+    __shared__ float gu[2][kRows][kDotTokens];
     const int wave = wave_index(), lane = threadIdx.x & 63, t8 = lane & 7, grp = lane >> 3;
     const int row0 = blockIdx.x * kRows;
-    const uint8_t *W = (wave ? batched_up(a, e) : batched_gate(a, e)) + (size_t)row0 * kRowBytes;
-    // h = silu(gate) * up of columns c0 .. c0 + 15 from gu (128 threads: 8 rows x 16 columns)
-    auto store_h = [&](int c0) {
-        __syncthreads();
-        const int r = threadIdx.x / kCols, cc = threadIdx.x % kCols;
-        if (c0 + cc < m) {
-            const float g = gu[0][r][cc], uu = gu[1][r][cc];
-            a.hbuf[((size_t)u * kMaxTok + c0 + cc) * a.n_ff + row0 + r] = g / (1.0f + expf(-g)) * uu;
-        }
-    };
-    if (TGU == kTypeQ4K && m >= kMfmaMinTokens) {
-        dma_wave_copy_nt(wt[wave], W, kTileBytes);
-        lds_dma_wait();
-        // 16 token columns at a time over the LDS tile
-        for (int c0 = 0; c0 < m; c0 += kCols) {
-            if (c0 > 0) __syncthreads();  // the previous columns' h is formed
-            const int c = c0 + (lane & 15);
-            const Q8L *xq = q8(a.q8x) + (size_t)tok[c < m ? c : 0] * NB;
-            float v[4];
-            tile_q4k<NB, 7>(wt[wave], kRowBytes, xq, v);
-            if (lane < 32) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) gu[wave][4 * (lane >> 4) + i][lane & 15] = v[i];
-            }
-            store_h(c0);
-        }
-        return;
-    }
-    // token by token: x goes into LDS with the tile, kXChunk tokens at a time (a
-    // vector load issued during the compute would queue behind the tile copies
-    // of the other workgroups on this CU); h is stored every 16 token columns
+    const uint8_t *W = (wave ? batched_up(a, w.e) : batched_gate(a, w.e)) + (size_t)row0 * kRowBytes;
     const Q8L *xl = reinterpret_cast<const Q8L *>(xs);
-    for (int c0 = 0; c0 < m; c0 += kXChunk) {
-        const int mc = min(m - c0, kXChunk);
-        if (c0 > 0) __syncthreads();  // both waves are done with the previous chunk
-        static_assert(kXChunk == 1, "one token a copy");
-        const int tt = c0 == 0 ? tok4.x : c0 == 1 ? tok4.y : c0 == 2 ? tok4.z : c0 == 3 ? tok4.w : tok[c0];
-        gather_token<NB>(xs, a.q8x, tt, wave, 2);
-        if (c0 == 0) dma_wave_copy_nt(wt[wave], W, kTileBytes);
+    for (int c = 0; c < w.n; ++c) {
+        if (c > 0) __syncthreads();  // both waves are done with the previous token
+        gather_token<NB>(xs, a.q8x, (int)((w.tok >> (8 * c)) & 0xffu), wave, 2);
+        if (c == 0) dma_wave_copy_nt(wt[wave], W, kTileBytes);
         lds_dma_wait();
         __syncthreads();
-#pragma unroll 1
-        for (int c = 0; c < mc; ++c) {
-            const uint8_t *rp = wt[wave] + grp * kRowBytes;
-            float v;
-            if constexpr (TGU == kTypeQ3K)
-                v = lpb_row_q3k_mem<NB, true>(rp, xl[c * NB + t8], t8);
-            else
-                v = lpb_row_q4k_mem<NB, true>(rp, xl[c * NB + t8], t8);
-            if (t8 == NB - 1) gu[wave][grp][(c0 + c) % kCols] = v;
-        }
-        static_assert(kCols % kXChunk == 0, "a chunk of tokens stays within 16 columns");
-        if ((c0 + mc) % kCols == 0 && c0 + mc < m) store_h(c0 + mc - kCols);  // a full 16 columns, more to come
+        const uint8_t *rp = wt[wave] + grp * kRowBytes;
+        float v;
+        if constexpr (TGU == kTypeQ3K)
+            v = lpb_row_q3k_mem<NB, true>(rp, xl[t8], t8);
+        else
+            v = lpb_row_q4k_mem<NB, true>(rp, xl[t8], t8);
+        if (t8 == NB - 1) gu[wave][grp][c] = v;
     }
-    store_h((m - 1) / kCols * kCols);
+    __syncthreads();
+    // h = silu(gate) * up
+    const int r = threadIdx.x % kRows, c = threadIdx.x / kRows;
+    if (c < w.n) {
+        const float g = gu[0][r][c], uu = gu[1][r][c];
+        a.hbuf[(size_t)(w.p0 + c) * a.n_ff + row0 + r] = g / (1.0f + expf(-g)) * uu;
+    }
 }
 
-// -- Q8_K of h per (expert, token) ---------------------------------------------
-// One workgroup per (group, token), a wave per 256-element block of h.
-__global__ __launch_bounds__(256) void quant_h_kernel(BatchedArgs a) {
-    const int u = blockIdx.y, c = blockIdx.x, b = wave_index();
-    const int nbh = a.n_ff / QK;
-    const size_t uc = (size_t)u * kMaxTok + c;
-    // h is loaded with the group count and size, not after them (its place
-    // does not depend on them; a place past the groups is in the buffer and
-    // its values are dropped), all three as vector loads in flight together
-    // (u < the grid's umax and b < nbh keep them in bounds)
-    const int nu = __hip_atomic_load(a.n_unique, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + a.sh;
-    const int cnt = __hip_atomic_load(a.ucount + u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const float4 v4 = *reinterpret_cast<const float4 *>(a.hbuf + uc * a.n_ff + (size_t)b * QK + 4 * (threadIdx.x & 63));
-    asm volatile("" ::"v"(v4.x), "v"(v4.y), "v"(v4.z), "v"(v4.w));  // the load is not moved past the test
-    if (u >= nu || c >= min(cnt, kMaxTok)) return;
-    const float v[4] = {v4.x, v4.y, v4.z, v4.w};
-    wave_quantize_q8l_regs(v, q8(a.q8h) + uc * nbh + b);
-}
-
-// -- down: one 16-row tile of one expert; y to Y[token][slot] -------------------
-// Q6_K rows are only 2-byte aligned, which LDS reads handle with alignbyte;
-// the per-token Q6_K dot wants one alignment per wave, so each pass takes the
-// rows of one parity (the row size is 2 mod 4).
-template <int TD, int NBH>
-__device__ __forceinline__ void down_group(const BatchedArgs &a, int u, int e, int m, uint8_t *tile, uint8_t *xs) {
-    constexpr int kRowBytes = NBH * QType<TD>::bytes;
-    constexpr int kTileBytes = kTile * kRowBytes;
-    const int lane = threadIdx.x & 63, t8 = lane & 7, grp = lane >> 3;
-    const int row0 = blockIdx.x * kTile;
-    const int *tok = a.utok + u * kMaxTok, *slot = a.uslot + u * kMaxTok;
-    const uint8_t *src = batched_down(a, e) + (size_t)row0 * kRowBytes;
+// -- down: rows of the unit's expert, y to its (token, slot) place -------------
+// grid (n_embd / (32 kRowSets), max units): a wave's rows (kRowSets an 8-lane
+// group) go from memory to registers whole, all their blocks in flight at once, while the workgroup forms
+// Q8_K(h) of the unit's pairs in LDS from h (a launch of its own for that took
+// 4 to 5 us); then each pair's dots from the registers.  Bound by the weight
+// stream's latency: Qwen3-30B at 4 tokens 10.6 us a launch, 16.4 with the tile
+// in LDS, one wave a workgroup and Q8_K(h) in a launch before it; at 16 tokens
+// 23.7 against 35.3, Qwen3-Next 31.9 against 31.6.
+template <int T, int NBH>
+__device__ __forceinline__ void down_unit(const BatchedArgs &a, const DotUnit &w, Q8L *q8h) {
+    const int wave = wave_index(), lane = threadIdx.x & 63, t8 = lane & 7, grp = lane >> 3;
+    constexpr int RS = kRowSets;
+    const int row0 = (blockIdx.x * 4 + wave) * 8 * RS;
+    const float *h = a.hbuf + (size_t)w.p0 * a.n_ff;  // the pairs' h is contiguous
+    int slot[kDotTokens];
+#pragma unroll
+    for (int c = 0; c < kDotTokens; ++c) slot[c] = a.pslot[w.p0 + min(c, w.n - 1)];
+    WaveQuant<NBH> hq;  // a wave forms at most NBH of the kDotTokens * NBH blocks
+    hq.load(h, wave, w.n * NBH, 4);
+    RowShare<T> s[RS][NBH];
+    const uint8_t *base = batched_down(a, w.e) + (size_t)row0 * (NBH * QType<T>::bytes);
+#pragma unroll
+    for (int p = 0; p < RS; ++p)
+#pragma unroll
+        for (int b = 0; b < NBH; ++b)
+            s[p][b].load(base + b * QType<T>::bytes, (uint32_t)((8 * p + grp) * (NBH * QType<T>::bytes)), t8);
+    hq.form(h, q8h, wave, w.n * NBH, 4);
+    lds_barrier();
     const int kk = a.k + a.sh;  // output slots per token
-    if (TD != kTypeQ5K && m >= kMfmaMinTokens) {  // Q5_K groups of any size run token by token
-        dma_wave_copy_nt(tile, src, kTileBytes);
-        lds_dma_wait();
-        // 16 token columns at a time over the LDS tile
-        for (int c0 = 0; c0 < m; c0 += kCols) {
-            const int c = c0 + (lane & 15);
-            const Q8L *xq = q8(a.q8h) + ((size_t)u * kMaxTok + (c < m ? c : 0)) * NBH;
-            float v[4];
-            if constexpr (TD == kTypeQ4K)
-                tile_q4k<NBH>(tile, kRowBytes, xq, v);
-            else if constexpr (TD == kTypeQ6K)
-                tile_q6k<NBH>(tile, kRowBytes, xq, v);
-            if (c < m) {
-                float *y = a.ybuf + ((size_t)tok[c] * kk + slot[c]) * a.n_embd + row0;
+    for (int c = 0; c < w.n; ++c) {
+        const Q8L *x = q8h + c * NBH;
+        float v = 0.0f;  // lane t of a group keeps row set t's value
 #pragma unroll
-                for (int i = 0; i < 4; ++i) y[4 * (lane >> 4) + i] = v[i];
+        for (int p = 0; p < RS; ++p) {
+            float acc = 0.0f, accm = 0.0f;
+#pragma unroll
+            for (int b = 0; b < NBH; ++b) {
+                int isum, msum;
+                s[p][b].sums(x[b], t8, isum, msum);
+                isum = group8_sum(isum);
+                acc = acc + (s[p][b].d() * x[b].d) * (float)isum;
+                if constexpr (QType<T>::has_min) accm = accm + (s[p][b].dmin() * x[b].d) * (float)group8_sum(msum);
+                __builtin_amdgcn_sched_barrier(0);  // a block's operands at a time
             }
+            const float r = QType<T>::has_min ? acc - accm : acc;
+            v = t8 == p ? r : v;
         }
-        return;
-    }
-    const Q8L *xl = reinterpret_cast<const Q8L *>(xs);
-    for (int c0 = 0; c0 < m; c0 += kXChunk) {
-        const int mc = min(m - c0, kXChunk);
-        // the group's Q8_K h rows are contiguous, token-major
-        dma_wave_copy(xs, a.q8h + ((size_t)u * kMaxTok + c0) * NBH * sizeof(Q8L), mc * NBH * (int)sizeof(Q8L));
-        if (c0 == 0) dma_wave_copy_nt(tile, src, kTileBytes);
-        lds_dma_wait();
-#pragma unroll 1
-        for (int c = 0; c < mc; ++c) {
-            float *y = a.ybuf + ((size_t)tok[c0 + c] * kk + slot[c0 + c]) * a.n_embd + row0;
-            if constexpr (TD == kTypeQ6K) {
-#pragma unroll 1
-                for (int p = 0; p < 2; ++p) {
-                    const int row = 2 * grp + p;
-                    const float v = g8_row_q6k_u<NBH>(tile + row * kRowBytes, xl + c * NBH, t8);
-                    if (t8 == 0) y[row] = v;
-                }
-            } else if constexpr (TD == kTypeQ5K) {
-#pragma unroll 1
-                for (int p = 0; p < 2; ++p) {  // the single-token down kernel's Q5_K row dot
-                    const int row = 8 * p + grp;
-                    const float v = g8_row_q5k(tile + row * kRowBytes, xl + c * NBH, NBH, t8);
-                    if (t8 == 0) y[row] = v;
-                }
-            } else {
-#pragma unroll 1
-                for (int p = 0; p < 2; ++p) {
-                    const int row = 8 * p + grp;
-                    const float v = lpb_row_q4k_mem<NBH>(tile + row * kRowBytes, xl[c * NBH + min(t8, NBH - 1)], t8);
-                    if (t8 == NBH - 1) y[row] = v;
-                }
-            }
-        }
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this chunk's LDS reads precede the next copy
+        const int sl = c == 0 ? slot[0] : c == 1 ? slot[1] : c == 2 ? slot[2] : slot[3];
+        float *y = a.ybuf + ((size_t)((w.tok >> (8 * c)) & 0xffu) * kk + sl) * a.n_embd + row0;
+        if (t8 < RS) y[8 * t8 + grp] = v;
     }
 }
 
 // TD: the routed experts' down type; TS: the shared expert's (Q6_K beside
 // Q5_K routed rows, as Qwen3.5 has them), run by the same launch.
 template <int TD, int NBH, int TS = TD>
-__global__ __launch_bounds__(64, 4) void down_kernel(BatchedArgs a) {
-    constexpr int kTileBytes = kTile * NBH * (QType<TD>::bytes > QType<TS>::bytes ? QType<TD>::bytes : QType<TS>::bytes);
-    const int u = blockIdx.y;
-    int e, m;
-    if (!load_group(a, u, e, m)) return;
-    __shared__ __align__(16) uint8_t tile[kTileBytes];
-    __shared__ __align__(16) uint8_t xs[kXChunk * NBH * sizeof(Q8L)];
-    if (TS != TD && a.sh && e == a.n_ids)
-        down_group<TS, NBH>(a, u, e, m, tile, xs);
+__global__ __launch_bounds__(256, (TD == kTypeQ4K && NBH > 2) || (TD == kTypeQ5K && NBH > 2) ? 3 : 4) void down_kernel(BatchedArgs a) {
+    __shared__ __align__(16) Q8L q8h[kDotTokens * NBH];
+    DotUnit w;
+    if (!load_dot_unit(a, blockIdx.y, w)) return;
+    if (TS != TD && a.sh && w.e == a.n_ids)
+        down_unit<TS, NBH>(a, w, q8h);
     else
-        down_group<TD, NBH>(a, u, e, m, tile, xs);
+        down_unit<TD, NBH>(a, w, q8h);
 }
 
 // -- combine: out[t][d] = (sum_j w[t][j] * y[t][j][d]) + res[t][d], j ascending --
@@ -940,22 +812,20 @@ namespace {
 // The launches after the grouping: gate/up, Q8_K(h), down, combine.
 hipError_t launch_groups(const BatchedArgs &a, hipStream_t s) {
     const int nbh = a.n_ff / QK;
-    if (a.unit) {
+    const dim3 cg((a.n_embd + 255) / 256, a.M);
+    if (a.unit != kDotTokens) {
         if (hipError_t e = launch_prefill_groups(a, s); e != hipSuccess) return e;
-        hipLaunchKernelGGL(combine_kernel, dim3((a.n_embd + 255) / 256, a.M), dim3(256), 0, s, a);
+        hipLaunchKernelGGL(combine_kernel, cg, dim3(256), 0, s, a);
         return hipGetLastError();
     }
-    const int umax = (a.n_ids < a.M * a.k ? a.n_ids : a.M * a.k) + a.sh;
     if (a.gu_type == kTypeQ3K)
-        hipLaunchKernelGGL((gateup_kernel<kTypeQ3K, 8>), dim3(a.n_ff / 8, umax), dim3(128), 0, s, a);
+        hipLaunchKernelGGL((gateup_kernel<kTypeQ3K, 8>), dim3(a.n_ff / 8, a.max_units), dim3(128), 0, s, a);
     else
-        hipLaunchKernelGGL((gateup_kernel<kTypeQ4K, 8>), dim3(a.n_ff / 8, umax), dim3(128), 0, s, a);
-    // a group holds at most M (<= kMaxTok) tokens
-    hipLaunchKernelGGL(quant_h_kernel, dim3(a.M, umax), dim3(64 * nbh), 0, s, a);
-    const dim3 dg(a.n_embd / kTile, umax);
+        hipLaunchKernelGGL((gateup_kernel<kTypeQ4K, 8>), dim3(a.n_ff / 8, a.max_units), dim3(128), 0, s, a);
+    const dim3 dg(a.n_embd / (32 * kRowSets), a.max_units);
 #define HOARD_DOWN(T, N, TS)                                                    \
     if (a.d_type == T && nbh == N && sd == TS) {                                \
-        hipLaunchKernelGGL((down_kernel<T, N, TS>), dg, dim3(64), 0, s, a);     \
+        hipLaunchKernelGGL((down_kernel<T, N, TS>), dg, dim3(256), 0, s, a);    \
     } else
     const int sd = a.sh ? a.sh_d_type : a.d_type;
     HOARD_DOWN(kTypeQ6K, 3, kTypeQ6K) HOARD_DOWN(kTypeQ6K, 2, kTypeQ6K) HOARD_DOWN(kTypeQ6K, 4, kTypeQ6K)
@@ -964,7 +834,7 @@ hipError_t launch_groups(const BatchedArgs &a, hipStream_t s) {
         return hipErrorInvalidValue;
     }
 #undef HOARD_DOWN
-    hipLaunchKernelGGL(combine_kernel, dim3((a.n_embd + 255) / 256, a.M), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(combine_kernel, cg, dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
@@ -973,13 +843,13 @@ bool args_ok(const BatchedArgs &a) {
            (a.gu_type == kTypeQ4K || a.gu_type == kTypeQ3K) &&
            a.k + a.sh <= kMaxK && a.n_ids >= 1 && a.n_ids + a.sh <= kMaxExperts && a.E + a.sh <= kMaxExperts &&
            (!a.sh || (a.sh == 1 && a.sh_gate && a.sh_up && a.sh_down && a.sh_gate_inp && a.sgl)) &&
-           (a.M <= kMaxTok || (a.goff && a.ptok && a.pslot && a.pexp && a.units && a.n_units));
+           a.ptok && a.pslot && a.pexp && a.units && a.n_units;
 }
 
 }  // namespace
 
-// Whether a batch runs as sorted pairs in work units of one expert (16, 32 or
-// 64 pairs each), and the unit size; 0: the per-token dots of expert groups.
+// The pairs per work unit: kDotTokens, computed by per-token dots, or 16, 32 or
+// 64 for the MFMA kernels of prefill.hip.
 //
 // Above 32 tokens always units, of the smallest size that holds most experts'
 // pairs: small units keep more weights in flight, larger ones read an expert's
@@ -990,28 +860,27 @@ bool args_ok(const BatchedArgs &a) {
 // 125.
 //
 // Up to 32 tokens the dots of most groups' one or two tokens cost less than
-// folding their weights for 16 MFMA columns, except where the row type makes
-// the dot dear: with P pairs over n experts, Q3_K gate/up from P = 1.25 n (64
-// experts: M = 8 67 against 69, M = 10 79 / 75, M = 32 175 / 92 us/layer with
-// units), Q4_K down from 0.75 n (M = 4 40.0 / 41.2, M = 6 46.2 / 45.8, M = 32
-// 119 / 71), Q5_K down beside Q4_K gate/up from n / 8 (256 experts and a shared
-// one: M = 3 36.6 / 36.5, M = 4 42.6 / 41.7, M = 8 52.6 / 50.9, M = 16 71 / 71,
-// M = 32 112 / 104), and any type from 2 n (128 experts: M = 24 92 / 97, M = 32
-// 108 / 103).
+// folding their weights for 16 MFMA columns, until experts have several tokens
+// or where the row type makes the dot dear.  us/layer with dots / 16-pair
+// units, P pairs over n experts:
+//   Q3_K gate/up (64 experts) M = 8 56 / 69, M = 10 79 / 75, M = 16 104 / 90: from 1.25 n
+//   Q4_K down (64) M = 4 36 / 41, M = 6 46.2 / 45.8, M = 16 77 / 65: from 0.75 n
+//   Q5_K down beside Q4_K gate/up (256, a shared one) M = 2 28 / 35, M = 4 42.6 / 41.7: from n / 8
+//   the rest (128) M = 24 83 / 97, M = 32 108 / 103: from 2 n
 static int unit_pairs(const BatchedArgs &a) {
     const int P = a.M * a.k, n = a.n_ids;
     if (a.M <= kMaxTok) {
         const bool units = P >= 2 * n || (a.gu_type == kTypeQ3K ? 4 * P >= 5 * n
                                           : a.d_type == kTypeQ4K ? 4 * P >= 3 * n
                                                                  : a.d_type == kTypeQ5K && 8 * P >= n);
-        return units ? kUnitTokensMin : 0;
+        return units ? kUnitTokensMin : kDotTokens;
     }
     return P <= 11 * n ? kUnitTokensMin : P <= 21 * n ? 2 * kUnitTokensMin : kUnitTokens;
 }
 static BatchedArgs with_units(const BatchedArgs &a) {
     BatchedArgs r = a;
     r.unit = unit_pairs(a);
-    if (r.unit) r.max_units = prefill_max_units(a.M, a.k + a.sh, a.n_ids + a.sh, r.unit);
+    r.max_units = prefill_max_units(a.M, a.k + a.sh, a.n_ids + a.sh, r.unit);
     return r;
 }
 

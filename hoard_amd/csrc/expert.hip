@@ -30,33 +30,6 @@ __device__ __forceinline__ size_t row_bytes(int type, int cols) {
     return (size_t)(cols / QK) * (size_t)kquant_block_bytes(type);
 }
 
-// Q8_K of blocks first, first + step, ... below end of x into q, by one wave.
-// load() issues the loads of the first K blocks; the rest are loaded one by
-// one as the blocks are formed (behind whatever the wave loaded in between).
-// One quantiser in a loop that shifts the loaded blocks down: unrolled K
-// times it was most of a kernel's code.  x is 4-byte aligned.
-template <int K>
-struct WaveQuant {
-    f32x4_a4 v[K];
-    __device__ __forceinline__ void load(const float *x, int first, int end, int step) {
-#pragma unroll
-        for (int i = 0; i < K; ++i) get(i, x, min(first + i * step, end - 1));
-    }
-    __device__ __forceinline__ void get(int i, const float *x, int b) {
-        v[i] = *reinterpret_cast<const f32x4_a4 *>(x + (size_t)b * QK + 4 * (threadIdx.x & 63));
-    }
-    __device__ __forceinline__ void form(const float *x, Q8L *q, int first, int end, int step) {
-#pragma unroll 1
-        for (int b = first; b < end; b += step) {
-            const float w[4] = {v[0][0], v[0][1], v[0][2], v[0][3]};
-#pragma unroll
-            for (int i = 0; i + 1 < K; ++i) v[i] = v[i + 1];
-            if (b + K * step < end) get(K - 1, x, b + K * step);
-            wave_quantize_q8l_regs(w, q + b);
-        }
-    }
-};
-
 // The dot of the lane group's row (row grp of the 8 at base) with q; prep()
 // runs once the rows' first loads are issued.
 template <int T, class P>

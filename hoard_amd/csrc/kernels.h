@@ -81,25 +81,21 @@ struct BatchedArgs {
     const uint8_t *gate, *up, *down;
     size_t gstride, ustride, dstride;
     uint8_t *q8x;           // Q8_K(fx): [M][n_embd/256] blocks of 304 bytes
-    uint8_t *q8h;           // Q8_K(h):  [umax][kBatchedMaxTokens][n_ff/256] blocks
-    float *hbuf;            // [umax][kBatchedMaxTokens][n_ff]
+    uint8_t *q8h;           // Q8_K(h):  [pairs][n_ff/256] blocks, by sorted pair
+    float *hbuf;            // [pairs][n_ff], by sorted pair
     float *ybuf;            // [M][k + sh][n_embd]: slot k holds the shared expert's output
     int *n_unique;          // [1]
-    int *slot_of;           // [E] scratch
-    int *uexp, *ucount;     // [umax] expert of each group, tokens in it
-    int *utok, *uslot;      // [umax][kBatchedMaxTokens] token and slot of each member
     unsigned *hist;         // [n_ids] tokens per expert (or slot) in the call
     int n_ids;              // id space the groups are formed over: E, or the slots of a pool
     int *ysrc;              // [M][k] caller ids only: the slot j' <= j whose output pair (t, j) takes
                             // (its first occurrence of the same id), else null
     int *bad;               // [M] caller ids only: 1 for a token with an id outside [0, n_ids), else null
-    // prefill-sized batches (M > kBatchedMaxTokens): the pairs sorted by (expert, token)
-    // and cut into work units of at most `unit` pairs of one expert
-    int unit;               // 16, 32 or 64 (kUnitTokens)
-    int *goff;              // [umax] first sorted position of each group
+    // the pairs sorted by (expert, token) and cut into work units of at most
+    // `unit` pairs of one expert
+    int unit;               // kDotTokens, 16, 32 or 64 (kUnitTokens)
     int *ptok, *pslot;      // [M*k] token and slot of each sorted pair
     int *pexp;              // [M*k] expert of each pair for the grouping, -1 for one that joins none
-    int *units;             // [max_units][4] expert, first sorted pair, pairs (0: no unit), unused
+    int *units;             // [max_units][4] expert, first sorted pair, pairs (0: no unit), tokens of a kDotTokens unit
     float *q8hd;            // [pairs][4] the scales d of each sorted pair's Q8_K(h) blocks (prefill)
     int *n_units;           // [1]
     int max_units;
@@ -122,10 +118,11 @@ __device__ __forceinline__ const uint8_t *batched_up(const BatchedArgs &a, int e
 __device__ __forceinline__ const uint8_t *batched_down(const BatchedArgs &a, int e) {
     return a.sh && e == a.n_ids ? a.sh_down : a.down + (size_t)e * a.dstride;
 }
-constexpr int kBatchedMaxTokens = 32;         // the verify-sized path: per-token dots or MFMA per group
-constexpr int kBatchedMaxTokensLarge = 512;   // the prefill-sized path: sorted pairs, MFMA units
+constexpr int kBatchedMaxTokens = 32;         // verify-sized: one routing launch, per-token dots or MFMA units
+constexpr int kBatchedMaxTokensLarge = 512;   // prefill-sized: router GEMM, MFMA units
 constexpr int kUnitTokens = 64;               // most pairs of one expert per prefill work unit
-constexpr int kUnitTokensMin = 16;            // the smallest unit size
+constexpr int kUnitTokensMin = 16;            // the smallest unit size of the MFMA kernels
+constexpr int kDotTokens = 4;                 // most pairs of a unit computed by per-token dots
 constexpr int kBatchedCounters = 160;         // route completion counters: one per 4 tokens, and the tails'
 constexpr size_t kQ8LBytes = 304;
 hipError_t launch_batched(const BatchedArgs &a, hipStream_t s);

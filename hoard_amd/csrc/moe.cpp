@@ -1199,7 +1199,7 @@ namespace {
 struct BatchedLayout {
     int T, Ts, umax, umax_s, max_units;
     size_t q8x, q8h, hbuf, ybuf, n_ints, hist, counters;  // bytes (n_ints: ints)
-    size_t o_slot_of, o_uexp, o_ucount, o_utok, o_uslot, o_ysrc, o_bad, o_goff, o_ptok, o_pslot, o_pexp, o_units, o_q8hd,
+    size_t o_ysrc, o_bad, o_ptok, o_pslot, o_pexp, o_units, o_q8hd,
         o_nunits, o_sgl;
 };
 
@@ -1213,7 +1213,9 @@ BatchedLayout batched_layout(const hoard_moe_cfg &c, int T) {
     L.Ts = std::min(T, hoard::kBatchedMaxTokens);
     L.umax_s = std::min(E, L.Ts * k);
     L.umax = std::min(E, T * k);
-    L.max_units = hoard::prefill_max_units(T, k, E, hoard::kUnitTokensMin);  // the most of any unit size
+    // the most units of any size a batch takes
+    L.max_units = std::max(hoard::prefill_max_units(T, k, E, hoard::kUnitTokensMin),
+                           hoard::prefill_max_units(L.Ts, k, E, hoard::kDotTokens));
     const size_t pairs_s = (size_t)L.umax_s * hoard::kBatchedMaxTokens, pairs = (size_t)T * k;
     L.q8x = (size_t)T * nb * hoard::kQ8LBytes;
     L.q8h = std::max(pairs_s, pairs) * nbh * hoard::kQ8LBytes;
@@ -1225,14 +1227,8 @@ BatchedLayout batched_layout(const hoard_moe_cfg &c, int T) {
         o = r + n;
         return r;
     };
-    L.o_slot_of = take(E);
-    L.o_uexp = take(L.umax);
-    L.o_ucount = take(L.umax);
-    L.o_utok = take(pairs_s);
-    L.o_uslot = take(pairs_s);
     L.o_ysrc = take(pairs);
     L.o_bad = take(T);
-    L.o_goff = take(L.umax);
     L.o_ptok = take(pairs);
     L.o_pslot = take(pairs);
     L.o_pexp = take(pairs);
@@ -1255,12 +1251,6 @@ void bind_batched(hoard::BatchedArgs &a, const BatchedLayout &L, uint8_t *q8x, u
     a.hbuf = hbuf;
     a.ybuf = ybuf;
     a.n_unique = ints;
-    a.slot_of = ints + L.o_slot_of;
-    a.uexp = ints + L.o_uexp;
-    a.ucount = ints + L.o_ucount;
-    a.utok = ints + L.o_utok;
-    a.uslot = ints + L.o_uslot;
-    a.goff = ints + L.o_goff;
     a.ptok = ints + L.o_ptok;
     a.pslot = ints + L.o_pslot;
     a.pexp = ints + L.o_pexp;

@@ -42,48 +42,8 @@ __device__ __forceinline__ float wave_quantize_q8l(const float *x, Q8L *out) {
     return wave_quantize_q8l_regs<Sums>(v, out);
 }
 
-// One Q4_K row of nb super-blocks (16-byte aligned in LDS) dotted with x.
-// t = lane & 7.  Lane t covers quant bytes [16t, 16t+16) of every block, i.e.
-// 16 elements of sub-block 2*(t/2) (low nibbles) and of 2*(t/2)+1 (high).
-__device__ __forceinline__ float g8_row_q4k(const uint8_t *row, const Q8L *x, int nb, int t) {
-    const int c = t >> 1, h = t & 1;
-    float acc = 0.0f, accm = 0.0f;
-#pragma unroll
-    for (int b = 0; b < nb; ++b) {
-        const uint8_t *blk = row + b * kQ4KBytes;
-        const uint4 hd = *reinterpret_cast<const uint4 *>(blk);
-        const uint4 q = *reinterpret_cast<const uint4 *>(blk + 16 + 16 * t);
-        const Q8L &xb = x[b];
-        const uint4 xl = *reinterpret_cast<const uint4 *>(&xb.qs[16 * c + 4 * h]);
-        const uint4 xh = *reinterpret_cast<const uint4 *>(&xb.qs[16 * c + 8 + 4 * h]);
-        int lo = 0, hi = 0;
-        lo = sdot4(q.x & 0x0f0f0f0fu, xl.x, lo);
-        lo = sdot4(q.y & 0x0f0f0f0fu, xl.y, lo);
-        lo = sdot4(q.z & 0x0f0f0f0fu, xl.z, lo);
-        lo = sdot4(q.w & 0x0f0f0f0fu, xl.w, lo);
-        hi = sdot4((q.x >> 4) & 0x0f0f0f0fu, xh.x, hi);
-        hi = sdot4((q.y >> 4) & 0x0f0f0f0fu, xh.y, hi);
-        hi = sdot4((q.z >> 4) & 0x0f0f0f0fu, xh.z, hi);
-        hi = sdot4((q.w >> 4) & 0x0f0f0f0fu, xh.w, hi);
-        int sc0, m0, sc1, m1;
-        q4k_scale_min(2 * c, hd.y, hd.z, hd.w, sc0, m0);
-        q4k_scale_min(2 * c + 1, hd.y, hd.z, hd.w, sc1, m1);
-        int isum = sc0 * lo + sc1 * hi;
-        int msum = h ? 0
-                     : m0 * ((int)xb.bsums[4 * c] + (int)xb.bsums[4 * c + 1]) +
-                           m1 * ((int)xb.bsums[4 * c + 2] + (int)xb.bsums[4 * c + 3]);
-        isum = group8_sum(isum);
-        msum = group8_sum(msum);
-        const float d = half_bits_to_float(hd.x & 0xffffu) * xb.d;
-        const float dm = half_bits_to_float(hd.x >> 16) * xb.d;
-        acc = acc + d * (float)isum;
-        accm = accm + dm * (float)msum;
-    }
-    return acc - accm;
-}
-
-// One Q5_K row of nb super-blocks (16-byte aligned in LDS) dotted with x:
-// g8_row_q4k with the fifth bit of each quant from qh.  Lane t covers quant
+// One Q5_K row of nb super-blocks (16-byte aligned in LDS) dotted with x.
+// t = lane & 7.  The fifth bit of each quant comes from qh: lane t covers quant
 // bytes [16t, 16t+16) (chunk t/2, positions l = 16(t&1) .. +15) and the qh
 // bytes of the same positions, bits 2(t/2) and 2(t/2)+1.
 __device__ __forceinline__ float g8_row_q5k(const uint8_t *row, const Q8L *x, int nb, int t) {
@@ -230,18 +190,6 @@ __device__ __forceinline__ float g8_row_q6k_u(const uint8_t *row, const Q8L *x, 
         acc = acc + (half_bits_to_float(dbits) * x[b].d) * (float)isum;
     }
     return acc;
-}
-
-// Row dot for a compile-time type and block count: the block loop unrolls
-// fully, so every LDS read of the row is issued before the first dot product
-// needs it, and a kernel instantiates only the bodies it uses.
-template <int TYPE, int NB>
-__device__ __forceinline__ float g8_row(const uint8_t *row, const Q8L *x, int t) {
-    static_assert(TYPE == kTypeQ4K || TYPE == kTypeQ6K, "Q4_K or Q6_K rows");
-    if constexpr (TYPE == kTypeQ4K)
-        return g8_row_q4k(row, x, NB, t);
-    else
-        return g8_row_q6k(row, x, NB, t);
 }
 
 // ---------------------------------------------------------------------------
@@ -409,78 +357,6 @@ __device__ __forceinline__ float lpb_row_q4k_mem(const uint8_t *row, const Q8L &
         uint32_t dm;
         int isum, msum;
         q4k_block_sums_mem<Split>(row + t * kQ4KBytes, xb, dm, isum, msum);
-        const float d = half_bits_to_float(dm & 0xffffu) * xb.d;
-        const float dmin = half_bits_to_float(dm >> 16) * xb.d;
-        p = d * (float)isum;
-        pm = dmin * (float)msum;
-    }
-    const float acc = group_chain_sum<NB>(p, t);
-    const float accm = group_chain_sum<NB>(pm, t);
-    return acc - accm;
-}
-
-// Q5_K super-block (16-byte aligned: d/dmin and the Q4_K-packed scales in the
-// first 16 bytes, qh[32], qs[128]) against an activation block in memory: the
-// Q4_K sums with each quant's fifth bit taken from qh (bit 2j of qh[l] for
-// the low nibbles of chunk j, bit 2j+1 for the high ones).
-__device__ __forceinline__ void q5k_block_sums_mem(const uint8_t *blk, const Q8L &x, uint32_t &dm_bits, int &isum,
-                                                   int &msum) {
-    const uint4 hd = *reinterpret_cast<const uint4 *>(blk);
-    const uint4 h0 = *reinterpret_cast<const uint4 *>(blk + 16);
-    const uint4 h1 = *reinterpret_cast<const uint4 *>(blk + 32);
-    const uint32_t qh[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
-    dm_bits = hd.x;
-    const uint32_t sw[3] = {hd.y, hd.z, hd.w};
-    auto byte = [&](int i) -> int { return (int)((sw[i >> 2] >> (8 * (i & 3))) & 0xffu); };
-    const uint4 *xq = reinterpret_cast<const uint4 *>(x.qs);
-    isum = 0;
-    msum = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const uint4 q0 = *reinterpret_cast<const uint4 *>(blk + 48 + 32 * j);
-        const uint4 q1 = *reinterpret_cast<const uint4 *>(blk + 64 + 32 * j);
-        const uint4 x0 = xq[4 * j], x1 = xq[4 * j + 1], x2 = xq[4 * j + 2], x3 = xq[4 * j + 3];
-        const uint32_t qw[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-        const uint32_t xl[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-        const uint32_t xh[8] = {x2.x, x2.y, x2.z, x2.w, x3.x, x3.y, x3.z, x3.w};
-        int lo = 0, hi = 0;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const uint32_t ql = (qw[k] & 0x0f0f0f0fu) | (((qh[k] >> (2 * j)) & 0x01010101u) << 4);
-            const uint32_t qu = ((qw[k] >> 4) & 0x0f0f0f0fu) | (((qh[k] >> (2 * j + 1)) & 0x01010101u) << 4);
-            lo = sdot4(ql, xl[k], lo);
-            hi = sdot4(qu, xh[k], hi);
-        }
-        const uint32_t bw = *reinterpret_cast<const uint32_t *>(&x.bsums[4 * j]);
-        const uint32_t bw1 = *reinterpret_cast<const uint32_t *>(&x.bsums[4 * j + 2]);
-        const int bsl = (int)(int16_t)(bw & 0xffffu) + (int)(int16_t)(bw >> 16);
-        const int bsh = (int)(int16_t)(bw1 & 0xffffu) + (int)(int16_t)(bw1 >> 16);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int s = 2 * j + h;
-            int sc, mn;
-            if (s < 4) {
-                sc = byte(s) & 63;
-                mn = byte(s + 4) & 63;
-            } else {
-                sc = (byte(s + 4) & 0x0f) | ((byte(s - 4) >> 6) << 4);
-                mn = (byte(s + 4) >> 4) | ((byte(s) >> 6) << 4);
-            }
-            isum += sc * (h ? hi : lo);
-            msum += mn * (h ? bsh : bsl);
-        }
-    }
-}
-
-// One Q5_K row of NB super-blocks (16-byte aligned), one lane per block with
-// the lane's activation block xb read from memory; valid in lane NB-1.
-template <int NB>
-__device__ __forceinline__ float lpb_row_q5k_mem(const uint8_t *row, const Q8L &xb, int t) {
-    float p = 0.0f, pm = 0.0f;
-    if (t < NB) {
-        uint32_t dm;
-        int isum, msum;
-        q5k_block_sums_mem(row + t * kQ5KBytes, xb, dm, isum, msum);
         const float d = half_bits_to_float(dm & 0xffffu) * xb.d;
         const float dmin = half_bits_to_float(dm >> 16) * xb.d;
         p = d * (float)isum;
