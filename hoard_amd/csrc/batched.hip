@@ -20,10 +20,11 @@ namespace hoard {
 
 namespace {
 
+constexpr int kMaxExperts = 1024;
 constexpr int kMaxTok = kBatchedMaxTokens;  // tokens of a verify-sized batch
 constexpr int kRowSets = 2;  // row sets of 8 a wave takes of the down rows (four of the shortest rows measured slower)
-static_assert(kDotTokens == 4 && kMaxTok <= 256, "a unit's tokens are the bytes of one word");
-constexpr int kMaxExperts = 1024;
+static_assert(kDotTokens == 4 && kMaxDotTokens <= 256, "a unit's tokens are the bytes of one word");
+static_assert(kMaxDotTokens / 32 * (kMaxExperts + 1) <= 8448, "their grouping takes the one-pass form");
 static_assert(sizeof(Q8L) == kQ8LBytes, "Q8_K block size shared with the host");
 
 __device__ __forceinline__ Q8L *q8(uint8_t *p) { return reinterpret_cast<Q8L *>(p); }
@@ -72,6 +73,11 @@ struct GroupLds {
 
 __device__ void group_units(const BatchedArgs &a, GroupLds &g);
 
+// Token t, the c-th of its expert's group, into its unit's record.
+__device__ __forceinline__ void unit_token(const BatchedArgs &a, int unit0, int c, int t) {
+    reinterpret_cast<uint8_t *>(a.units + 4 * (unit0 + c / kDotTokens) + 3)[c % kDotTokens] = (uint8_t)t;
+}
+
 // Grouping of a batch of at most 32 tokens (all threads of the workgroup): a
 // group's mask gives its size and each pair's place.  sel: the pairs' selected
 // experts, in LDS.  Units of kDotTokens pairs carry their tokens in the record.
@@ -103,8 +109,7 @@ __device__ void group_by_expert(const BatchedArgs &a, GroupLds &g, const int *se
         const int c = __popc(mask[e] & ((1u << t) - 1u));
         a.ptok[g.base[e] + c] = t;
         a.pslot[g.base[e] + c] = j;
-        if (a.unit == kDotTokens)
-            reinterpret_cast<uint8_t *>(a.units + 4 * (g.ubase[e] + c / kDotTokens) + 3)[c % kDotTokens] = (uint8_t)t;
+        if (a.unit == kDotTokens) unit_token(a, g.ubase[e], c, t);
     }
 }
 
@@ -538,6 +543,7 @@ __device__ void group_large_chunks(const BatchedArgs &a, GroupLds &g, const int 
     __syncthreads();
     if (tid < 64) {
         group_units(a, g);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the records are written before their token bytes
     } else {
         for (int e = tid - 64; e < E; e += nt - 64) {
             int run = 0;
@@ -552,8 +558,9 @@ __device__ void group_large_chunks(const BatchedArgs &a, GroupLds &g, const int 
         const int e = pe[p];
         if (e < 0) continue;
         const int t = p / k, c = t >> 5;
-        const int pos = g.base[e] + cb[c * E + e] + __popc(cm[c * E + e] & ((1u << (t & 31)) - 1u));
-        sorted[pos] = t | (p - t * k) << 16;
+        const int c0 = cb[c * E + e] + __popc(cm[c * E + e] & ((1u << (t & 31)) - 1u));  // its place in the group
+        sorted[g.base[e] + c0] = t | (p - t * k) << 16;
+        if (a.unit == kDotTokens) unit_token(a, g.ubase[e], c0, t);
     }
 }
 
@@ -799,6 +806,55 @@ __global__ __launch_bounds__(256) void combine_kernel(BatchedArgs a) {
     a.out[(size_t)t * a.n_embd + d] = acc + r;
 }
 
+// The same for prefill-sized batches.
+__global__ __launch_bounds__(256) void pf_combine_kernel(BatchedArgs a) {
+    // four consecutive elements a thread (n_embd is a multiple of 1024): at
+    // hundreds of tokens the wider loads pay; at 16 tokens the one-element
+    // form of the batched path keeps more workgroups in flight
+    const int t = blockIdx.y;
+    const int d = 4 * (blockIdx.x * blockDim.x + threadIdx.x);
+    if (d >= a.n_embd) return;
+    float4 *o = reinterpret_cast<float4 *>(a.out + (size_t)t * a.n_embd + d);
+    if (a.bad && a.bad[t]) {  // an id outside the pool or expert set: the token's row is poisoned
+        const float nan = __builtin_nanf("");
+        *o = make_float4(nan, nan, nan, nan);
+        return;
+    }
+    const int kk = a.k + a.sh;
+    // every load is issued before the first is used: one memory latency, not k
+    float w[kMaxK];
+    float4 y[kMaxK];
+#pragma unroll
+    for (int j = 0; j < kMaxK; ++j) {
+        if (j < a.k) {
+            const int js = a.ysrc ? a.ysrc[t * a.k + j] : j;  // a repeated id takes its first output
+            w[j] = a.wsel[t * a.k + j];
+            y[j] = *reinterpret_cast<const float4 *>(a.ybuf + ((size_t)t * kk + js) * a.n_embd + d);
+        }
+    }
+    const float4 ysh = a.sh ? *reinterpret_cast<const float4 *>(a.ybuf + ((size_t)t * kk + a.k) * a.n_embd + d)
+                            : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const float4 r = *reinterpret_cast<const float4 *>(a.res + (size_t)t * a.n_embd + d);
+    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int j = 0; j < kMaxK; ++j) {
+        if (j < a.k) {
+            acc.x = acc.x + w[j] * y[j].x;
+            acc.y = acc.y + w[j] * y[j].y;
+            acc.z = acc.z + w[j] * y[j].z;
+            acc.w = acc.w + w[j] * y[j].w;
+        }
+    }
+    if (a.sh) {  // + sigmoid(gate logit) * shared expert output
+        const float sg = 1.0f / (1.0f + expf(-a.sgl[t]));
+        acc.x = acc.x + ysh.x * sg;
+        acc.y = acc.y + ysh.y * sg;
+        acc.z = acc.z + ysh.z * sg;
+        acc.w = acc.w + ysh.w * sg;
+    }
+    *o = make_float4(acc.x + r.x, acc.y + r.y, acc.z + r.z, acc.w + r.w);
+}
+
 }  // namespace
 
 bool batched_shape_compiled(int gu_type, int n_embd, int d_type, int n_ff) {
@@ -809,14 +865,20 @@ bool batched_shape_compiled(int gu_type, int n_embd, int d_type, int n_ff) {
 
 namespace {
 
+hipError_t launch_combine(const BatchedArgs &a, hipStream_t s) {
+    if (a.M > kMaxTok)
+        hipLaunchKernelGGL(pf_combine_kernel, dim3((a.n_embd + 1023) / 1024, a.M), dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL(combine_kernel, dim3((a.n_embd + 255) / 256, a.M), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
 // The launches after the grouping: gate/up, Q8_K(h), down, combine.
 hipError_t launch_groups(const BatchedArgs &a, hipStream_t s) {
     const int nbh = a.n_ff / QK;
-    const dim3 cg((a.n_embd + 255) / 256, a.M);
     if (a.unit != kDotTokens) {
         if (hipError_t e = launch_prefill_groups(a, s); e != hipSuccess) return e;
-        hipLaunchKernelGGL(combine_kernel, cg, dim3(256), 0, s, a);
-        return hipGetLastError();
+        return launch_combine(a, s);
     }
     if (a.gu_type == kTypeQ3K)
         hipLaunchKernelGGL((gateup_kernel<kTypeQ3K, 8>), dim3(a.n_ff / 8, a.max_units), dim3(128), 0, s, a);
@@ -834,8 +896,7 @@ hipError_t launch_groups(const BatchedArgs &a, hipStream_t s) {
         return hipErrorInvalidValue;
     }
 #undef HOARD_DOWN
-    hipLaunchKernelGGL(combine_kernel, cg, dim3(256), 0, s, a);
-    return hipGetLastError();
+    return launch_combine(a, s);
 }
 
 bool args_ok(const BatchedArgs &a) {
@@ -851,30 +912,23 @@ bool args_ok(const BatchedArgs &a) {
 // The pairs per work unit: kDotTokens, computed by per-token dots, or 16, 32 or
 // 64 for the MFMA kernels of prefill.hip.
 //
-// Above 32 tokens always units, of the smallest size that holds most experts'
-// pairs: small units keep more weights in flight, larger ones read an expert's
-// weights once for more pairs.  Mean pairs an expert against us/layer with
-// units of 16 / 32 / 64: 4 (256 experts, M = 128) 151 / 158 / 179, 8 (128
-// experts, M = 128) 124 / 129 / 128, 10 (512 experts, M = 512) 336 / 336 / 349,
-// 16 (64 experts, M = 128) 102 / 97 / 104, 32 (64 experts, M = 256) 146 / 131 /
-// 125.
-//
-// Up to 32 tokens the dots of most groups' one or two tokens cost less than
-// folding their weights for 16 MFMA columns, until experts have several tokens
-// or where the row type makes the dot dear.  us/layer with dots / 16-pair
-// units, P pairs over n experts:
-//   Q3_K gate/up (64 experts) M = 8 56 / 69, M = 10 79 / 75, M = 16 104 / 90: from 1.25 n
-//   Q4_K down (64) M = 4 36 / 41, M = 6 46.2 / 45.8, M = 16 77 / 65: from 0.75 n
-//   Q5_K down beside Q4_K gate/up (256, a shared one) M = 2 28 / 35, M = 4 42.6 / 41.7: from n / 8
-//   the rest (128) M = 24 83 / 97, M = 32 108 / 103: from 2 n
+// While an expert has one or two tokens, dots cost less than folding its weights
+// for 16 MFMA columns; the line lies near two pairs an expert for every type.
+// us/layer with dots / units of 16, P pairs over n experts:
+//   Q3_K / Q5_K, 64 experts:    M = 8 60 / 71, M = 16 (2 n) 85 / 91, M = 24 110 / 94
+//   Q4_K, 64:                   M = 8 48 / 56, M = 16 (2 n) 67.5 / 68.9, M = 24 84 / 73
+//   Q4_K / Q6_K, 128:           M = 24 86 / 93, M = 32 (2 n) 97.8 / 99.2, M = 48 121 / 111
+//   Q4_K / Q5_K, 256, a shared: M = 16 66 / 75, M = 40 102 / 111, M = 64 (2 n) 128 / 128
+//   Q4_K / Q6_K, 512, a shared: M = 40 142 / 153, M = 96 (1.9 n) 229 / 228, M = 128 267 / 248
+// Above, units of the smallest size that holds most experts' pairs: small ones
+// keep more weights in flight, larger ones read an expert's weights once for
+// more pairs.  Mean pairs an expert against us/layer with units of 16 / 32 /
+// 64: 4 (256 experts, M = 128) 151 / 158 / 179, 8 (128 experts, M = 128) 124 /
+// 129 / 128, 10 (512 experts, M = 512) 336 / 336 / 349, 16 (64 experts, M = 128)
+// 102 / 97 / 104, 32 (64 experts, M = 256) 146 / 131 / 125.
 static int unit_pairs(const BatchedArgs &a) {
     const int P = a.M * a.k, n = a.n_ids;
-    if (a.M <= kMaxTok) {
-        const bool units = P >= 2 * n || (a.gu_type == kTypeQ3K ? 4 * P >= 5 * n
-                                          : a.d_type == kTypeQ4K ? 4 * P >= 3 * n
-                                                                 : a.d_type == kTypeQ5K && 8 * P >= n);
-        return units ? kUnitTokensMin : kDotTokens;
-    }
+    if (a.M <= kMaxDotTokens && P <= 2 * n) return kDotTokens;
     return P <= 11 * n ? kUnitTokensMin : P <= 21 * n ? 2 * kUnitTokensMin : kUnitTokens;
 }
 static BatchedArgs with_units(const BatchedArgs &a) {
@@ -901,7 +955,7 @@ hipError_t launch_batched(const BatchedArgs &args, hipStream_t s) {
             hipLaunchKernelGGL((route_gemm_kernel<512, 8>), dim3(et, (a.M + 7) / 8), dim3(512), 0, s, a);
         hipLaunchKernelGGL(route_tails_kernel, dim3(a.M), dim3(640), 0, s, a);
         hipLaunchKernelGGL(group_kernel, dim3(1), dim3(1024), 0, s, a);
-        return launch_prefill_groups(a, s);
+        return launch_groups(a, s);
     }
     // row workgroups: a remainder of one row joins the last workgroup
     const int nr = a.E + a.sh, ntg = (a.M + kRouteTok - 1) / kRouteTok;
@@ -919,7 +973,7 @@ hipError_t launch_batched_ids(const BatchedArgs &args, hipStream_t s) {
     if (a.M > kMaxTok) {
         hipLaunchKernelGGL(prep_ids_large_kernel, dim3(a.M), dim3(512), 0, s, a);
         hipLaunchKernelGGL(group_kernel, dim3(1), dim3(1024), 0, s, a);
-        return launch_prefill_groups(a, s);
+        return launch_groups(a, s);
     }
     hipLaunchKernelGGL(prep_ids_kernel, dim3((unsigned)a.M + 1), dim3(512), 0, s, a);
     return launch_groups(a, s);

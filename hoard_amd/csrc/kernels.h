@@ -123,6 +123,7 @@ constexpr int kBatchedMaxTokensLarge = 512;   // prefill-sized: router GEMM, MFM
 constexpr int kUnitTokens = 64;               // most pairs of one expert per prefill work unit
 constexpr int kUnitTokensMin = 16;            // the smallest unit size of the MFMA kernels
 constexpr int kDotTokens = 4;                 // most pairs of a unit computed by per-token dots
+constexpr int kMaxDotTokens = 256;            // largest batch that takes them
 constexpr int kBatchedCounters = 160;         // route completion counters: one per 4 tokens, and the tails'
 constexpr size_t kQ8LBytes = 304;
 hipError_t launch_batched(const BatchedArgs &a, hipStream_t s);

@@ -1215,7 +1215,7 @@ BatchedLayout batched_layout(const hoard_moe_cfg &c, int T) {
     L.umax = std::min(E, T * k);
     // the most units of any size a batch takes
     L.max_units = std::max(hoard::prefill_max_units(T, k, E, hoard::kUnitTokensMin),
-                           hoard::prefill_max_units(L.Ts, k, E, hoard::kDotTokens));
+                           hoard::prefill_max_units(std::min(T, hoard::kMaxDotTokens), k, E, hoard::kDotTokens));
     const size_t pairs_s = (size_t)L.umax_s * hoard::kBatchedMaxTokens, pairs = (size_t)T * k;
     L.q8x = (size_t)T * nb * hoard::kQ8LBytes;
     L.q8h = std::max(pairs_s, pairs) * nbh * hoard::kQ8LBytes;

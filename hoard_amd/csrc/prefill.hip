@@ -15,7 +15,6 @@
 //   Q8_K(h)  per pair;
 //   down     64 rows per workgroup, the tile staged in LDS in one burst;
 //            y goes to its (token, slot) place;
-//   combine  per token, slots in order, plus the residual.
 // Every expert's weights are read once per unit (once per call for a group of
 // one unit's pairs); each (row, token) value is formed from the per-token
 // path's integer sub-block sums in its fp32 order, so every token's result is
@@ -882,55 +881,6 @@ __global__ __launch_bounds__(256, (kDownWaves<TD, NBH, TS, CH>)) void pf_down_ke
     }
 }
 
-// -- combine: out[t][d] = (sum_j w[t][j] * y[t][j][d]) + res[t][d], j ascending --
-__global__ __launch_bounds__(256) void pf_combine_kernel(BatchedArgs a) {
-    // four consecutive elements a thread (n_embd is a multiple of 1024): at
-    // hundreds of tokens the wider loads pay; at 16 tokens the one-element
-    // form of the batched path keeps more workgroups in flight
-    const int t = blockIdx.y;
-    const int d = 4 * (blockIdx.x * blockDim.x + threadIdx.x);
-    if (d >= a.n_embd) return;
-    float4 *o = reinterpret_cast<float4 *>(a.out + (size_t)t * a.n_embd + d);
-    if (a.bad && a.bad[t]) {  // an id outside the pool or expert set: the token's row is poisoned
-        const float nan = __builtin_nanf("");
-        *o = make_float4(nan, nan, nan, nan);
-        return;
-    }
-    const int kk = a.k + a.sh;
-    // every load is issued before the first is used: one memory latency, not k
-    float w[kMaxK];
-    float4 y[kMaxK];
-#pragma unroll
-    for (int j = 0; j < kMaxK; ++j) {
-        if (j < a.k) {
-            const int js = a.ysrc ? a.ysrc[t * a.k + j] : j;  // a repeated id takes its first output
-            w[j] = a.wsel[t * a.k + j];
-            y[j] = *reinterpret_cast<const float4 *>(a.ybuf + ((size_t)t * kk + js) * a.n_embd + d);
-        }
-    }
-    const float4 ysh = a.sh ? *reinterpret_cast<const float4 *>(a.ybuf + ((size_t)t * kk + a.k) * a.n_embd + d)
-                            : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    const float4 r = *reinterpret_cast<const float4 *>(a.res + (size_t)t * a.n_embd + d);
-    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-#pragma unroll
-    for (int j = 0; j < kMaxK; ++j) {
-        if (j < a.k) {
-            acc.x = acc.x + w[j] * y[j].x;
-            acc.y = acc.y + w[j] * y[j].y;
-            acc.z = acc.z + w[j] * y[j].z;
-            acc.w = acc.w + w[j] * y[j].w;
-        }
-    }
-    if (a.sh) {  // + sigmoid(gate logit) * shared expert output
-        const float sg = 1.0f / (1.0f + expf(-a.sgl[t]));
-        acc.x = acc.x + ysh.x * sg;
-        acc.y = acc.y + ysh.y * sg;
-        acc.z = acc.z + ysh.z * sg;
-        acc.w = acc.w + ysh.w * sg;
-    }
-    *o = make_float4(acc.x + r.x, acc.y + r.y, acc.z + r.z, acc.w + r.w);
-}
-
 }  // namespace
 
 namespace {
@@ -982,9 +932,7 @@ hipError_t launch_prefill_groups(const BatchedArgs &a, hipStream_t s) {
         return hipErrorInvalidValue;
     const hipError_t e = a.unit == 16 ? launch_units<1>(a, s) : a.unit == 32 ? launch_units<2>(a, s)
                          : a.unit == kUnitTokens ? launch_units<4>(a, s) : hipErrorInvalidValue;
-    if (e != hipSuccess || a.M <= kBatchedMaxTokens) return e;  // (a small batch's combine follows the caller)
-    hipLaunchKernelGGL(pf_combine_kernel, dim3((a.n_embd + 1023) / 1024, a.M), dim3(256), 0, s, a);
-    return hipGetLastError();
+    return e;
 }
 
 }  // namespace hoard

@@ -1,4 +1,4 @@
-"""Work units of 16, 32 and 64 pairs: caller ids whose expert groups end just
+"""Work units of 4 (per-token dots), 16, 32 and 64 pairs: caller ids whose expert groups end just
 before, at and after a unit's and an MFMA chunk's edge, at batches that take
 each unit size (and verify-sized ones that run as units), and hiddens whose
 Q8_K quants and sums are the largest there are.  The folded operands and the
@@ -13,10 +13,11 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 EDGES = [1, 15, 16, 17, 31, 32, 33, 48, 63, 64, 65, 129]
-# tokens of units of 16 (10, 31, 32: as verify-sized batches), 32 and 64 pairs over 64 experts
-CASES = [(s, m) for s in (W.OLMOE_Q3, W.OLMOE) for m in (10, 31, 32, 66, 140, 200)]
+# tokens of units of 4 (10, 16), 16 (31, 32: as verify-sized batches), 32 and 64 pairs over 64 experts
+CASES = [(s, m) for s in (W.OLMOE_Q3, W.OLMOE) for m in (10, 16, 31, 32, 66, 140, 200)]
 # a shared expert's group of every token beside Q5_K routed rows; Q4_K / Q6_K rows
-CASES += [(W.QWEN35, 8), (W.QWEN35, 66), (W.QWEN35, 400), (W.QWEN3_30B, 32), (W.QWEN3_30B, 66), (W.QWEN3_30B, 200),
+# (Qwen3.5 at 33 and 64 and Qwen3-Next at 102: prefill-sized on units of 4)
+CASES += [(W.QWEN35, 8), (W.QWEN35, 33), (W.QWEN35, 64), (W.QWEN35, 66), (W.QWEN3_NEXT, 102), (W.QWEN35, 400), (W.QWEN3_30B, 32), (W.QWEN3_30B, 66), (W.QWEN3_30B, 200),
           (W.QWEN3_30B, 400)]
 
 
