@@ -253,36 +253,36 @@ __device__ __forceinline__ uint4 lds_u128_a2(const uint8_t *p) {
 __device__ __forceinline__ void q6_fold(const uint8_t *T, size_t rb, int b, Q6Fold &o) {
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const uint8_t *blk = T + (size_t)r * rb + (size_t)b * kQ6KBytes;
+    const uint32_t h2 = 2u * (uint32_t)(g >> 1);
 #pragma unroll
     for (int jc = 0; jc < 4; ++jc) {
         const uint4 ql = lds_u128_a2(blk + 64 * (jc >> 1) + 16 * g);
         const uint4 qh = lds_u128_a2(blk + 128 + 32 * (jc >> 1) + 16 * (g & 1));
         const int sc = (int)(int8_t)blk[192 + 4 * jc + g];
-        const uint32_t nsh = 4u * (uint32_t)(jc & 1), hsh = 4u * (uint32_t)(jc & 1) + 2u * (uint32_t)(g >> 1);
-        const uint32_t sc16 = ((uint32_t)sc & 0xffffu) * 0x00010001u;  // sc in both 16-bit halves
-        typedef short v2s __attribute__((ext_vector_type(2)));
-        const v2s s2 = __builtin_bit_cast(v2s, sc16), z2 = {(short)(-32 * sc), (short)(-32 * sc)};
+        const v2s16 s2 = {(short)sc, (short)sc}, z2 = {(short)(128 - 32 * sc), (short)(128 - 32 * sc)};
         const uint32_t qlw[4] = {ql.x, ql.y, ql.z, ql.w}, qhw[4] = {qh.x, qh.y, qh.z, qh.w};
         int hw[4], lw[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const uint32_t q = ((qlw[k] >> nsh) & 0x0f0f0f0fu) | (((qhw[k] >> hsh) & 0x03030303u) << 4);
-            // bytes 0, 2 and 1, 3 in 16-bit halves; w = sc * q in each half
-            const uint32_t w02 = __builtin_amdgcn_perm(0u, q, 0x0c020c00u) ;
-            const uint32_t w13 = __builtin_amdgcn_perm(0u, q, 0x0c030c01u);
-            const v2s a02 = __builtin_bit_cast(v2s, w02) * s2 + z2, a13 = __builtin_bit_cast(v2s, w13) * s2 + z2;
-            const v2s r = {128, 128};
-            lw[k] = halves_to_bytes(__builtin_bit_cast(uint32_t, a02), __builtin_bit_cast(uint32_t, a13));
-            hw[k] = high_bytes(__builtin_bit_cast(uint32_t, a02 + r), __builtin_bit_cast(uint32_t, a13 + r));
+            // the upper two bits, at 2 (g / 2) or 4 + 2 (g / 2) of each byte, moved to bits 4 and 5
+            const uint32_t up = ((jc & 1) ? qhw[k] >> h2 : qhw[k] << (4u - h2)) & 0x30303030u;
+            const uint32_t q = ((qlw[k] >> (4 * (jc & 1))) & 0x0f0f0f0fu) | up;
+            // w + 128 in 16-bit halves (bytes 0, 2 and 1, 3): the high byte is hi,
+            // the low one lo with its top bit turned
+            uint32_t q02, q13;
+            bytes_to_halves(q, q02, q13);
+            const uint32_t a02 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2s16, q02) * s2 + z2);
+            const uint32_t a13 = __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2s16, q13) * s2 + z2);
+            lw[k] = (int)((uint32_t)halves_to_bytes(a02, a13) ^ 0x80808080u);
+            hw[k] = high_bytes(a02, a13);
         }
         o.hi[jc] = v4i{hw[0], hw[1], hw[2], hw[3]};
         o.lo[jc] = v4i{lw[0], lw[1], lw[2], lw[3]};
     }
+    // the factors of the lane's four result rows, from the lanes that hold those rows
+    const uint32_t d = (uint32_t)*reinterpret_cast<const uint16_t *>(blk + 208);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint8_t *blk_i = T + (size_t)(4 * g + i) * rb + (size_t)b * kQ6KBytes;
-        o.d[i] = half_bits_to_float((uint32_t)blk_i[208] | ((uint32_t)blk_i[209] << 8));
-    }
+    for (int i = 0; i < 4; ++i) o.d[i] = half_bits_to_float((uint32_t)__shfl((int)d, 4 * g + i));
 }
 
 // The quants of one token's block as the Q3_K, Q5_K and Q6_K folds take them:
@@ -444,16 +444,18 @@ __device__ __forceinline__ void q5_fold(const uint8_t *T, size_t rb, int b, Q5Fo
     const uint32_t qhw[4] = {qh.x, qh.y, qh.z, qh.w};
     const uint32_t nsh = 4u * (uint32_t)(g >> 1), bsh = 8u * (uint32_t)(g >> 1);
     o.mn = min_operand(mn);
+    const uint32_t qh1[4] = {qhw[0] >> (g >> 1), qhw[1] >> (g >> 1), qhw[2] >> (g >> 1), qhw[3] >> (g >> 1)};
 #pragma unroll
     for (int jc = 0; jc < 4; ++jc) {
-        const int s = 2 * jc + (g >> 1);
         const uint32_t sh = 16u * (uint32_t)(jc & 1) + bsh;  // byte 2 (jc & 1) + g / 2 of word jc / 2
         const uint32_t scs = (sc[jc >> 1] >> sh) & 0xffu;
         const uint4 qv = *reinterpret_cast<const uint4 *>(blk + 48 + 32 * jc + 16 * (g & 1));
         const uint32_t qw[4] = {qv.x, qv.y, qv.z, qv.w};
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const uint32_t q = ((qw[k] >> nsh) & 0x0f0f0f0fu) | (((qhw[k] >> s) & 0x01010101u) << 4);
+            // the fifth bit, bit s = 2 jc + g / 2 of each qh byte, moved to bit 4
+            const uint32_t up = (jc < 2 ? qh1[k] << (4 - 2 * jc) : qh1[k] >> (2 * jc - 4)) & 0x10101010u;
+            const uint32_t q = ((qw[k] >> nsh) & 0x0f0f0f0fu) | up;
             o.p[0][jc][k] = nib_mul(q, scs & 3u);
             o.p[1][jc][k] = nib_mul(q, (scs >> 2) & 3u);
             o.p[2][jc][k] = nib_mul(q, scs >> 4);
@@ -461,7 +463,7 @@ __device__ __forceinline__ void q5_fold(const uint8_t *T, size_t rb, int b, Q5Fo
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const uint32_t dm = *reinterpret_cast<const uint32_t *>(T + (size_t)(4 * g + i) * rb + (size_t)b * kQ5KBytes);
+        const uint32_t dm = (uint32_t)__shfl((int)hd.x, 4 * g + i);  // from the lanes that hold those rows
         o.d[i] = half_bits_to_float(dm & 0xffffu);
         o.dmin[i] = half_bits_to_float(dm >> 16);
     }
