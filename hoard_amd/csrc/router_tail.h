@@ -92,6 +92,7 @@ __device__ __forceinline__ bool topk_ranked(const float (&p)[NT], int k, int &my
         ce = mine ? e : ce;
         c += n;
     }
+    if (c < k) return false;  // NaN beside absent experts
     int r = 0;
     for (int i = 0; i < c; ++i) {
         const float v = readlane_f(cv, i);

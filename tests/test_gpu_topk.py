@@ -1,7 +1,8 @@
 """Router selections around the ranked top-k's bounds, against the oracle: the
 most experts that tie at one probability (its candidates overflow, the
 round-by-round form runs), zero probabilities, E not a multiple of 64, E of one
-lane pair, k of 1 and 16; the per-layer router and the batched tails."""
+lane pair, k of 1 and 16, NaN; the per-layer router, the one-launch layer and the batched
+tails."""
 import numpy as np
 import pytest
 
@@ -52,5 +53,13 @@ def test_selection_matches_oracle(orc, E, k):
                 assert np.array_equal(sel_l, sel) and np.array_equal(w_l.view(np.uint32), w.view(np.uint32))
             _, sel, w = st.forward_batched(0, toks, toks)
             assert np.array_equal(sel, np.stack([v[0] for v in want])), what
+            if what == "random":  # a NaN selects no expert, for its token alone
+                bad = toks.copy()
+                bad[1, 5] = np.nan
+                assert (st.route(0, bad[1])[0] >= E).all()
+                assert np.isnan(st.layer(0, bad[1], toks[1])[0]).all()
+                out, sel, _ = st.forward_batched(0, bad, toks)
+                assert (sel[1] >= E).all()
+                assert np.isfinite(np.delete(out, 1, 0)).all()
         finally:
             st.close()
