@@ -16,6 +16,7 @@
 #include "kernels.h"
 #include "lds_dma.h"
 #include "qblocks.h"
+#include "router_tail.h"
 #include "rowstream.h"
 #include "wave.h"
 
@@ -57,15 +58,46 @@ __device__ __forceinline__ float stream_row(int type, const uint8_t *base, const
     }
 }
 
+// The selection of a small router, by every workgroup that needs it: all rows
+// and x go to LDS with their copies in flight together, a half-wave forms each
+// row in the router's order (router.hip) and one wave runs the tail.
+__device__ void route_in_place(const GateUpArgs &a, float *lds, int32_t *sel, float *w) {
+    const int wave = wave_index(), lane = threadIdx.x & 63, l = lane & 31, nw = (int)(blockDim.x >> 6);
+    const int n = a.n_embd;
+    float *xl = lds, *wl = lds + n, *lg = wl + (size_t)a.E * n;
+    for (int e = wave; e < a.E; e += nw)
+        dma_wave_copy(reinterpret_cast<uint8_t *>(wl + (size_t)e * n), reinterpret_cast<const uint8_t *>(a.router + (size_t)e * n),
+                      n * (int)sizeof(float));
+    for (int i = 4 * threadIdx.x; i < n; i += 4 * blockDim.x)
+        *reinterpret_cast<u32x4 *>(xl + i) = *reinterpret_cast<const u32x4_a4 *>(a.fx + i);
+    lds_dma_wait();
+    __syncthreads();
+    for (int e0 = 2 * wave; e0 < a.E; e0 += 2 * nw) {
+        const int e = e0 + (lane >> 5);
+        const float *wp = wl + (size_t)(e < a.E ? e : e0) * n + l, *xp = xl + l;
+        float acc = 0.0f;
+#pragma unroll 16
+        for (int i = 0; i < n; i += 32) acc = fmaf(wp[i], xp[i], acc);
+        acc = acc + __shfl_xor(acc, 16);
+        acc = row16_ggml_fold(acc);
+        if (l == 0 && e < a.E) lg[e] = acc;
+    }
+    __syncthreads();
+    if (wave == 0) router_tail<false>(lg, a.E, a.k, a.renorm, sel, w, 0);
+    __syncthreads();
+}
+
 // ---------------------------------------------------------------------------
 // gate/up + SwiGLU.  grid = (rows_max / R, k + has_shared, plus a workgroup row
 // for the shared expert's gate); block = 64 * R / 4: R / 8 waves stream the
 // gate rows and R / 8 the up rows.
 // ---------------------------------------------------------------------------
-template <int T>
+template <int T, bool ROUTE>
 __global__ __launch_bounds__(512) void gateup_kernel(GateUpArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     __shared__ float gu[64];
+    __shared__ int32_t sel_s[16];
+    __shared__ float w_s[16];
     const int wave = wave_index(), lane = threadIdx.x & 63, t = lane & 7, grp = lane >> 3;
     const int nw = (int)(blockDim.x >> 6), R = nw / 2 * kWaveRows;
     const int j = blockIdx.y;
@@ -89,8 +121,15 @@ __global__ __launch_bounds__(512) void gateup_kernel(GateUpArgs a) {
     const int nb = a.n_embd / QK;
     float *hout = a.h + (size_t)j * a.hstride + r0;
     const uint8_t *src = W.base;
+    if (ROUTE && !shared) {
+        route_in_place(a, reinterpret_cast<float *>(smem + (size_t)nb * sizeof(Q8L)), sel_s, w_s);
+        if (blockIdx.x == 0 && j == 0 && threadIdx.x < a.k) {
+            a.sel[threadIdx.x] = sel_s[threadIdx.x];
+            a.wsel[threadIdx.x] = w_s[threadIdx.x];
+        }
+    }
     if (!shared) {
-        const int id = a.ids[j];
+        const int id = ROUTE ? __builtin_amdgcn_readfirstlane(sel_s[j]) : a.ids[j];
         if (id < 0 || id >= W.n_ids) {  // invalid id: poison this expert's rows
             if (threadIdx.x < R) hout[threadIdx.x] = __builtin_nanf("");
             return;
@@ -170,8 +209,13 @@ __global__ __launch_bounds__(1024) void down_combine_kernel(DownArgs a, int G) {
 
 size_t block_bytes(int type) { return (size_t)kquant_block_bytes(type); }
 
-hipError_t launch_gateup(const GateUpArgs &a, hipStream_t s) {
-    const size_t lds = (size_t)(a.n_embd / QK) * sizeof(Q8L);
+namespace {
+
+size_t route_lds(const GateUpArgs &a) { return ((size_t)(a.E + 1) * a.n_embd + a.E) * sizeof(float); }
+
+template <bool ROUTE>
+hipError_t launch_gateup_t(const GateUpArgs &a, hipStream_t s) {
+    const size_t lds = (size_t)(a.n_embd / QK) * sizeof(Q8L) + (ROUTE ? route_lds(a) : 0);
     if (lds > kMaxLds) return hipErrorInvalidConfiguration;
     const bool sh = a.sh_gate.base != nullptr;
     const int rows = sh && a.sh_gate.rows > a.gate.rows ? a.sh_gate.rows : a.gate.rows;
@@ -182,13 +226,37 @@ hipError_t launch_gateup(const GateUpArgs &a, hipStream_t s) {
     const dim3 grid((unsigned)(rows / (4 * waves)), (unsigned)(units + (sh ? 1 : 0)));
     const int T = a.gate.type;
     const bool one = a.up.type == T && (!sh || (a.sh_gate.type == T && a.sh_up.type == T));
-    auto *fn = !one             ? gateup_kernel<0>
-               : T == kTypeQ4K ? gateup_kernel<kTypeQ4K>
-               : T == kTypeQ5K ? gateup_kernel<kTypeQ5K>
-               : T == kTypeQ3K ? gateup_kernel<kTypeQ3K>
-                               : gateup_kernel<kTypeQ6K>;
+    auto *fn = !one             ? gateup_kernel<0, ROUTE>
+               : T == kTypeQ4K ? gateup_kernel<kTypeQ4K, ROUTE>
+               : T == kTypeQ5K ? gateup_kernel<kTypeQ5K, ROUTE>
+               : T == kTypeQ3K ? gateup_kernel<kTypeQ3K, ROUTE>
+                               : gateup_kernel<kTypeQ6K, ROUTE>;
     hipLaunchKernelGGL(fn, grid, dim3(64 * waves), lds, s, a);
     return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_gateup(const GateUpArgs &a, hipStream_t s) { return launch_gateup_t<false>(a, s); }
+
+// A router (16-byte aligned, for the LDS copies) whose rows fit LDS beside the workgroup's own blocks, in a launch of
+// at most one workgroup a CU: every workgroup reads the whole router (from its
+// XCD's L2 after the first), which costs less than the router's own launch and
+// the boundary after it until the rows are many.  A layer, us, with the launch
+// and without: n_embd 1024, 8 experts, top 2, n_ff 512 15.3 and 12.9; 2048, 6,
+// 4, 1024 19.4 and 17.6; 2304, 4, 2, 2048 23.7 and 20.8; 256, 32, 16, 256 16.7
+// and 15.8.  Past the lines: 256, 50, 4, 256 13.4 and 14.0 (few columns a row
+// and many rows a wave); 1024, 14, 8, 2048 23.2 and 23.5; 3072, 4, 2 and a
+// shared expert, 1536 23.8 and 24.0.
+bool gateup_routed_ok(const GateUpArgs &a) {
+    const bool sh = a.sh_gate.base != nullptr;
+    const int rows = sh && a.sh_gate.rows > a.gate.rows ? a.sh_gate.rows : a.gate.rows;
+    return a.router && ((uintptr_t)a.router & 15) == 0 && a.E <= 32 && rows * (a.k + sh) <= 4096 &&
+           (size_t)(a.n_embd / QK) * sizeof(Q8L) + route_lds(a) <= 61440;
+}
+hipError_t launch_gateup_routed(const GateUpArgs &a, hipStream_t s) {
+    if (!gateup_routed_ok(a)) return hipErrorInvalidConfiguration;
+    return launch_gateup_t<true>(a, s);
 }
 
 hipError_t launch_down_combine(const DownArgs &a, hipStream_t s) {

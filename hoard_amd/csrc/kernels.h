@@ -46,8 +46,18 @@ struct GateUpArgs {
     int n_embd, k;
     float *h;               // [(k+1)][hstride]
     int hstride;
+    // a small router's rows (launch_gateup_routed): every workgroup forms the
+    // selection for itself, the first one writes it to sel / wsel (ids unused)
+    const float *router;    // [E][n_embd]
+    int E, renorm;
+    int32_t *sel;           // [k]
+    float *wsel;            // [k]
 };
 hipError_t launch_gateup(const GateUpArgs &a, hipStream_t s);
+// Router and gate/up in one launch where the router is small enough to be formed
+// by every workgroup.
+bool gateup_routed_ok(const GateUpArgs &a);
+hipError_t launch_gateup_routed(const GateUpArgs &a, hipStream_t s);
 
 // Down GEMVs over all selected experts for a slice of output rows, fused with
 // the weighted combine: out[d] = ((sum_j w_j*y_j[d]) + sgate*ysh[d]) + res[d].

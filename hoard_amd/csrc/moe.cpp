@@ -325,8 +325,12 @@ int run_route(hoard_moe *h, const Layer &L, const float *xin, int is_residual, f
     return HOARD_OK;
 }
 
+// routed (optional): set to whether the router's selection was formed by the
+// gate/up launch, into sel / wsel, which ids and w then name; without it the
+// caller has routed already.
 int run_ffn(hoard_moe *h, const Layer &L, const float *fx, const int32_t *ids, const float *w,
-            const float *res, float *out, hipStream_t s) {
+            const float *res, float *out, hipStream_t s, int32_t *sel = nullptr, float *wsel = nullptr,
+            bool *routed = nullptr) {
     const hoard_moe_cfg &c = h->cfg;
     const int n_ids = c.pool_k > 0 ? c.pool_k : c.n_expert;  // ids are slots in pool mode
     const bool sh = c.n_ff_shexp > 0;
@@ -358,10 +362,19 @@ int run_ffn(hoard_moe *h, const Layer &L, const float *fx, const int32_t *ids, c
     d.res = res;
     d.out = out;
     const bool fast = h->layer_kernels && hoard::layer_ffn_ok(g, d);
+    if (routed) {
+        g.router = L.router;
+        g.E = c.n_expert;
+        g.renorm = c.renorm;
+        g.sel = sel;
+        g.wsel = wsel;
+        *routed = !fast && c.pool_k == 0 && !h->profiling && hoard::gateup_routed_ok(g);
+        if (!*routed) return HOARD_OK;
+    }
     hipError_t e;
     {
         KernelMark mark(h, HOARD_KERNEL_GATEUP, s);
-        e = fast ? hoard::launch_layer_gateup(g, s) : hoard::launch_gateup(g, s);
+        e = routed ? hoard::launch_gateup_routed(g, s) : fast ? hoard::launch_layer_gateup(g, s) : hoard::launch_gateup(g, s);
     }
     if (e != hipSuccess) return fail(HOARD_ERR_HIP, "gate/up launch: %s", hipGetErrorString(e));
     {
@@ -1119,6 +1132,9 @@ int hoard_moe_layer(hoard_moe *h, int layer, const float *fx_dev, const float *r
     bool fused = false;
     rc = run_layer_fused(h, L, fx_dev, 0, 0.0f, res_dev, out_dev, sel, w, s, &fused);
     if (rc || fused) return rc;
+    bool routed = false;
+    rc = run_ffn(h, L, fx_dev, sel, w, res_dev, out_dev, s, sel, w, &routed);
+    if (rc || routed) return rc;
     rc = run_route(h, L, fx_dev, 0, 0.0f, sel, w, s, h->pin_sel);
     if (rc) return rc;
     const int32_t *ids = sel;
