@@ -355,7 +355,11 @@ def run_pool(args, shape, n_layer):
     print(json.dumps(result), flush=True)
 
 
-MFMA_MIN_TOKENS = 12  # smallest expert group the batched kernels run on MFMA (kMfmaMinTokens)
+def dot_units(M, k, n):
+    """Whether a batch of M tokens runs per-token dots rather than MFMA units (unit_pairs in batched.hip)."""
+    return M <= 256 and M * k <= 2 * n
+
+
 MFMA_INT8_PEAK = 5.0e15  # MI355X dense int8 MFMA ops/s
 
 
@@ -442,10 +446,9 @@ def batched_measure(lib, h, shape, n_layer, M, steps, warm, seed, same=False):
     macs_per_pair = 3 * shape.n_ff * shape.n_embd
     sh_pairs = M * n_layer if shape.n_ff_shexp else 0  # the shared expert's group: all M tokens
     int8_ops = 2 * macs_per_pair * (int(hist.sum()) + sh_pairs)
-    # verify-sized batches run groups of MFMA_MIN_TOKENS or more on MFMA; prefill-sized
-    # ones (more than 32 tokens) run every group on MFMA
-    mfma_groups = hist >= (MFMA_MIN_TOKENS if M <= 32 else 1)
-    sh_mfma = sh_pairs if (M > 32 or M >= MFMA_MIN_TOKENS) else 0
+    dots = dot_units(M, shape.n_used, shape.n_expert)
+    mfma_groups = (hist > 0) & (not dots)
+    sh_mfma = 0 if dots else sh_pairs
     mfma_ops = 2 * macs_per_pair * (int(hist[mfma_groups].sum()) + sh_mfma)
     result = {
         "metric": f"batched MoE-layer us per step of {M} tokens + HBM GB/s, "
@@ -456,8 +459,8 @@ def batched_measure(lib, h, shape, n_layer, M, steps, warm, seed, same=False):
         "data": "synthetic weights and N(0,1) hiddens, every token routed independently",
         "config": {"workload": f"{shape.name}: {n_layer} layers, {M} tokens per step, all experts resident",
                    "tokens_per_step": M, "layers": n_layer,
-                   "path": "verify-sized: expert groups of 32 token places" if M <= 32 else
-                           "prefill-sized: pairs sorted by expert, 64-pair units on MFMA"},
+                   "path": "pairs sorted by expert, " + ("units of four on per-token dots" if dots else
+                                                          "units of 16, 32 or 64 on MFMA")},
         "tokens_per_s": round(M * 1000.0 / ms, 2),
         "unique_experts_per_layer": round(float(uniq.mean()), 2),
         "tokens_per_expert_max": int(hist.max()),
@@ -467,8 +470,7 @@ def batched_measure(lib, h, shape, n_layer, M, steps, warm, seed, same=False):
         "roofline": {"bound": "hbm", "kernel": "batched_experts", "achieved": round(gbps, 1),
                      "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": round(gbps / HBM_PEAK_GBPS, 4),
                      "traffic": None, "avg_us": round(bat_us, 3)},
-        # expert groups of 12 or more tokens run on int8 MFMA, smaller ones on
-        # the per-token int8 dot (MFMA_MIN_TOKENS in the batched kernels)
+        # a call's expert groups run on the per-token int8 dot or on int8 MFMA
         "expert_groups": {"per_token_dot": int(((hist > 0) & ~mfma_groups).sum()),
                           "mfma": int(((hist > 0) & mfma_groups).sum())},
         # int8 operations of the expert products (2 per multiply-add: gate, up and

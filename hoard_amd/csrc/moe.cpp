@@ -1209,9 +1209,11 @@ int hoard_moe_attach_store(hoard_moe *h, hoard_store *st) {
 namespace {
 
 // Scratch of the batched entry points for batches of up to T tokens: the
-// byte size of every buffer and the layout of the int arrays.  The verify-sized
-// path (M <= 32) keeps 32 token places per expert group; the prefill-sized one
-// keeps the pairs sorted by expert.
+// byte size of every buffer and the layout of the int arrays.  The
+// pairs lie sorted by expert; Q8_K(h) and h also hold kBatchedMaxTokens places
+// an expert for batches of up to that many tokens, more than their pairs, so
+// that what the fixed scratch of the allocation-free entry point takes and
+// refuses stays as it is.
 struct BatchedLayout {
     int T, Ts, umax, umax_s, max_units;
     size_t q8x, q8h, hbuf, ybuf, n_ints, hist, counters;  // bytes (n_ints: ints)

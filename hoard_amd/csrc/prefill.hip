@@ -691,8 +691,7 @@ __global__ __launch_bounds__(256, CH == 4 ? 3 : 4) void pf_gateup_kernel(Batched
 // flight, and all of the unit's activation blocks fit LDS at once (39 KB, four
 // workgroups a CU): one barrier after they land, then every wave streams its
 // rows from memory at its own pace.  Qwen3.5 at 131 tokens (302 MB): 85 -> 72 us
-// a launch against units of 64; Q3_K at 27
-// tokens 75 (per-token dots) -> 54.
+// a launch against units of 64; Q3_K at 27 tokens 75 (per-token dots) -> 54.
 // The quants and scale of a Q8_K block in LDS (17 granules: 16 tokens' reads
 // of one place fall into different banks).
 struct Q8S {

@@ -307,7 +307,9 @@ int hoard_moe_get_option(hoard_moe *h, int option, int *value);
    the FFN of layer l.  The slots go to slot_host and/or slot_dev (int32[n_used]),
    to be passed as ids to hoard_moe_ffn_combine.  hoard_moe_layer and
    hoard_moe_decode on a pool handle read the device-routed selection back
-   (a synchronisation, as the reference's D2H at :367) and call the same step. */
+   (a synchronisation, as the reference's D2H at :367) and take the same step,
+   their uploads by a kernel on `stream` itself (with a storage tier by copies, as
+   here). */
 int hoard_moe_pool_ensure(hoard_moe *h, int layer, const int32_t *sel_host, int32_t *slot_host,
                           int32_t *slot_dev, void *stream, void *copy_stream);
 
