@@ -355,9 +355,10 @@ def run_pool(args, shape, n_layer):
     print(json.dumps(result), flush=True)
 
 
-def dot_units(M, k, n):
-    """Whether a batch of M tokens runs per-token dots rather than MFMA units (unit_pairs in batched.hip)."""
-    return M <= 256 and M * k <= 2 * n
+def dot_groups(M, k, n, pairs):
+    """Which groups of `pairs` pairs run per-token dots (above 32 tokens in gate/up alone) rather than MFMA units
+    (units_mode and unit_shift of the batched kernels)."""
+    return (M <= 256 and M * k <= 2 * n) & (pairs < 8)
 
 
 MFMA_INT8_PEAK = 5.0e15  # MI355X dense int8 MFMA ops/s
@@ -446,9 +447,9 @@ def batched_measure(lib, h, shape, n_layer, M, steps, warm, seed, same=False):
     macs_per_pair = 3 * shape.n_ff * shape.n_embd
     sh_pairs = M * n_layer if shape.n_ff_shexp else 0  # the shared expert's group: all M tokens
     int8_ops = 2 * macs_per_pair * (int(hist.sum()) + sh_pairs)
-    dots = dot_units(M, shape.n_used, shape.n_expert)
-    mfma_groups = (hist > 0) & (not dots)
-    sh_mfma = 0 if dots else sh_pairs
+    dots = dot_groups(M, shape.n_used, shape.n_expert, hist)
+    mfma_groups = (hist > 0) & ~dots
+    sh_mfma = 0 if dot_groups(M, shape.n_used, shape.n_expert, M) else sh_pairs
     mfma_ops = 2 * macs_per_pair * (int(hist[mfma_groups].sum()) + sh_mfma)
     result = {
         "metric": f"batched MoE-layer us per step of {M} tokens + HBM GB/s, "
@@ -459,8 +460,8 @@ def batched_measure(lib, h, shape, n_layer, M, steps, warm, seed, same=False):
         "data": "synthetic weights and N(0,1) hiddens, every token routed independently",
         "config": {"workload": f"{shape.name}: {n_layer} layers, {M} tokens per step, all experts resident",
                    "tokens_per_step": M, "layers": n_layer,
-                   "path": "pairs sorted by expert, " + ("units of four on per-token dots" if dots else
-                                                          "units of 16, 32 or 64 on MFMA")},
+                   "path": "pairs sorted by expert, units of four on per-token dots (few pairs an expert) or of 16, 32 "
+                           "or 64 on MFMA"},
         "tokens_per_s": round(M * 1000.0 / ms, 2),
         "unique_experts_per_layer": round(float(uniq.mean()), 2),
         "tokens_per_expert_max": int(hist.max()),

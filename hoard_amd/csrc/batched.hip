@@ -1,19 +1,17 @@
 // Batched expert stage for M tokens (speculative verify / prefill): routing,
 // grouping by expert into work units, so that every selected expert's weights
-// are read once per unit, and the expert products of small units.
+// are read once per unit, and the combine.
 //
 // Counterpart of ggml_mul_mat_id over the slot pool with per-token ids
 // (src/run_specloop.cpp:126-139; all-resident form src/run_m1.cpp:97-108)
 // followed by the weighted sum over the selected experts.
 //
-// Units of a few pairs run here on per-token dots; larger ones on the int8
-// MFMA kernels of prefill.hip.
+// The expert products are in prefill.hip: units of a few pairs on per-token
+// dots, larger ones on int8 MFMA.
 #include "kernels.h"
 #include "lds_dma.h"
-#include "mfma.h"
 #include "qblocks.h"
 #include "rowdot.h"
-#include "rowstream.h"
 #include "router_tail.h"
 
 namespace hoard {
@@ -22,7 +20,6 @@ namespace {
 
 constexpr int kMaxExperts = 1024;
 constexpr int kMaxTok = kBatchedMaxTokens;  // tokens of a verify-sized batch
-constexpr int kRowSets = 2;  // row sets of 8 a wave takes of the down rows (four of the shortest rows measured slower)
 static_assert(kDotTokens == 4 && kMaxDotTokens <= 256, "a unit's tokens are the bytes of one word");
 static_assert(kMaxDotTokens / 32 * (kMaxExperts + 1) <= 8448, "their grouping takes the one-pass form");
 static_assert(sizeof(Q8L) == kQ8LBytes, "Q8_K block size shared with the host");
@@ -73,14 +70,16 @@ struct GroupLds {
 
 __device__ void group_units(const BatchedArgs &a, GroupLds &g);
 
-// Token t, the c-th of its expert's group, into its unit's record.
-__device__ __forceinline__ void unit_token(const BatchedArgs &a, int unit0, int c, int t) {
-    reinterpret_cast<uint8_t *>(a.units + 4 * (unit0 + c / kDotTokens) + 3)[c % kDotTokens] = (uint8_t)t;
+// Token t, the c-th of expert e's group, into its unit's record where the group
+// is cut into dot units.
+__device__ __forceinline__ void unit_token(const BatchedArgs &a, const GroupLds &g, int e, int c, int t) {
+    if (a.units_mode <= kUnitsDotGateUp && g.cnt[e] < kMfmaPairs)
+        reinterpret_cast<uint8_t *>(a.units + 4 * (g.ubase[e] + c / kDotTokens) + 3)[c % kDotTokens] = (uint8_t)t;
 }
 
 // Grouping of a batch of at most 32 tokens (all threads of the workgroup): a
 // group's mask gives its size and each pair's place.  sel: the pairs' selected
-// experts, in LDS.  Units of kDotTokens pairs carry their tokens in the record.
+// experts, in LDS.  Dot units carry their tokens in the record.
 __device__ void group_by_expert(const BatchedArgs &a, GroupLds &g, const int *sel, const int *ysrc = nullptr,
                                 const int *bad = nullptr) {
     unsigned *mask = g.mask;
@@ -109,15 +108,17 @@ __device__ void group_by_expert(const BatchedArgs &a, GroupLds &g, const int *se
         const int c = __popc(mask[e] & ((1u << t) - 1u));
         a.ptok[g.base[e] + c] = t;
         a.pslot[g.base[e] + c] = j;
-        if (a.unit == kDotTokens) unit_token(a, g.ubase[e], c, t);
+        unit_token(a, g, e, c, t);
     }
 }
 
-// Groups and units in ascending expert order from the per-expert pair counts
-// g.cnt (wave 0 of the grouping workgroup): hist, the unit records {expert,
+// Groups in ascending expert order and their units from the per-expert pair
+// counts g.cnt (wave 0 of the grouping workgroup): hist, the unit records {expert,
 // first sorted pair, pairs, 0} (every place past the last unit zeroed),
 // n_unique / n_units, and g.base[e] / g.ubase[e], the first sorted place and
-// the first unit of expert e.
+// the first unit of expert e.  The shared expert's units, which hold the most
+// pairs and take longest, come first: at the end they outlast the rest (512
+// experts, 16 tokens 68 us/layer, 61 so; 256 experts 57 and 51).
 __device__ void group_units(const BatchedArgs &a, GroupLds &g) {
     const int tid = threadIdx.x, E = a.n_ids + a.sh;
     {
@@ -127,7 +128,8 @@ __device__ void group_units(const BatchedArgs &a, GroupLds &g) {
         for (int e = e0; e < e0 + per && e < E; ++e) {
             const int c = (int)g.cnt[e];
             cg += c ? 1 : 0;
-            cu += (c + a.unit - 1) / a.unit;
+            const int us = unit_shift(a.units_mode, c);
+            cu += (c + (1 << us) - 1) >> us;
             cp += c;
         }
         int ig = cg, iu = cu, ip = cp;
@@ -140,16 +142,18 @@ __device__ void group_units(const BatchedArgs &a, GroupLds &g) {
                 ip += op;
             }
         }
-        int ui = iu - cu, pi = ip - cp;
+        const int us = a.sh ? unit_shift(a.units_mode, (int)g.cnt[E - 1]) : 0;
+        const int shu = a.sh ? ((int)g.cnt[E - 1] + (1 << us) - 1) >> us : 0;
+        int ui = shu + iu - cu, pi = ip - cp;
         for (int e = e0; e < e0 + per && e < E; ++e) {
             const int c = (int)g.cnt[e];
+            if (e == a.n_ids) ui = 0;
             a.hist[e] = (unsigned)c;
             g.base[e] = pi;
             g.ubase[e] = ui;
-            if (c) {
-                for (int s0 = 0; s0 < c; s0 += a.unit, ++ui)
-                    *reinterpret_cast<int4 *>(a.units + 4 * ui) = make_int4(e, pi + s0, min(a.unit, c - s0), 0);
-            }
+            const int u = 1 << unit_shift(a.units_mode, c), flag = u == kDotTokens ? kDotUnit : 0;
+            for (int s0 = 0; s0 < c; s0 += u, ++ui)
+                *reinterpret_cast<int4 *>(a.units + 4 * ui) = make_int4(e, pi + s0, min(u, c - s0) | flag, 0);
             pi += c;
         }
         if (lane == 63) {
@@ -167,7 +171,7 @@ __device__ void group_units(const BatchedArgs &a, GroupLds &g) {
 // Grouping of a prefill-sized batch (all threads of one workgroup): the
 // computed (token, slot) pairs sorted by (expert, token) into ptok / pslot, the
 // groups (used experts in ascending order) and the work
-// units (at most a.unit pairs of one group each).  pe[p] (in LDS) is the
+// units (of one group each).  pe[p] (in LDS) is the
 // expert of pair p, or -1 for a pair that joins no group.  The order within an
 // expert comes from chunks of at most 32 tokens taken in token order: a pair's
 // place is its expert's running base plus the tokens of its chunk before it
@@ -204,9 +208,9 @@ __device__ void group_large(const BatchedArgs &a, GroupLds &g, const int *pe, in
 
 // Q8_K of a block of fx with the sums the expert kernels of this call read.
 __device__ __forceinline__ void quantize_x(const BatchedArgs &a, const float *x, Q8L *out) {
-    if (a.unit != kDotTokens && a.gu_type == kTypeQ3K)
+    if (a.units_mode > kUnitsDotGateUp && a.gu_type == kTypeQ3K)
         wave_quantize_q8l<kSums16>(x, out);
-    else if (a.unit != kDotTokens)
+    else if (a.units_mode > kUnitsDotGateUp)
         wave_quantize_q8l<kSums32>(x, out);
     else
         wave_quantize_q8l(x, out);
@@ -560,7 +564,7 @@ __device__ void group_large_chunks(const BatchedArgs &a, GroupLds &g, const int 
         const int t = p / k, c = t >> 5;
         const int c0 = cb[c * E + e] + __popc(cm[c * E + e] & ((1u << (t & 31)) - 1u));  // its place in the group
         sorted[g.base[e] + c0] = t | (p - t * k) << 16;
-        if (a.unit == kDotTokens) unit_token(a, g.ubase[e], c0, t);
+        unit_token(a, g, e, c0, t);
     }
 }
 
@@ -628,149 +632,6 @@ __global__ __launch_bounds__(512) void prep_ids_kernel(BatchedArgs a) {
     __syncthreads();
     for (int t = tid; t < a.M; t += blockDim.x) a.bad[t] = bad_s[t];
     group_by_expert(a, g, sel_s, ysrc_s, bad_s);
-}
-
-// Few tokens an expert: units of at most kDotTokens pairs computed token by
-// token with the per-token row dots, which give the single-token path's bits.
-// A larger group is cut into several units (its weights are then read again,
-// from the caches), so that no workgroup is left with a long chain of tokens: a
-// shared expert's group of 8 tokens in one piece set the launches' time
-// (Qwen3-Next at M = 8: 75.4 us/layer, 58.7 as it is now).
-struct DotUnit {
-    int e, p0, n;
-    uint32_t tok;  // the pairs' tokens, a byte each
-};
-// One memory latency; a place past the last unit holds no pairs.
-__device__ __forceinline__ bool load_dot_unit(const BatchedArgs &a, int unit, DotUnit &w) {
-    const int4 r = *reinterpret_cast<const int4 *>(a.units + 4 * unit);
-    w.e = r.x;
-    w.p0 = r.y;
-    w.n = min(r.z, kDotTokens);
-    w.tok = (uint32_t)r.w;
-    return w.n > 0;
-}
-
-// Gather the Q8_K row (nb blocks) of token tt into LDS at xs, 16-byte granules
-// spread over the workgroup's nw waves (issued, not waited for).
-template <int NBX>
-__device__ __forceinline__ void gather_token(uint8_t *xs, const uint8_t *q8base, int tt, int wave, int nw) {
-    constexpr int kTokGran = NBX * (int)sizeof(Q8L) / 16;
-    const int lane = threadIdx.x & 63;
-    for (int k = wave; 64 * k < kTokGran; k += nw) {
-        const int p = 64 * k + lane;
-        if (p < kTokGran) dma_lanes(xs + 1024 * k, q8base + (size_t)tt * (NBX * sizeof(Q8L)) + 16 * p);
-    }
-}
-
-// -- gate/up: 8 rows of gate (wave 0) and up (wave 1) of one expert ----------
-// One 8-lane group per row, lane t holding the token's Q8_K block t; the weight
-// tile is contiguous rows, copied into LDS in one burst.  x goes into LDS with
-// the tile, a token at a time (a vector load issued during the compute would
-// queue behind the tile copies of the other workgroups on this CU).
-template <int TGU, int NB>
-__global__ __launch_bounds__(128, 3) void gateup_kernel(BatchedArgs a) {
-    static_assert(NB == 8, "one 8-lane group per row, one lane per super-block");
-    static_assert(TGU == kTypeQ4K || TGU == kTypeQ3K, "gate/up rows are Q4_K or Q3_K");
-    constexpr int kRows = 8;
-    constexpr int kRowBytes = NB * QType<TGU>::bytes;
-    constexpr int kTileBytes = kRows * kRowBytes;
-    static_assert(kTileBytes % 16 == 0, "the tile copies in 16-byte units");
-    DotUnit w;
-    if (!load_dot_unit(a, blockIdx.y, w)) return;
-    __shared__ __align__(16) uint8_t wt[2][kTileBytes];
-    __shared__ __align__(16) uint8_t xs[NB * sizeof(Q8L)];
-    __shared__ float gu[2][kRows][kDotTokens];
-    const int wave = wave_index(), lane = threadIdx.x & 63, t8 = lane & 7, grp = lane >> 3;
-    const int row0 = blockIdx.x * kRows;
-    const uint8_t *W = (wave ? batched_up(a, w.e) : batched_gate(a, w.e)) + (size_t)row0 * kRowBytes;
-    const Q8L *xl = reinterpret_cast<const Q8L *>(xs);
-    for (int c = 0; c < w.n; ++c) {
-        if (c > 0) __syncthreads();  // both waves are done with the previous token
-        gather_token<NB>(xs, a.q8x, (int)((w.tok >> (8 * c)) & 0xffu), wave, 2);
-        if (c == 0) dma_wave_copy_nt(wt[wave], W, kTileBytes);
-        lds_dma_wait();
-        __syncthreads();
-        const uint8_t *rp = wt[wave] + grp * kRowBytes;
-        float v;
-        if constexpr (TGU == kTypeQ3K)
-            v = lpb_row_q3k_mem<NB, true>(rp, xl[t8], t8);
-        else
-            v = lpb_row_q4k_mem<NB, true>(rp, xl[t8], t8);
-        if (t8 == NB - 1) gu[wave][grp][c] = v;
-    }
-    __syncthreads();
-    // h = silu(gate) * up
-    const int r = threadIdx.x % kRows, c = threadIdx.x / kRows;
-    if (c < w.n) {
-        const float g = gu[0][r][c], uu = gu[1][r][c];
-        a.hbuf[(size_t)(w.p0 + c) * a.n_ff + row0 + r] = g / (1.0f + expf(-g)) * uu;
-    }
-}
-
-// -- down: rows of the unit's expert, y to its (token, slot) place -------------
-// grid (n_embd / (32 kRowSets), max units): a wave's rows (kRowSets an 8-lane
-// group) go from memory to registers whole, all their blocks in flight at once, while the workgroup forms
-// Q8_K(h) of the unit's pairs in LDS from h (a launch of its own for that took
-// 4 to 5 us); then each pair's dots from the registers.  Bound by the weight
-// stream's latency: Qwen3-30B at 4 tokens 10.6 us a launch, 16.4 with the tile
-// in LDS, one wave a workgroup and Q8_K(h) in a launch before it; at 16 tokens
-// 23.7 against 35.3, Qwen3-Next 31.9 against 31.6.
-template <int T, int NBH>
-__device__ __forceinline__ void down_unit(const BatchedArgs &a, const DotUnit &w, Q8L *q8h) {
-    const int wave = wave_index(), lane = threadIdx.x & 63, t8 = lane & 7, grp = lane >> 3;
-    constexpr int RS = kRowSets;
-    const int row0 = (blockIdx.x * 4 + wave) * 8 * RS;
-    const float *h = a.hbuf + (size_t)w.p0 * a.n_ff;  // the pairs' h is contiguous
-    int slot[kDotTokens];
-#pragma unroll
-    for (int c = 0; c < kDotTokens; ++c) slot[c] = a.pslot[w.p0 + min(c, w.n - 1)];
-    WaveQuant<NBH> hq;  // a wave forms at most NBH of the kDotTokens * NBH blocks
-    hq.load(h, wave, w.n * NBH, 4);
-    RowShare<T> s[RS][NBH];
-    const uint8_t *base = batched_down(a, w.e) + (size_t)row0 * (NBH * QType<T>::bytes);
-#pragma unroll
-    for (int p = 0; p < RS; ++p)
-#pragma unroll
-        for (int b = 0; b < NBH; ++b)
-            s[p][b].load(base + b * QType<T>::bytes, (uint32_t)((8 * p + grp) * (NBH * QType<T>::bytes)), t8);
-    hq.form(h, q8h, wave, w.n * NBH, 4);
-    lds_barrier();
-    const int kk = a.k + a.sh;  // output slots per token
-    for (int c = 0; c < w.n; ++c) {
-        const Q8L *x = q8h + c * NBH;
-        float v = 0.0f;  // lane t of a group keeps row set t's value
-#pragma unroll
-        for (int p = 0; p < RS; ++p) {
-            float acc = 0.0f, accm = 0.0f;
-#pragma unroll
-            for (int b = 0; b < NBH; ++b) {
-                int isum, msum;
-                s[p][b].sums(x[b], t8, isum, msum);
-                isum = group8_sum(isum);
-                acc = acc + (s[p][b].d() * x[b].d) * (float)isum;
-                if constexpr (QType<T>::has_min) accm = accm + (s[p][b].dmin() * x[b].d) * (float)group8_sum(msum);
-                __builtin_amdgcn_sched_barrier(0);  // a block's operands at a time
-            }
-            const float r = QType<T>::has_min ? acc - accm : acc;
-            v = t8 == p ? r : v;
-        }
-        const int sl = c == 0 ? slot[0] : c == 1 ? slot[1] : c == 2 ? slot[2] : slot[3];
-        float *y = a.ybuf + ((size_t)((w.tok >> (8 * c)) & 0xffu) * kk + sl) * a.n_embd + row0;
-        if (t8 < RS) y[8 * t8 + grp] = v;
-    }
-}
-
-// TD: the routed experts' down type; TS: the shared expert's (Q6_K beside
-// Q5_K routed rows, as Qwen3.5 has them), run by the same launch.
-template <int TD, int NBH, int TS = TD>
-__global__ __launch_bounds__(256, (TD == kTypeQ4K && NBH > 2) || (TD == kTypeQ5K && NBH > 2) ? 3 : 4) void down_kernel(BatchedArgs a) {
-    __shared__ __align__(16) Q8L q8h[kDotTokens * NBH];
-    DotUnit w;
-    if (!load_dot_unit(a, blockIdx.y, w)) return;
-    if (TS != TD && a.sh && w.e == a.n_ids)
-        down_unit<TS, NBH>(a, w, q8h);
-    else
-        down_unit<TD, NBH>(a, w, q8h);
 }
 
 // -- combine: out[t][d] = (sum_j w[t][j] * y[t][j][d]) + res[t][d], j ascending --
@@ -873,29 +734,9 @@ hipError_t launch_combine(const BatchedArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// The launches after the grouping: gate/up, Q8_K(h), down, combine.
+// The launches after the grouping.
 hipError_t launch_groups(const BatchedArgs &a, hipStream_t s) {
-    const int nbh = a.n_ff / QK;
-    if (a.unit != kDotTokens) {
-        if (hipError_t e = launch_prefill_groups(a, s); e != hipSuccess) return e;
-        return launch_combine(a, s);
-    }
-    if (a.gu_type == kTypeQ3K)
-        hipLaunchKernelGGL((gateup_kernel<kTypeQ3K, 8>), dim3(a.n_ff / 8, a.max_units), dim3(128), 0, s, a);
-    else
-        hipLaunchKernelGGL((gateup_kernel<kTypeQ4K, 8>), dim3(a.n_ff / 8, a.max_units), dim3(128), 0, s, a);
-    const dim3 dg(a.n_embd / (32 * kRowSets), a.max_units);
-#define HOARD_DOWN(T, N, TS)                                                    \
-    if (a.d_type == T && nbh == N && sd == TS) {                                \
-        hipLaunchKernelGGL((down_kernel<T, N, TS>), dg, dim3(256), 0, s, a);    \
-    } else
-    const int sd = a.sh ? a.sh_d_type : a.d_type;
-    HOARD_DOWN(kTypeQ6K, 3, kTypeQ6K) HOARD_DOWN(kTypeQ6K, 2, kTypeQ6K) HOARD_DOWN(kTypeQ6K, 4, kTypeQ6K)
-    HOARD_DOWN(kTypeQ4K, 4, kTypeQ4K) HOARD_DOWN(kTypeQ4K, 3, kTypeQ4K) HOARD_DOWN(kTypeQ4K, 2, kTypeQ4K)
-    HOARD_DOWN(kTypeQ5K, 2, kTypeQ5K) HOARD_DOWN(kTypeQ5K, 4, kTypeQ5K) HOARD_DOWN(kTypeQ5K, 2, kTypeQ6K) {
-        return hipErrorInvalidValue;
-    }
-#undef HOARD_DOWN
+    if (hipError_t e = launch_expert_units(a, s); e != hipSuccess) return e;
     return launch_combine(a, s);
 }
 
@@ -909,41 +750,50 @@ bool args_ok(const BatchedArgs &a) {
 
 }  // namespace
 
-// The pairs per work unit: kDotTokens, computed by per-token dots, or 16, 32 or
-// 64 for the MFMA kernels of prefill.hip.
+// How the batch's groups are cut into units (unit_shift).  Figures: us/layer of
+// ffn_combine_batched with uniform ids and, after the bar, every token on the same
+// experts; P pairs over n experts.
 //
-// While an expert has one or two tokens, dots cost less than folding its weights
-// for 16 MFMA columns; the line lies near two pairs an expert for every type.
-// us/layer with dots / units of 16, P pairs over n experts:
-//   Q3_K / Q5_K, 64 experts:    M = 8 60 / 71, M = 16 (2 n) 85 / 91, M = 24 110 / 94
-//   Q4_K, 64:                   M = 8 48 / 56, M = 16 (2 n) 67.5 / 68.9, M = 24 84 / 73
-//   Q4_K / Q6_K, 128:           M = 24 86 / 93, M = 32 (2 n) 97.8 / 99.2, M = 48 121 / 111
-//   Q4_K / Q5_K, 256, a shared: M = 16 66 / 75, M = 40 102 / 111, M = 64 (2 n) 128 / 128
-//   Q4_K / Q6_K, 512, a shared: M = 40 142 / 153, M = 96 (1.9 n) 229 / 228, M = 128 267 / 248
-// The rule knows pairs, not where they fall: 128 experts whose 16 tokens all take
-// the same eight run 49.9 us here, and 45.8 with MFMA for such groups; spread
-// over the experts, 71.6 and 73.8.
-// Above, units of the smallest size that holds most experts' pairs: small ones
-// keep more weights in flight, larger ones read an expert's weights once for
-// more pairs.  Mean pairs an expert against us/layer with units of 16 / 32 /
-// 64: 4 (256 experts, M = 128) 151 / 158 / 179, 8 (128 experts, M = 128) 124 /
-// 129 / 128, 10 (512 experts, M = 512) 336 / 336 / 349, 16 (64 experts, M = 128)
-// 102 / 97 / 104, 32 (64 experts, M = 256) 146 / 131 / 125.
-static int unit_pairs(const BatchedArgs &a) {
+// Dots for the small groups while experts hold up to two pairs on average: a dot
+// costs less than folding a row's weights for 16 MFMA columns.  In the down
+// launch, which then forms Q8_K(h) itself, only for the verify-sized batches: its
+// dots and the forming grow with the pairs, a launch for Q8_K(h) hardly does.
+// Dots in both launches / in gate/up alone / nowhere:
+//   Q3_K / Q5_K, 64 experts:    M = 8 52 / 61 / 65, M = 16 (2 n) 80 / 87 / 82, M = 24 102 / 107 / 88
+//   Q4_K, 64:                   M = 8 43 / 48 / 50, M = 16 (2 n) 60 / 62 / 62, M = 24 75 / 74 / 66
+//   Q4_K / Q6_K, 128:           M = 16 65 / 68 / 76, M = 32 (2 n) 90 / 91 / 94 | 38 / 30 / 29, M = 40 102 / 103 / 100
+//   Q4_K / Q5_K, 256, a shared: M = 32 77 / 80 / 89 | 39 / 32 / 30, M = 64 (2 n) 115 / 113 / 116 | 54 / 41 / 38
+//   Q4_K / Q6_K, 512, a shared: M = 32 105 / 102 / 118 | 42 / 33 / 32, M = 40 125 / 118 / 142 | 54 / 40 / 38,
+//                               M = 102 (2 n) 216 / 206 / 216 | 89 / 52 / 49
+// A group of kMfmaPairs = 8 pairs goes to MFMA all the same (tokens of one prompt
+// or draft share experts).  Lines of 6 / 8 / 10 / 12, tokens that pick among
+// 2 k experts: 128 experts M = 8 35.9 / 33.5 / 33.3 / 33.5, M = 16 38.6 / 41.4 /
+// 43.0 / 43.7; 512 M = 24 40.1 / 40.1 / 43.2 / 46.1; Q3_K M = 16 52 / 50 / 61 / 70.
+//
+// Units of 16 and 32 by group until experts hold 21 pairs on average, then of
+// 64: small ones keep more weights in flight, large ones read and fold an
+// expert's weights once for more pairs.  16 and 32 / 64:
+//   256 experts, M = 128 (4 n):  137 / 161 | 48 / 52
+//   512, M = 512 (10 n):         296 / 306 | 129 / 117
+//   64, M = 128 (16 n):          92 / 97 | 54 / 52
+//   128, M = 256 (16 n):         133 / 135 | 73 / 65
+//   64, M = 256 (32 n):          127 / 118 | 88 / 82
+static int units_mode(const BatchedArgs &a) {
     const int P = a.M * a.k, n = a.n_ids;
-    if (a.M <= kMaxDotTokens && P <= 2 * n) return kDotTokens;
-    return P <= 11 * n ? kUnitTokensMin : P <= 21 * n ? 2 * kUnitTokensMin : kUnitTokens;
+    if (a.M <= kMaxDotTokens && P <= 2 * n) return a.M <= kMaxTok ? kUnitsDots : kUnitsDotGateUp;
+    return P <= 21 * n ? kUnitsMixed : kUnitsLarge;
 }
 static BatchedArgs with_units(const BatchedArgs &a) {
     BatchedArgs r = a;
-    r.unit = unit_pairs(a);
-    r.max_units = prefill_max_units(a.M, a.k + a.sh, a.n_ids + a.sh, r.unit);
+    r.units_mode = units_mode(a);
+    const int least = r.units_mode <= kUnitsDotGateUp ? kDotTokens : r.units_mode == kUnitsMixed ? kUnitTokensMin : kUnitTokens;
+    r.max_units = prefill_max_units(a.M, a.k + a.sh, a.n_ids + a.sh, least);
     return r;
 }
 
 // Batches of up to 32 tokens route, group and form Q8_K(fx) in one launch;
 // larger ones in three, the router as a matrix product.  Both then run units of
-// sorted pairs: dots here, MFMA in prefill.hip.
+// sorted pairs (prefill.hip).
 hipError_t launch_batched(const BatchedArgs &args, hipStream_t s) {
     const BatchedArgs a = with_units(args);
     if (!args_ok(a) || a.ysrc || a.n_ids != a.E || (a.M + kRouteTok - 1) / kRouteTok > kBatchedCounters - 1)

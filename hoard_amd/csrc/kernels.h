@@ -100,12 +100,11 @@ struct BatchedArgs {
     int *ysrc;              // [M][k] caller ids only: the slot j' <= j whose output pair (t, j) takes
                             // (its first occurrence of the same id), else null
     int *bad;               // [M] caller ids only: 1 for a token with an id outside [0, n_ids), else null
-    // the pairs sorted by (expert, token) and cut into work units of at most
-    // `unit` pairs of one expert
-    int unit;               // kDotTokens, 16, 32 or 64 (kUnitTokens)
+    // the pairs sorted by (expert, token) and cut into work units of one expert
+    int units_mode;         // kUnitsDots, kUnitsMixed or kUnitsLarge: how groups are cut (unit_shift)
     int *ptok, *pslot;      // [M*k] token and slot of each sorted pair
     int *pexp;              // [M*k] expert of each pair for the grouping, -1 for one that joins none
-    int *units;             // [max_units][4] expert, first sorted pair, pairs (0: no unit), tokens of a kDotTokens unit
+    int *units;             // [max_units][4] expert, first sorted pair, pairs (0: no unit) | kDotUnit, tokens of a dot unit
     float *q8hd;            // [pairs][4] the scales d of each sorted pair's Q8_K(h) blocks (prefill)
     int *n_units;           // [1]
     int max_units;
@@ -128,12 +127,28 @@ __device__ __forceinline__ const uint8_t *batched_up(const BatchedArgs &a, int e
 __device__ __forceinline__ const uint8_t *batched_down(const BatchedArgs &a, int e) {
     return a.sh && e == a.n_ids ? a.sh_down : a.down + (size_t)e * a.dstride;
 }
-constexpr int kBatchedMaxTokens = 32;         // verify-sized: one routing launch, per-token dots or MFMA units
-constexpr int kBatchedMaxTokensLarge = 512;   // prefill-sized: router GEMM, MFMA units
-constexpr int kUnitTokens = 64;               // most pairs of one expert per prefill work unit
+constexpr int kBatchedMaxTokens = 32;         // verify-sized: one routing launch
+constexpr int kBatchedMaxTokensLarge = 512;   // prefill-sized: router GEMM
+constexpr int kUnitTokens = 64;               // most pairs of one expert per work unit
 constexpr int kUnitTokensMin = 16;            // the smallest unit size of the MFMA kernels
 constexpr int kDotTokens = 4;                 // most pairs of a unit computed by per-token dots
+constexpr int kDotUnit = 1 << 16;             // flag beside the pairs of such a unit
 constexpr int kMaxDotTokens = 256;            // largest batch that takes them
+constexpr int kMfmaPairs = 8;                 // a dot batch's smallest group that goes to the MFMA units
+// How a batch cuts its expert groups into work units.  kUnitsDots: groups of
+// fewer than kMfmaPairs pairs into dot units, larger ones into units of 16;
+// kUnitsDotGateUp: such groups into units of kDotTokens pairs, which run dots in
+// the gate/up launch alone, larger ones into units of 16 (of at most 16 pairs) or
+// 32; kUnitsMixed: units of 16 or 32; kUnitsLarge: units of 64.  Within a batch
+// the size of every group decides: tokens of one prompt or draft share experts.
+constexpr int kUnitsDots = 0, kUnitsDotGateUp = 1, kUnitsMixed = 2, kUnitsLarge = 3;
+// log2 of the pairs a unit of a group of c pairs takes at most
+__host__ __device__ inline int unit_shift(int mode, int c) {
+    return mode <= kUnitsDotGateUp && c < kMfmaPairs ? 2
+           : mode == kUnitsDots || (mode != kUnitsLarge && c <= kUnitTokensMin) ? 4
+           : mode != kUnitsLarge                                                ? 5
+                                                                                : 6;
+}
 constexpr int kBatchedCounters = 160;         // route completion counters: one per 4 tokens, and the tails'
 constexpr size_t kQ8LBytes = 304;
 hipError_t launch_batched(const BatchedArgs &a, hipStream_t s);
@@ -147,9 +162,9 @@ constexpr size_t kNoAllocCounterBytes = 1024;
 hipError_t noalloc_setup(int device);
 uint8_t *noalloc_scratch(int device);
 size_t noalloc_scratch_bytes();
-// The expert products and combine of a prefill-sized batch after its grouping
-// (prefill.hip): gate/up + SwiGLU, Q8_K(h), down, ordered combine.
-hipError_t launch_prefill_groups(const BatchedArgs &a, hipStream_t s);
+// The expert products of a batch after its grouping (prefill.hip): gate/up +
+// SwiGLU, Q8_K(h), down.
+hipError_t launch_expert_units(const BatchedArgs &a, hipStream_t s);
 // Upper bound of the work units of `unit` pairs for M*k pairs over n_ids
 // groups: a group of c pairs takes at most (c + unit - 1) / unit of them.
 inline int prefill_max_units(int M, int k, int n_ids, int unit) {

@@ -1,24 +1,23 @@
-// Expert products of a prefill-sized batch (more than 32 tokens): the
-// counterpart of ggml_mul_mat_id over all T prompt tokens
-// (src/run_m1.cpp:93-108) and of the verify step's mul_mat_id with per-token
-// ids (src/run_specloop.cpp:126-139), followed by the weighted sum over the
-// selected experts.
+// Expert products of a batch: the counterpart of ggml_mul_mat_id over all T
+// prompt tokens (src/run_m1.cpp:93-108) and of the verify step's mul_mat_id with
+// per-token ids (src/run_specloop.cpp:126-139).
 //
 // batched.hip routes the tokens (or takes the caller's ids), forms Q8_K(fx)
-// and sorts the (token, slot) pairs by (expert, token) into work units of at
-// most 16, 32 or 64 pairs of one expert.  Here, per unit:
+// and sorts the (token, slot) pairs by (expert, token) into work units of one
+// expert: of 4 pairs for the per-token dots of dotunits.h, of 16, 32 or 64 for
+// the MFMA bodies here; the size of the expert's group decides, and one launch
+// holds units of both of its batch's kinds.  Per MFMA unit:
 //   gate/up  32 rows of gate and of up per workgroup (16 rows of one matrix per
 //            wave) against the unit's tokens on v_mfma_i32_16x16x64_i8, 16
 //            token columns per MFMA, the sub-block scales folded into the
 //            weight operand; each weight super-block is loaded and folded once
 //            and used for every token chunk of the unit; SwiGLU fused;
-//   Q8_K(h)  per pair;
-//   down     64 rows per workgroup, the tile staged in LDS in one burst;
-//            y goes to its (token, slot) place;
-// Every expert's weights are read once per unit (once per call for a group of
-// one unit's pairs); each (row, token) value is formed from the per-token
-// path's integer sub-block sums in its fp32 order, so every token's result is
-// the single-token path's bit for bit.
+//   Q8_K(h)  per pair (by the down launch where that runs dots);
+//   down     64 rows per workgroup; y goes to its (token, slot) place.
+// Each (row, token) value is formed from the per-token path's integer sub-block
+// sums in its fp32 order, so every token's result is the single-token path's bit
+// for bit.
+#include "dotunits.h"
 #include "kernels.h"
 #include "lds_dma.h"
 #include "mfma.h"
@@ -35,20 +34,6 @@ constexpr int kGuRows = 32;    // gate (and up) rows per workgroup: two 16-row t
 constexpr int kDnRows = 64;    // down rows per workgroup
 
 __device__ __forceinline__ const Q8L *q8c(const uint8_t *p) { return reinterpret_cast<const Q8L *>(p); }
-
-// A work unit: expert e, its pairs [p0, p0 + n) in sorted order; one 16-byte
-// record (a place past the last unit holds n = 0), so a workgroup knows its
-// work after one memory latency.
-struct Unit {
-    int e, p0, n;
-};
-__device__ __forceinline__ bool load_unit(const BatchedArgs &a, int unit, Unit &w) {
-    const int4 r = *reinterpret_cast<const int4 *>(a.units + 4 * unit);
-    w.e = r.x;
-    w.p0 = r.y;
-    w.n = r.z;
-    return w.n > 0;
-}
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
@@ -201,6 +186,25 @@ __device__ __forceinline__ v8h load_sums(const X &x) {
     return reinterpret_cast<const v8h *>(x.bsums)[((threadIdx.x & 63) >> 4) & 1];
 }
 
+// The same operand from a block whose sums are int16 (kSumsInt): b, its sixteen
+// 16-element sums; half: which v8h (load_sums).  Q3_K takes the sums as they are
+// (kSums16), the others the 32-element sums in two parts (kSums32).
+template <int TG>
+__device__ __forceinline__ v8h sums_from_int(const v4i (&b)[2], int half) {
+    v8h r;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        if constexpr (TG == kTypeQ3K) {
+            const int w = half ? b[1][s >> 1] : b[0][s >> 1];
+            r[s] = (_Float16)(float)((s & 1) ? w >> 16 : (int)(int16_t)w);
+        } else {
+            const int w = b[s >> 2][s & 3], v = (int)(int16_t)w + (w >> 16);
+            r[s] = (_Float16)(float)(half ? v & 1 : v & ~1);
+        }
+    }
+    return r;
+}
+
 // -- Q8_K of h per sorted pair --------------------------------------------------
 // grid (pairs), block 64 * NBH: wave b quantises block b of the pair's h.
 __global__ __launch_bounds__(256) void pf_quant_h_kernel(BatchedArgs a) {
@@ -244,21 +248,59 @@ struct Q6Fold {
     float d[4];  // factors of the four rows whose results the lane receives
 };
 
-// 16 bytes at a 2-byte aligned LDS address, as four words.
+// 16 bytes at a 2-byte aligned address in memory, which takes such loads at any
+// width, and in LDS.
+__device__ __forceinline__ uint4 mem_u128_a2(const uint8_t *p) {
+    typedef uint32_t v4u_a2 __attribute__((ext_vector_type(4), aligned(2)));
+    const v4u_a2 v = *reinterpret_cast<const v4u_a2 *>(p);
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
 __device__ __forceinline__ uint4 lds_u128_a2(const uint8_t *p) {
     const uint2 a = lds_u64_a2(p), b = lds_u64_a2(p + 8);
     return make_uint4(a.x, a.y, b.x, b.y);
 }
 
-__device__ __forceinline__ void q6_fold(const uint8_t *T, size_t rb, int b, Q6Fold &o) {
+// The lane's raw bytes of the block: its ql and qh pieces of both halves, the
+// scales of its groups, its row's factor; from LDS or from memory.
+struct Q6Raw {
+    uint4 ql[2], qh[2];
+    int sc[4];
+    uint32_t d;
+};
+__device__ __forceinline__ void raw_lds(const uint8_t *T, size_t rb, int b, Q6Raw &o) {
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const uint8_t *blk = T + (size_t)r * rb + (size_t)b * kQ6KBytes;
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+        o.ql[n] = lds_u128_a2(blk + 64 * n + 16 * g);
+        o.qh[n] = lds_u128_a2(blk + 128 + 32 * n + 16 * (g & 1));
+    }
+#pragma unroll
+    for (int jc = 0; jc < 4; ++jc) o.sc[jc] = (int)(int8_t)blk[192 + 4 * jc + g];
+    o.d = (uint32_t)*reinterpret_cast<const uint16_t *>(blk + 208);
+}
+__device__ __forceinline__ void raw_load(const uint8_t *W, size_t rb, int b, Q6Raw &o) {
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const uint8_t *blk = W + (size_t)r * rb + (size_t)b * kQ6KBytes;
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+        o.ql[n] = mem_u128_a2(blk + 64 * n + 16 * g);
+        o.qh[n] = mem_u128_a2(blk + 128 + 32 * n + 16 * (g & 1));
+    }
+    const uint4 sc = mem_u128_a2(blk + 192);
+    const uint32_t scw[4] = {sc.x, sc.y, sc.z, sc.w};
+#pragma unroll
+    for (int jc = 0; jc < 4; ++jc) o.sc[jc] = (int)(int8_t)(scw[jc] >> (8 * g));
+    o.d = *reinterpret_cast<const uint16_t *>(blk + 208);
+}
+
+__device__ __forceinline__ void fold(const Q6Raw &raw, Q6Fold &o) {
+    const int g = (threadIdx.x & 63) >> 4;
     const uint32_t h2 = 2u * (uint32_t)(g >> 1);
 #pragma unroll
     for (int jc = 0; jc < 4; ++jc) {
-        const uint4 ql = lds_u128_a2(blk + 64 * (jc >> 1) + 16 * g);
-        const uint4 qh = lds_u128_a2(blk + 128 + 32 * (jc >> 1) + 16 * (g & 1));
-        const int sc = (int)(int8_t)blk[192 + 4 * jc + g];
+        const uint4 ql = raw.ql[jc >> 1], qh = raw.qh[jc >> 1];
+        const int sc = raw.sc[jc];
         const v2s16 s2 = {(short)sc, (short)sc}, z2 = {(short)(128 - 32 * sc), (short)(128 - 32 * sc)};
         const uint32_t qlw[4] = {ql.x, ql.y, ql.z, ql.w}, qhw[4] = {qh.x, qh.y, qh.z, qh.w};
         int hw[4], lw[4];
@@ -280,9 +322,8 @@ __device__ __forceinline__ void q6_fold(const uint8_t *T, size_t rb, int b, Q6Fo
         o.lo[jc] = v4i{lw[0], lw[1], lw[2], lw[3]};
     }
     // the factors of the lane's four result rows, from the lanes that hold those rows
-    const uint32_t d = (uint32_t)*reinterpret_cast<const uint16_t *>(blk + 208);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) o.d[i] = half_bits_to_float((uint32_t)__shfl((int)d, 4 * g + i));
+    for (int i = 0; i < 4; ++i) o.d[i] = half_bits_to_float((uint32_t)__shfl((int)raw.d, 4 * g + i));
 }
 
 // The quants of one token's block as the Q3_K, Q5_K and Q6_K folds take them:
@@ -308,8 +349,7 @@ __device__ __forceinline__ void fold_step(const Q6Fold &w, const XOps &x, float 
     }
 }
 
-// Q3_K super-block b of a 16-row tile in LDS (row r at T + r*rb; 110-byte
-// blocks, only 2-byte aligned), folded for v_mfma_i32_16x16x64_i8.  Lane group
+// Q3_K super-block b of a 16-row tile (110-byte blocks, only 2-byte aligned), folded for v_mfma_i32_16x16x64_i8.  Lane group
 // g of chunk jc supplies elements 64 jc + 16 g .. + 15 of its row: 32-element
 // range 2 jc + g / 2 (half n = jc / 2, quarter j = 2 (jc & 1) + g / 2),
 // positions l = 16 (g & 1) .. + 15, one 16-element scale group G = 4 jc + g.
@@ -331,33 +371,14 @@ struct Q3Raw {
     uint4 hm, qv[2];
     uint32_t s[3], d;
 };
-__device__ __forceinline__ void q3_raw_lds(const uint8_t *T, size_t rb, int b, Q3Raw &o) {
-    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    const uint8_t *blk = T + (size_t)r * rb + (size_t)b * kQ3KBytes;
-    o.hm = lds_u128_a2(blk + 16 * (g & 1));
-    o.qv[0] = lds_u128_a2(blk + 32 + 16 * (g & 1));
-    o.qv[1] = lds_u128_a2(blk + 64 + 16 * (g & 1));
-    const uint2 s01 = lds_u64_a2(blk + 96);
-    o.s[0] = s01.x;
-    o.s[1] = s01.y;
-    o.s[2] = lds_u32(blk + 104);
-    o.d = (uint32_t)blk[108] | ((uint32_t)blk[109] << 8);
-}
-// The same from memory, which takes 2-byte aligned loads of any width.
 __device__ __forceinline__ void raw_load(const uint8_t *W, size_t rb, int b, Q3Raw &o) {
-    typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-    typedef uint32_t v3u __attribute__((ext_vector_type(3)));
-    typedef v4u v4u_a2 __attribute__((aligned(2)));
-    typedef v3u v3u_a2 __attribute__((aligned(2)));
+    typedef uint32_t v3u_a2 __attribute__((ext_vector_type(3), aligned(2)));
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const uint8_t *blk = W + (size_t)r * rb + (size_t)b * kQ3KBytes;
-    const v4u h = *reinterpret_cast<const v4u_a2 *>(blk + 16 * (g & 1));
-    const v4u q0 = *reinterpret_cast<const v4u_a2 *>(blk + 32 + 16 * (g & 1));
-    const v4u q1 = *reinterpret_cast<const v4u_a2 *>(blk + 64 + 16 * (g & 1));
-    const v3u sc = *reinterpret_cast<const v3u_a2 *>(blk + 96);
-    o.hm = make_uint4(h[0], h[1], h[2], h[3]);
-    o.qv[0] = make_uint4(q0[0], q0[1], q0[2], q0[3]);
-    o.qv[1] = make_uint4(q1[0], q1[1], q1[2], q1[3]);
+    const v3u_a2 sc = *reinterpret_cast<const v3u_a2 *>(blk + 96);
+    o.hm = mem_u128_a2(blk + 16 * (g & 1));
+    o.qv[0] = mem_u128_a2(blk + 32 + 16 * (g & 1));
+    o.qv[1] = mem_u128_a2(blk + 64 + 16 * (g & 1));
     o.s[0] = sc[0];
     o.s[1] = sc[1];
     o.s[2] = sc[2];
@@ -419,8 +440,7 @@ __device__ __forceinline__ void fold_step(const Q3Fold &w, const XOps &x, float 
     }
 }
 
-// Q5_K super-block b of a 16-row tile in LDS (16-byte aligned 176-byte blocks:
-// d, dmin, Q4_K-packed scales and mins, qh[32], qs[128]), folded as the Q4_K
+// Q5_K super-block b of a 16-row tile (16-byte aligned 176-byte blocks: d, dmin, Q4_K-packed scales and mins, qh[32], qs[128]), folded as the Q4_K
 // gate/up tile is: lane group g of chunk jc takes nibble g / 2 of qs bytes
 // 32 jc + 16 (g & 1) .. + 15 with bit 2 jc + g / 2 of qh[l] on top (q5 in
 // [0, 31]), sub-block s = 2 jc + g / 2.  sc_s is taken two bits at a time, so
@@ -434,11 +454,23 @@ struct Q5Fold {
     float d[4], dmin[4];  // factors of the four rows whose results the lane receives
 };
 
-__device__ __forceinline__ void q5_fold(const uint8_t *T, size_t rb, int b, Q5Fold &o) {
+// The lane's raw bytes of the block: its row's header, its half of qh (l = 16 (g & 1)
+// .. + 15) and of each chunk's qs; from LDS or from memory.
+struct Q5Raw {
+    uint4 hd, qh, qv[4];
+};
+__device__ __forceinline__ void raw_load(const uint8_t *W, size_t rb, int b, Q5Raw &o) {
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    const uint8_t *blk = T + (size_t)r * rb + (size_t)b * kQ5KBytes;
-    const uint4 hd = *reinterpret_cast<const uint4 *>(blk);
-    const uint4 qh = *reinterpret_cast<const uint4 *>(blk + 16 + 16 * (g & 1));  // qh[l], l = 16 (g & 1) .. + 15
+    const uint8_t *blk = W + (size_t)r * rb + (size_t)b * kQ5KBytes;
+    o.hd = *reinterpret_cast<const uint4 *>(blk);
+    o.qh = *reinterpret_cast<const uint4 *>(blk + 16 + 16 * (g & 1));
+#pragma unroll
+    for (int jc = 0; jc < 4; ++jc) o.qv[jc] = *reinterpret_cast<const uint4 *>(blk + 48 + 32 * jc + 16 * (g & 1));
+}
+
+__device__ __forceinline__ void fold(const Q5Raw &raw, Q5Fold &o) {
+    const int g = (threadIdx.x & 63) >> 4;
+    const uint4 hd = raw.hd, qh = raw.qh;
     uint32_t sc[2], mn[2];
     q4k_scales_packed(hd, sc, mn);
     const uint32_t qhw[4] = {qh.x, qh.y, qh.z, qh.w};
@@ -449,7 +481,7 @@ __device__ __forceinline__ void q5_fold(const uint8_t *T, size_t rb, int b, Q5Fo
     for (int jc = 0; jc < 4; ++jc) {
         const uint32_t sh = 16u * (uint32_t)(jc & 1) + bsh;  // byte 2 (jc & 1) + g / 2 of word jc / 2
         const uint32_t scs = (sc[jc >> 1] >> sh) & 0xffu;
-        const uint4 qv = *reinterpret_cast<const uint4 *>(blk + 48 + 32 * jc + 16 * (g & 1));
+        const uint4 qv = raw.qv[jc];
         const uint32_t qw[4] = {qv.x, qv.y, qv.z, qv.w};
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -488,17 +520,17 @@ __device__ __forceinline__ void fold_step(const Q5Fold &w, const XOps &x, float 
     }
 }
 
-// The fold of a type's super-block from a tile in LDS, and its operands.
+// A type's super-block of a 16-row tile: the lane's raw bytes from memory (load)
+// or from LDS (lds), their fold, and the fold's operands.
 template <int T>
 struct Tile;
 template <>
 struct Tile<kTypeQ4K> {
+    using Raw = Q4Raw;
     using Fold = Q4Fold;
-    static __device__ __forceinline__ void fold(const uint8_t *t, size_t rb, int b, Fold &o) {
-        Q4Raw raw;
-        q4_raw_load(t, rb, b, raw);
-        q4_fold(raw, o);
-    }
+    static __device__ __forceinline__ void load(const uint8_t *W, size_t rb, int b, Raw &o) { q4_raw_load(W, rb, b, o); }
+    static __device__ __forceinline__ void lds(const uint8_t *t, size_t rb, int b, Raw &o) { q4_raw_load(t, rb, b, o); }
+    static __device__ __forceinline__ void fold(const Raw &r, Fold &o) { q4_fold(r, o); }
     static __device__ __forceinline__ void load_x(const Q8L &x, XOps &o) {
         q4_load_x(x, o);
         o.bs = load_sums(x);
@@ -509,8 +541,11 @@ struct Tile<kTypeQ4K> {
 };
 template <>
 struct Tile<kTypeQ5K> {
+    using Raw = Q5Raw;
     using Fold = Q5Fold;
-    static __device__ __forceinline__ void fold(const uint8_t *t, size_t rb, int b, Fold &o) { q5_fold(t, rb, b, o); }
+    static __device__ __forceinline__ void load(const uint8_t *W, size_t rb, int b, Raw &o) { raw_load(W, rb, b, o); }
+    static __device__ __forceinline__ void lds(const uint8_t *t, size_t rb, int b, Raw &o) { raw_load(t, rb, b, o); }
+    static __device__ __forceinline__ void fold(const Raw &r, Fold &o) { hoard::fold(r, o); }
     static __device__ __forceinline__ void load_x(const Q8L &x, XOps &o) {
         q6_load_x(x, o);
         o.bs = load_sums(x);
@@ -521,8 +556,11 @@ struct Tile<kTypeQ5K> {
 };
 template <>
 struct Tile<kTypeQ6K> {
+    using Raw = Q6Raw;
     using Fold = Q6Fold;
-    static __device__ __forceinline__ void fold(const uint8_t *t, size_t rb, int b, Fold &o) { q6_fold(t, rb, b, o); }
+    static __device__ __forceinline__ void load(const uint8_t *W, size_t rb, int b, Raw &o) { raw_load(W, rb, b, o); }
+    static __device__ __forceinline__ void lds(const uint8_t *t, size_t rb, int b, Raw &o) { raw_lds(t, rb, b, o); }
+    static __device__ __forceinline__ void fold(const Raw &r, Fold &o) { hoard::fold(r, o); }
     static __device__ __forceinline__ void load_x(const Q8L &x, XOps &o) { q6_load_x(x, o); }
     static __device__ __forceinline__ void step(const Fold &w, const XOps &x, float acc[4], float accm[4]) {
         fold_step(w, x, acc, accm);
@@ -573,29 +611,32 @@ struct GateUp<kTypeQ3K> {
     }
 };
 // -- gate/up + SwiGLU ------------------------------------------------------------
-// grid (n_ff / 32, max units), block 256: wave w takes rows [32 x + 16 (w % 2), +16)
+// 32 rows of gate and of up per workgroup: wave w takes rows [32 x + 16 (w % 2), +16)
 // of gate (w < 2) or up (w >= 2) of the unit's expert against every token of the
 // unit.  Per super-block the workgroup copies the Q8_K blocks of the unit's
 // token chunks into LDS (one buffer ahead) while each wave holds the next
 // super-block of its rows in registers; the gate waves hand their values to the
 // up waves through LDS, which form h and store it to hbuf[sorted pair][row].
-// Four chunks: three workgroups share a CU (47 KB of LDS each).  Bound by its
-// vector and matrix instructions, which share a SIMD's issue, and the weight
-// stream together: Qwen3-30B at 512 tokens 89 us a launch (226 MB).  Q3_K rows
-// took 174 us at 512 tokens of 64 experts with a tile in LDS and every wave
-// loading its tokens' blocks, 120 here.
-// CH: the 16-token chunks of a unit (units of 16 CH pairs).
+// Bound by its vector and matrix instructions, which share a SIMD's issue, and
+// the weight stream together: Qwen3-30B at 512 tokens 89 us a launch (226 MB).
+// Q3_K rows took 174 us at 512 tokens of 64 experts with a tile in LDS and every
+// wave loading its tokens' blocks, 120 here.
+// LDS: xs, two buffers of the unit's Q8_K block b; gx, the gate values [row
+// tile][chunk][row i][lane].  CH: the 16-token chunks of a unit.  kInt: the blocks'
+// sums are int16 (a batch that runs dots too).
 constexpr int kXGran = (int)sizeof(Q8L) / 16;  // 16-byte granules staged per token
+template <int CH>
+constexpr int kLargeXBytes = 2 * 16 * CH * (int)sizeof(Q8L);
+template <int CH>
+constexpr int kLargeGxBytes = 2 * CH * 4 * 64 * (int)sizeof(float);
 
-template <int TG, int NB, int CH>
-__global__ __launch_bounds__(256, CH == 4 ? 3 : 4) void pf_gateup_kernel(BatchedArgs a) {
+template <int TG, int NB, int CH, bool kInt>
+__device__ __forceinline__ void gateup_large(const BatchedArgs &a, const Unit &w, uint8_t *smem) {
     using S = GateUp<TG>;
     constexpr int kTok = 16 * CH;
     constexpr int kXChunksPerBlock = (kTok * kXGran + 63) / 64;  // 1 KB copies per unit block
-    __shared__ __align__(16) Q8L xs[2][kTok];  // the unit's Q8_K block b (two buffers)
-    __shared__ float gx[2][CH][4][64];         // gate values: [row tile][chunk][row i][lane]
-    Unit w;
-    if (!load_unit(a, blockIdx.y, w)) return;
+    Q8L(*xs)[kTok] = reinterpret_cast<Q8L(*)[kTok]>(smem);
+    float(*gx)[CH][4][64] = reinterpret_cast<float(*)[CH][4][64]>(smem + kLargeXBytes<CH>);
     const int wave = wave_index(), lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
     const int m = wave >> 1, rt = wave & 1;
     const int row0 = blockIdx.x * kGuRows + rt * kWaveRows;
@@ -656,7 +697,12 @@ __global__ __launch_bounds__(256, CH == 4 ? 3 : 4) void pf_gateup_kernel(Batched
                 const Q8L &x = xb[ch * 16 + c];
                 XOps xo;
                 S::load_x(x, xo);
-                xo.bs = load_sums(x);
+                if constexpr (kInt) {
+                    const v4i *b2 = reinterpret_cast<const v4i *>(x.bsums), s2[2] = {b2[0], b2[1]};
+                    xo.bs = sums_from_int<TG>(s2, q & 1);
+                } else {
+                    xo.bs = load_sums(x);
+                }
                 xo.xd = x.d;
                 S::step(t, xo, acc[ch], accm[ch]);
             }
@@ -686,12 +732,12 @@ __global__ __launch_bounds__(256, CH == 4 ? 3 : 4) void pf_gateup_kernel(Batched
 }
 
 // -- gate/up + SwiGLU for units of at most 16 pairs ------------------------------
-// grid (n_ff / 32, max units), block 256, waves as above.  With one token chunk
-// a wave's registers leave room for kDepth super-blocks of raw weights in
-// flight, and all of the unit's activation blocks fit LDS at once (39 KB, four
-// workgroups a CU): one barrier after they land, then every wave streams its
-// rows from memory at its own pace.  Qwen3.5 at 131 tokens (302 MB): 85 -> 72 us
-// a launch against units of 64; Q3_K at 27 tokens 75 (per-token dots) -> 54.
+// Rows and waves as above.  With one token chunk a wave's registers leave room
+// for kDepth super-blocks of raw weights in flight, and all of the unit's
+// activation blocks fit LDS at once (39 KB, four workgroups a CU): one barrier
+// after they land, then every wave streams its rows from memory at its own
+// pace.  Qwen3.5 at 131 tokens (302 MB): 85 -> 72 us a launch against units of
+// 64; Q3_K at 27 tokens 75 (per-token dots) -> 54.
 // The quants and scale of a Q8_K block in LDS (17 granules: 16 tokens' reads
 // of one place fall into different banks).
 struct Q8S {
@@ -700,16 +746,16 @@ struct Q8S {
     int32_t pad[3];
 };
 static_assert(sizeof(Q8S) == 272 && offsetof(Q8L, d) == 288 && offsetof(Q8L, bsums) == 256, "Q8S from Q8L");
+template <int NB>
+constexpr int kSmallLds = NB * 16 * (int)sizeof(Q8S) + NB * 32 * 16;
 
-template <int TG, int NB>
-__global__ __launch_bounds__(256, 4) void pf_gateup16_kernel(BatchedArgs a) {
+template <int TG, int NB, bool kInt>
+__device__ __forceinline__ void gateup_small(const BatchedArgs &a, const Unit &w, uint8_t *smem) {
     using S = GateUp<TG>;
     constexpr int D = S::kDepth, kGran = (int)sizeof(Q8S) / 16, kCopies = (16 * kGran + 63) / 64;
     static_assert(NB % 4 == 0 && NB >= D, "a wave copies NB / 4 blocks of every token");
-    __shared__ __align__(16) Q8S xs[NB][16];
-    __shared__ __align__(16) v8h sums[NB][32];
-    Unit w;
-    if (!load_unit(a, blockIdx.y, w)) return;
+    Q8S(*xs)[16] = reinterpret_cast<Q8S(*)[16]>(smem);
+    v4i(*sums)[32] = reinterpret_cast<v4i(*)[32]>(smem + NB * 16 * sizeof(Q8S));
     const int wave = wave_index(), lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
     const int m = wave >> 1, rt = wave & 1;
     const int row0 = blockIdx.x * kGuRows + rt * kWaveRows;
@@ -754,7 +800,12 @@ __global__ __launch_bounds__(256, 4) void pf_gateup16_kernel(BatchedArgs a) {
         const Q8S &x = xs[b][c];
         XOps xo;
         xo.xd = x.d;
-        xo.bs = sums[b][2 * c + (q & 1)];
+        if constexpr (kInt) {
+            const v4i s2[2] = {sums[b][2 * c], sums[b][2 * c + 1]};
+            xo.bs = sums_from_int<TG>(s2, q & 1);
+        } else {
+            xo.bs = __builtin_bit_cast(v8h, sums[b][2 * c + (q & 1)]);
+        }
         S::load_x(x, xo);
         S::step(f, xo, acc, accm);
     }
@@ -777,12 +828,55 @@ __global__ __launch_bounds__(256, 4) void pf_gateup16_kernel(BatchedArgs a) {
         make_float4(hv[0], hv[1], hv[2], hv[3]);
 }
 
+// grid (n_ff / 32, max units), block 256.  With kRows = 16 rows of a dot unit per
+// workgroup it is (n_ff / 16, max units) and an MFMA unit leaves the upper half of
+// the row blocks idle.
+template <int TG, int NB, int kRows>
+__global__ __launch_bounds__(256, 4) void gateup_dots_kernel(BatchedArgs a) {
+    using Dots = DotGateUp<TG, NB>;
+    __shared__ __align__(16) uint8_t smem[Dots::kLds > kSmallLds<NB> ? Dots::kLds : kSmallLds<NB>];
+    Unit w;
+    if (!load_unit(a, blockIdx.y, w)) return;
+    if (w.dots) {
+#pragma unroll 1
+        for (int r = 0; r < kRows; r += kDotGuRows) {
+            if (r > 0) __syncthreads();  // every wave is done with the rows before
+            Dots::run(a, w, blockIdx.x * kRows + r, smem);
+        }
+    } else if (kRows != kGuRows) {
+        if ((int)blockIdx.x * kGuRows < a.n_ff) gateup_small<TG, NB, true>(a, w, smem);
+    } else if (w.n <= 16) {
+        gateup_small<TG, NB, true>(a, w, smem);
+    } else {
+        gateup_large<TG, NB, 2, true>(a, w, smem);
+    }
+}
+template <int TG, int NB>
+__global__ __launch_bounds__(256, 4) void gateup_mixed_kernel(BatchedArgs a) {
+    constexpr int CH = 2;
+    static_assert(kSmallLds<NB> >= kLargeXBytes<CH> + kLargeGxBytes<CH>, "both units' LDS");
+    __shared__ __align__(16) uint8_t smem[kSmallLds<NB>];
+    Unit w;
+    if (!load_unit(a, blockIdx.y, w)) return;
+    if (w.n <= 16)
+        gateup_small<TG, NB, false>(a, w, smem);
+    else
+        gateup_large<TG, NB, CH, false>(a, w, smem);
+}
+// Three workgroups share a CU (47 KB of LDS each).
+template <int TG, int NB>
+__global__ __launch_bounds__(256, 3) void gateup_large_kernel(BatchedArgs a) {
+    __shared__ __align__(16) uint8_t smem[kLargeXBytes<4> + kLargeGxBytes<4>];
+    Unit w;
+    if (load_unit(a, blockIdx.y, w)) gateup_large<TG, NB, 4, false>(a, w, smem);
+}
+
 // -- down: 64 rows of the unit's expert, y to its (token, slot) place -----------
-// grid (n_embd / 64, max units), block 256.  Each wave copies its own 16 rows
-// into LDS in one burst and waits for them alone (no barrier before the folds);
-// each super-block of them is folded once, then run against every token chunk
-// of the unit (CH of 16 pairs).  TS: the shared expert's row type beside
-// routed rows of type TD (Qwen3.5: Q6_K beside Q5_K), in the same launch.
+// block 256.  Each wave copies its own 16 rows into LDS in one burst and waits
+// for them alone (no barrier before the folds); each super-block of them is
+// folded once, then run against every token chunk of a pass (CH of 16 pairs).
+// TS: the shared expert's row type beside routed rows of type TD (Qwen3.5: Q6_K
+// beside Q5_K), in the same launch.
 // With four chunks, Q6_K keeps two operand sets (chunk ch's loaded while the one
 // before it computes, three workgroups a CU); Q4_K and Q5_K load every chunk's
 // before the fold, which covers them, and one chunk always is.
@@ -797,11 +891,13 @@ __device__ __forceinline__ void down_rows16(const uint8_t *tile, int nch, const 
     };
 #pragma unroll 1
     for (int b = 0; b < NBH; ++b) {
+        typename K::Raw raw;
         typename K::Fold f;
         if constexpr (T == kTypeQ6K && CH == 4) {
             XOps xa, xb;
             load_x(0, b, xa);
-            K::fold(tile, NBH * QType<T>::bytes, b, f);
+            K::lds(tile, NBH * QType<T>::bytes, b, raw);
+            K::fold(raw, f);
             if (nch > 1) load_x(1, b, xb);
             K::step(f, xa, acc[0], accm[0]);
             if (nch > 1) {
@@ -818,7 +914,8 @@ __device__ __forceinline__ void down_rows16(const uint8_t *tile, int nch, const 
 #pragma unroll
             for (int ch = 0; ch < CH; ++ch)
                 if (ch < nch) load_x(ch, b, xc[ch]);
-            K::fold(tile, NBH * QType<T>::bytes, b, f);
+            K::lds(tile, NBH * QType<T>::bytes, b, raw);
+            K::fold(raw, f);
 #pragma unroll
             for (int ch = 0; ch < CH; ++ch)
                 if (ch < nch) K::step(f, xc[ch], acc[ch], accm[ch]);
@@ -826,90 +923,202 @@ __device__ __forceinline__ void down_rows16(const uint8_t *tile, int nch, const 
     }
 }
 
-template <int TD, int NBH, int TS, int CH>
-constexpr int kDownWaves = CH == 1 ? 4 : (CH == 2 || TD == kTypeQ6K) ? 3 : 2;  // waves a SIMD (register bound)
-
-template <int TD, int NBH, int TS, int CH>
-__global__ __launch_bounds__(256, (kDownWaves<TD, NBH, TS, CH>)) void pf_down_kernel(BatchedArgs a) {
-    constexpr int kRowBytesD = NBH * QType<TD>::bytes, kRowBytesS = NBH * QType<TS>::bytes;
-    constexpr int kTileBytes = kDnRows * (kRowBytesD > kRowBytesS ? kRowBytesD : kRowBytesS);
+// kPairs: the most pairs of a unit; CH, CHS: the chunks of a pass over the tile,
+// of routed rows and of the shared expert's (a unit of more takes several
+// passes, its rows folded again for each).
+template <int TD, int NBH, int TS, int kPairs, int CH, int CHS = CH>
+struct DownTile {
+    static constexpr int kRowBytesD = NBH * QType<TD>::bytes, kRowBytesS = NBH * QType<TS>::bytes;
     static_assert(kWaveRows * kRowBytesD % 16 == 0 && kWaveRows * kRowBytesS % 16 == 0, "16-byte copies");
-    __shared__ __align__(16) uint8_t tile[kTileBytes];
-    __shared__ int yrow[16 * CH];  // y row (token * slots + slot) of each of the unit's pairs
-    __shared__ __align__(16) float xds[4][16 * CH][4];  // each wave's copy of the pairs' Q8_K(h) scales
-    Unit w;
-    if (!load_unit(a, blockIdx.y, w)) return;
-    const bool shx = TS != TD && a.sh && w.e == a.n_ids;  // the shared expert's rows
-    const int wave = wave_index(), lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
-    const int rt0 = blockIdx.x * kDnRows;
-    // the pairs' places, read while the tile lands
-    const int tid = threadIdx.x;
-    const int pt = tid < w.n ? a.ptok[w.p0 + tid] : 0, ps = tid < w.n ? a.pslot[w.p0 + tid] : 0;
-    const int wbytes = kWaveRows * (shx ? kRowBytesS : kRowBytesD);
-    uint8_t *T = tile + wave * wbytes;
-    // the pairs' block scales with the tile: a 4-byte load of a scale with every
-    // chunk's quants cost more
-    if (CH == 4 || lane < 16 * CH)
-        dma_lanes(reinterpret_cast<uint8_t *>(&xds[wave][0][0]),
-                  reinterpret_cast<const uint8_t *>(a.q8hd + (size_t)(w.p0 + min(lane, w.n - 1)) * 4));
-    dma_wave_copy_nt(T, batched_down(a, w.e) + (size_t)(rt0 + wave * kWaveRows) * (wbytes / kWaveRows), wbytes);
-    lds_dma_wait();
-    if (tid < w.n) yrow[tid] = pt * (a.k + a.sh) + ps;
-    const int nch = (w.n + 15) >> 4;
-    const Q8L *x0 = reinterpret_cast<const Q8L *>(a.q8h) + (size_t)w.p0 * NBH;
-    int xi[CH];  // the lane's pair of each chunk (places past the last repeat it)
+    // LDS: the tile, y row (token * slots + slot) of each of the unit's pairs,
+    // each wave's copy of the pairs' Q8_K(h) scales
+    static constexpr int kTileBytes = kDnRows * (kRowBytesD > kRowBytesS ? kRowBytesD : kRowBytesS);
+    static constexpr int kLds = kTileBytes + kPairs * (int)sizeof(int) + 4 * kPairs * 4 * (int)sizeof(float);
+
+    template <int T, int C>
+    static __device__ __forceinline__ void passes(const BatchedArgs &a, const Unit &w, const uint8_t *tile,
+                                                  const int *yrow, const float (*xds)[4], int row0) {
+        const int lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
+        const Q8L *x0 = reinterpret_cast<const Q8L *>(a.q8h) + (size_t)w.p0 * NBH;
+        constexpr bool kOne = kPairs == 16 * C;
+        if (!kOne) __syncthreads();  // yrow is written
+#pragma unroll 1
+        for (int p0 = 0; p0 < w.n; p0 += 16 * C) {
+            const int nch = min((w.n - p0 + 15) >> 4, C);
+            int xi[C];  // the lane's pair of each chunk (places past the last repeat it)
 #pragma unroll
-    for (int ch = 0; ch < CH; ++ch) xi[ch] = min(ch * 16 + c, w.n - 1);
-    float acc[CH][4], accm[CH][4];
+            for (int ch = 0; ch < C; ++ch) xi[ch] = min(p0 + ch * 16 + c, w.n - 1);
+            float acc[C][4], accm[C][4];
 #pragma unroll
-    for (int ch = 0; ch < CH; ++ch)
+            for (int ch = 0; ch < C; ++ch)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[ch][i] = accm[ch][i] = 0.0f;
-    if (TS != TD && shx)
-        down_rows16<TS, NBH, CH>(T, nch, x0, xi, xds[wave], acc, accm);
-    else
-        down_rows16<TD, NBH, CH>(T, nch, x0, xi, xds[wave], acc, accm);
-    __syncthreads();  // yrow is written
+                for (int i = 0; i < 4; ++i) acc[ch][i] = accm[ch][i] = 0.0f;
+            down_rows16<T, NBH, C>(tile, nch, x0, xi, xds + p0, acc, accm);
+            if (kOne) __syncthreads();  // yrow is written
 #pragma unroll
-    for (int ch = 0; ch < CH; ++ch) {
-        const int idx = ch * 16 + c;
-        if (ch < nch && idx < w.n) {
-            // accm stays 0 for rows without a min term
-            *reinterpret_cast<float4 *>(a.ybuf + (size_t)yrow[idx] * a.n_embd + rt0 + wave * kWaveRows + 4 * q) =
-                make_float4(acc[ch][0] - accm[ch][0], acc[ch][1] - accm[ch][1], acc[ch][2] - accm[ch][2],
-                            acc[ch][3] - accm[ch][3]);
+            for (int ch = 0; ch < C; ++ch) {
+                const int idx = p0 + ch * 16 + c;
+                if (ch < nch && idx < w.n) {
+                    // accm stays 0 for rows without a min term
+                    *reinterpret_cast<float4 *>(a.ybuf + (size_t)yrow[idx] * a.n_embd + row0 + 4 * q) =
+                        make_float4(acc[ch][0] - accm[ch][0], acc[ch][1] - accm[ch][1], acc[ch][2] - accm[ch][2],
+                                    acc[ch][3] - accm[ch][3]);
+                }
+            }
+            if (kOne) break;
         }
     }
+
+    static __device__ __forceinline__ void run(const BatchedArgs &a, const Unit &w, uint8_t *smem) {
+        int *yrow = reinterpret_cast<int *>(smem + kTileBytes);
+        float(*xds)[kPairs][4] = reinterpret_cast<float(*)[kPairs][4]>(yrow + kPairs);
+        const bool shx = TS != TD && a.sh && w.e == a.n_ids;  // the shared expert's rows
+        const int wave = wave_index(), lane = threadIdx.x & 63, tid = threadIdx.x;
+        const int row0 = blockIdx.x * kDnRows + wave * kWaveRows;
+        // the pairs' places, read while the tile lands
+        const int pt = tid < w.n ? a.ptok[w.p0 + tid] : 0, ps = tid < w.n ? a.pslot[w.p0 + tid] : 0;
+        const int wbytes = kWaveRows * (shx ? kRowBytesS : kRowBytesD);
+        uint8_t *T = smem + wave * wbytes;
+        // the pairs' block scales with the tile: a 4-byte load of a scale with every
+        // chunk's quants cost more
+        if (kPairs == 64 || lane < kPairs)
+            dma_lanes(reinterpret_cast<uint8_t *>(&xds[wave][0][0]),
+                      reinterpret_cast<const uint8_t *>(a.q8hd + (size_t)(w.p0 + min(lane, w.n - 1)) * 4));
+        dma_wave_copy_nt(T, batched_down(a, w.e) + (size_t)row0 * (wbytes / kWaveRows), wbytes);
+        lds_dma_wait();
+        if (tid < w.n) yrow[tid] = pt * (a.k + a.sh) + ps;
+        if (TS != TD && shx)
+            passes<TS, CHS>(a, w, T, yrow, xds[wave], row0);
+        else
+            passes<TD, CH>(a, w, T, yrow, xds[wave], row0);
+    }
+};
+
+// -- down for the 16-pair units beside dot units -----------------------
+// 64 rows per workgroup, 16 a wave.  Q8_K(h) of the unit's pairs is formed in
+// LDS as the dots form it (no launch of its own), the rows come from memory with
+// two super-blocks of raw bytes in flight.
+template <int T, int NBH>
+__device__ __forceinline__ void down_small(const BatchedArgs &a, const Unit &w, Q8L *q8h) {
+    using K = Tile<T>;
+    constexpr int D = 2;
+    static_assert(NBH >= D, "the raw bytes' ring");
+    const int wave = wave_index(), lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
+    const int row0 = blockIdx.x * kDnRows + wave * kWaveRows;
+    constexpr size_t rb = (size_t)NBH * QType<T>::bytes;
+    const uint8_t *W = batched_down(a, w.e) + (size_t)row0 * rb;
+    const float *h = a.hbuf + (size_t)w.p0 * a.n_ff;  // the pairs' h is contiguous
+    const int pc = w.p0 + min(c, w.n - 1), yr = a.ptok[pc] * (a.k + a.sh) + a.pslot[pc];
+    WaveQuant<4> hq;
+    hq.load(h, wave, w.n * NBH, 4);
+    typename K::Raw raw[D];
+#pragma unroll
+    for (int i = 0; i < D; ++i) K::load(W, rb, i, raw[i]);
+    hq.form<kSums32>(h, q8h, wave, w.n * NBH, 4);
+    lds_barrier();
+    const Q8L *x = q8h + min(c, w.n - 1) * NBH;
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f}, accm[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int b = 0; b < NBH; ++b) {
+        typename K::Fold f;
+        K::fold(raw[b % D], f);
+        if (b + D < NBH) K::load(W, rb, b + D, raw[b % D]);
+        XOps xo;
+        K::load_x(x[b], xo);
+        xo.xd = x[b].d;
+        K::step(f, xo, acc, accm);
+    }
+    if (c < w.n)
+        *reinterpret_cast<float4 *>(a.ybuf + (size_t)yr * a.n_embd + row0 + 4 * q) =
+            make_float4(acc[0] - accm[0], acc[1] - accm[1], acc[2] - accm[2], acc[3] - accm[3]);
+}
+
+// grid (n_embd / 64, max units)
+template <int TD, int NBH, int TS>
+__global__ __launch_bounds__(256, (TD == kTypeQ4K && NBH > 2) || (TD == kTypeQ5K && NBH > 2) ? 3 : 4) void down_dots_kernel(BatchedArgs a) {
+    static_assert(kDnRows == 32 * kRowSets, "both units' rows per workgroup");
+    __shared__ __align__(16) Q8L q8h[16 * NBH];
+    Unit w;
+    if (!load_unit(a, blockIdx.y, w)) return;
+    if (TS != TD && a.sh && w.e == a.n_ids) {
+        if (w.dots)
+            down_dots<TS, NBH>(a, w, q8h);
+        else
+            down_small<TS, NBH>(a, w, q8h);
+    } else {
+        if (w.dots)
+            down_dots<TD, NBH>(a, w, q8h);
+        else
+            down_small<TD, NBH>(a, w, q8h);
+    }
+}
+// Waves a SIMD (register bound).
+template <int TD, int NBH>
+constexpr int kMixedWaves = TD == kTypeQ5K && NBH > 2 ? 3 : 4;
+template <int TD, int NBH, int TS>
+__global__ __launch_bounds__(256, (kMixedWaves<TD, NBH>)) void down_mixed_kernel(BatchedArgs a) {
+    using Small = DownTile<TD, NBH, TS, 16, 1>;
+    // (two chunks of Q6_K beside Q5_K rows take the registers of a fourth wave)
+    using Large = DownTile<TD, NBH, TS, 32, 2, TS == TD ? 2 : 1>;
+    __shared__ __align__(16) uint8_t smem[Large::kLds];
+    Unit w;
+    if (!load_unit(a, blockIdx.y, w)) return;
+    if (w.n <= 16)
+        Small::run(a, w, smem);
+    else
+        Large::run(a, w, smem);
+}
+template <int TD, int NBH, int TS>
+__global__ __launch_bounds__(256, TD == kTypeQ6K ? 3 : 2) void down_large_kernel(BatchedArgs a) {
+    using Large = DownTile<TD, NBH, TS, 64, 4>;
+    __shared__ __align__(16) uint8_t smem[Large::kLds];
+    Unit w;
+    if (load_unit(a, blockIdx.y, w)) Large::run(a, w, smem);
+}
+
+template <int TG>
+void launch_gateup_units(const BatchedArgs &a, hipStream_t s) {
+    const dim3 gg(a.n_ff / kGuRows, a.max_units);
+    if (a.units_mode == kUnitsDots)
+        hipLaunchKernelGGL((gateup_dots_kernel<TG, 8, kDotGuRows>), dim3(a.n_ff / kDotGuRows, a.max_units), dim3(256), 0, s, a);
+    else if (a.units_mode == kUnitsDotGateUp)
+        hipLaunchKernelGGL((gateup_dots_kernel<TG, 8, kGuRows>), gg, dim3(256), 0, s, a);
+    else if (a.units_mode == kUnitsMixed)
+        hipLaunchKernelGGL((gateup_mixed_kernel<TG, 8>), gg, dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((gateup_large_kernel<TG, 8>), gg, dim3(256), 0, s, a);
+}
+
+template <int TD, int NBH, int TS>
+void launch_down_units(const BatchedArgs &a, hipStream_t s) {
+    const dim3 dg(a.n_embd / kDnRows, a.max_units);
+    if (a.units_mode == kUnitsDots)
+        hipLaunchKernelGGL((down_dots_kernel<TD, NBH, TS>), dg, dim3(256), 0, s, a);
+    else if (a.units_mode <= kUnitsMixed)
+        hipLaunchKernelGGL((down_mixed_kernel<TD, NBH, TS>), dg, dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((down_large_kernel<TD, NBH, TS>), dg, dim3(256), 0, s, a);
 }
 
 }  // namespace
 
-namespace {
-
-template <int CH>
-hipError_t launch_units(const BatchedArgs &a, hipStream_t s) {
-    const int nbh = a.n_ff / QK;
-    const dim3 gg(a.n_ff / kGuRows, a.max_units);
-    if (a.gu_type == kTypeQ4K) {
-        if constexpr (CH == 1)
-            hipLaunchKernelGGL((pf_gateup16_kernel<kTypeQ4K, 8>), gg, dim3(256), 0, s, a);
-        else
-            hipLaunchKernelGGL((pf_gateup_kernel<kTypeQ4K, 8, CH>), gg, dim3(256), 0, s, a);
-    } else if (a.gu_type == kTypeQ3K) {
-        if constexpr (CH == 1)
-            hipLaunchKernelGGL((pf_gateup16_kernel<kTypeQ3K, 8>), gg, dim3(256), 0, s, a);
-        else
-            hipLaunchKernelGGL((pf_gateup_kernel<kTypeQ3K, 8, CH>), gg, dim3(256), 0, s, a);
-    } else {
+hipError_t launch_expert_units(const BatchedArgs &a, hipStream_t s) {
+    if (a.n_embd != 2048 || a.n_ff % kGuRows || a.n_embd % kDnRows || a.n_ff / QK > 4 || a.max_units < 1)
         return hipErrorInvalidValue;
-    }
-    hipLaunchKernelGGL(pf_quant_h_kernel, dim3(a.M * (a.k + a.sh)), dim3(64 * nbh), 0, s, a);
-    const dim3 dg(a.n_embd / kDnRows, a.max_units);
+    const int nbh = a.n_ff / QK;
+    if (a.gu_type == kTypeQ4K)
+        launch_gateup_units<kTypeQ4K>(a, s);
+    else if (a.gu_type == kTypeQ3K)
+        launch_gateup_units<kTypeQ3K>(a, s);
+    else
+        return hipErrorInvalidValue;
+    if (a.units_mode != kUnitsDots)  // (the launch with down dots forms it)
+        hipLaunchKernelGGL(pf_quant_h_kernel, dim3(a.M * (a.k + a.sh)), dim3(64 * nbh), 0, s, a);
     const int sd = a.sh ? a.sh_d_type : a.d_type;
-// one kernel instance per (routed down type, super-blocks per row, shared down type)
-#define HOARD_DOWN(T, N, TS)                                                          \
-    if (a.d_type == T && nbh == N && sd == TS) {                                      \
-        hipLaunchKernelGGL((pf_down_kernel<T, N, TS, CH>), dg, dim3(256), 0, s, a);   \
+// one set of kernels per (routed down type, super-blocks per row, shared down type)
+#define HOARD_DOWN(T, N, TS)                          \
+    if (a.d_type == T && nbh == N && sd == TS) {      \
+        launch_down_units<T, N, TS>(a, s);            \
     } else
     HOARD_DOWN(kTypeQ6K, 3, kTypeQ6K)
     HOARD_DOWN(kTypeQ6K, 2, kTypeQ6K)
@@ -924,16 +1133,6 @@ hipError_t launch_units(const BatchedArgs &a, hipStream_t s) {
     }
 #undef HOARD_DOWN
     return hipGetLastError();
-}
-
-}  // namespace
-
-hipError_t launch_prefill_groups(const BatchedArgs &a, hipStream_t s) {
-    if (a.n_embd != 2048 || a.n_ff % kGuRows || a.n_embd % kDnRows || a.n_ff / QK > 4 || a.max_units < 1)
-        return hipErrorInvalidValue;
-    const hipError_t e = a.unit == 16 ? launch_units<1>(a, s) : a.unit == 32 ? launch_units<2>(a, s)
-                         : a.unit == kUnitTokens ? launch_units<4>(a, s) : hipErrorInvalidValue;
-    return e;
 }
 
 }  // namespace hoard

@@ -266,6 +266,7 @@ struct WaveQuant {
     __device__ __forceinline__ void get(int i, const float *x, int b) {
         v[i] = *reinterpret_cast<const f32x4_a4 *>(x + (size_t)b * QK + 4 * (threadIdx.x & 63));
     }
+    template <int Sums = kSumsInt>
     __device__ __forceinline__ void form(const float *x, Q8L *q, int first, int end, int step) {
 #pragma unroll 1
         for (int b = first; b < end; b += step) {
@@ -273,7 +274,7 @@ struct WaveQuant {
 #pragma unroll
             for (int i = 0; i + 1 < K; ++i) v[i] = v[i + 1];
             if (b + K * step < end) get(K - 1, x, b + K * step);
-            wave_quantize_q8l_regs(w, q + b);
+            wave_quantize_q8l_regs<Sums>(w, q + b);
         }
     }
 };
