@@ -517,19 +517,18 @@ int pool_ensure(hoard_moe *h, int layer, const int32_t *sel, int n, bool sequent
         f.n_ids = n;
         for (int j = 0; j < n; ++j) {
             f.slot[j] = slots[j];
-            h->stats.reqs += 1;
-            if (!miss[j]) {
-                h->stats.hits += 1;
-                continue;
-            }
+            if (!miss[j]) continue;
             if (h->fail_upload > 0 && --h->fail_upload == 0) POOL_TRY(hipErrorOutOfMemory);
             f.src[f.n] = L.host_experts + (size_t)sel[j] * f.bytes;
             f.dst[f.n++] = L.slots + (size_t)slots[j] * f.bytes;
-            h->stats.misses += 1;
-            h->stats.bytes_h2d += f.bytes;
         }
         if (f.n && L.used) POOL_TRY(hipStreamWaitEvent(s, L.last_use, 0));
         POOL_TRY(hoard::launch_slot_fill(f, s));
+        // counted once issued: of a refused step nothing was
+        h->stats.reqs += n;
+        h->stats.hits += n - f.n;
+        h->stats.misses += f.n;
+        h->stats.bytes_h2d += f.n * f.bytes;
         return HOARD_OK;
     }
     // misses are dealt round-robin to the caller's copy stream and the internal
