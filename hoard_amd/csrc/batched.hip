@@ -115,7 +115,7 @@ __device__ void group_by_expert(const BatchedArgs &a, GroupLds &g, const int *se
 // Groups in ascending expert order and their units from the per-expert pair
 // counts g.cnt (wave 0 of the grouping workgroup): hist, the unit records {expert,
 // first sorted pair, pairs, 0} (every place past the last unit zeroed),
-// n_unique / n_units, and g.base[e] / g.ubase[e], the first sorted place and
+// n_unique, and g.base[e] / g.ubase[e], the first sorted place and
 // the first unit of expert e.  The shared expert's units, which hold the most
 // pairs and take longest, come first: at the end they outlast the rest (512
 // experts, 16 tokens 68 us/layer, 61 so; 256 experts 57 and 51).
@@ -158,7 +158,6 @@ __device__ void group_units(const BatchedArgs &a, GroupLds &g) {
         }
         if (lane == 63) {
             a.n_unique[0] = ig - a.sh;  // routed experts used
-            a.n_units[0] = iu;
             g.total = ip;  // pairs in all groups
         }
         // the grid's unit places past the last unit hold no pairs, so a workgroup
@@ -745,7 +744,7 @@ bool args_ok(const BatchedArgs &a) {
            (a.gu_type == kTypeQ4K || a.gu_type == kTypeQ3K) &&
            a.k + a.sh <= kMaxK && a.n_ids >= 1 && a.n_ids + a.sh <= kMaxExperts && a.E + a.sh <= kMaxExperts &&
            (!a.sh || (a.sh == 1 && a.sh_gate && a.sh_up && a.sh_down && a.sh_gate_inp && a.sgl)) &&
-           a.ptok && a.pslot && a.pexp && a.units && a.n_units;
+           a.ptok && a.pslot && a.pexp && a.units;
 }
 
 }  // namespace

@@ -1214,10 +1214,9 @@ namespace {
 // that what the fixed scratch of the allocation-free entry point takes and
 // refuses stays as it is.
 struct BatchedLayout {
-    int T, Ts, umax, umax_s, max_units;
+    int T, Ts, umax_s, max_units;
     size_t q8x, q8h, hbuf, ybuf, n_ints, hist, counters;  // bytes (n_ints: ints)
-    size_t o_ysrc, o_bad, o_ptok, o_pslot, o_pexp, o_units, o_q8hd,
-        o_nunits, o_sgl;
+    size_t o_ysrc, o_bad, o_ptok, o_pslot, o_pexp, o_units, o_q8hd, o_sgl;
 };
 
 BatchedLayout batched_layout(const hoard_moe_cfg &c, int T) {
@@ -1229,7 +1228,6 @@ BatchedLayout batched_layout(const hoard_moe_cfg &c, int T) {
     L.T = T;
     L.Ts = std::min(T, hoard::kBatchedMaxTokens);
     L.umax_s = std::min(E, L.Ts * k);
-    L.umax = std::min(E, T * k);
     // the most units of any size a batch takes
     L.max_units = std::max(hoard::prefill_max_units(T, k, E, hoard::kUnitTokensMin),
                            hoard::prefill_max_units(std::min(T, hoard::kMaxDotTokens), k, E, hoard::kDotTokens));
@@ -1251,7 +1249,6 @@ BatchedLayout batched_layout(const hoard_moe_cfg &c, int T) {
     L.o_pexp = take(pairs);
     L.o_units = take((size_t)4 * L.max_units);
     L.o_q8hd = take((size_t)4 * pairs);  // floats
-    L.o_nunits = take(1);
     L.o_sgl = take(T);  // floats
     L.n_ints = o;
     L.hist = sizeof(unsigned) * E;
@@ -1273,7 +1270,6 @@ void bind_batched(hoard::BatchedArgs &a, const BatchedLayout &L, uint8_t *q8x, u
     a.pexp = ints + L.o_pexp;
     a.units = ints + L.o_units;
     a.q8hd = reinterpret_cast<float *>(ints + L.o_q8hd);
-    a.n_units = ints + L.o_nunits;
     a.sgl = reinterpret_cast<float *>(ints + L.o_sgl);
     a.hist = hist;
     a.counters = counters;

@@ -33,8 +33,6 @@ constexpr int kWaveRows = 16;  // rows per wave: one MFMA tile
 constexpr int kGuRows = 32;    // gate (and up) rows per workgroup: two 16-row tiles
 constexpr int kDnRows = 64;    // down rows per workgroup
 
-__device__ __forceinline__ const Q8L *q8c(const uint8_t *p) { return reinterpret_cast<const Q8L *>(p); }
-
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 

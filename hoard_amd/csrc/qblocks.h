@@ -33,9 +33,6 @@ __host__ __device__ constexpr int kquant_block_bytes(int type) {
                             : type == kTypeQ6K ? kQ6KBytes
                                                : type == kTypeQ5K ? kQ5KBytes : type == kTypeQ3K ? kQ3KBytes : 0;
 }
-// Types whose blocks carry a min term (value = d*sc*q - dmin*m).
-__host__ __device__ constexpr bool kquant_has_min(int type) { return type == kTypeQ4K || type == kTypeQ5K; }
-
 template <int T>
 struct QType;
 template <>
@@ -61,15 +58,6 @@ struct QType<kTypeQ3K> {
 
 __device__ __forceinline__ float half_bits_to_float(uint32_t bits16) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)bits16);
-}
-
-// 32-bit little-endian word at a 2-byte aligned LDS address.
-__device__ __forceinline__ uint32_t lds_u32(const uint8_t *p) {
-    const uintptr_t a = reinterpret_cast<uintptr_t>(p);
-    const uint32_t *w = reinterpret_cast<const uint32_t *>(a & ~(uintptr_t)3);
-    const uint32_t sh = (uint32_t)(a & 3u);
-    if (sh == 0) return w[0];
-    return __builtin_amdgcn_alignbyte(w[1], w[0], sh);
 }
 
 // ggml's nearest_int (round to nearest even through the fp32 adder).

@@ -83,48 +83,6 @@ __device__ __forceinline__ float g8_row_q5k(const uint8_t *row, const Q8L *x, in
     return acc - accm;
 }
 
-// One Q6_K row of nb super-blocks (2-byte aligned in LDS) dotted with x.
-// Lane t covers positions l in [8*(t&3), +8) of half t>>2 for all four
-// 32-element quarters: 32 of the block's 256 elements.
-__device__ __forceinline__ float g8_row_q6k(const uint8_t *row, const Q8L *x, int nb, int t) {
-    const int n = t >> 2, lh = t & 3;
-    float acc = 0.0f;
-#pragma unroll
-    for (int b = 0; b < nb; ++b) {
-        const uint8_t *blk = row + b * kQ6KBytes;
-        const Q8L &xb = x[b];
-        int s[4] = {0, 0, 0, 0}, z[4] = {0, 0, 0, 0};
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-            const uint32_t A = lds_u32(blk + 64 * n + 8 * lh + 4 * w);
-            const uint32_t B = lds_u32(blk + 64 * n + 32 + 8 * lh + 4 * w);
-            const uint32_t C = lds_u32(blk + 128 + 32 * n + 8 * lh + 4 * w);
-            const uint32_t q[4] = {
-                (A & 0x0f0f0f0fu) | ((C & 0x03030303u) << 4),
-                (B & 0x0f0f0f0fu) | (((C >> 2) & 0x03030303u) << 4),
-                ((A >> 4) & 0x0f0f0f0fu) | (((C >> 4) & 0x03030303u) << 4),
-                ((B >> 4) & 0x0f0f0f0fu) | (((C >> 6) & 0x03030303u) << 4),
-            };
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t xw = (uint32_t)xb.qs[32 * n + 8 * i + 2 * lh + w];
-                s[i] = sdot4(q[i], xw, s[i]);
-                z[i] = sdot4(0x01010101u, xw, z[i]);
-            }
-        }
-        int isum = 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int g = 8 * n + 2 * i + (lh >> 1);
-            isum += (int)(int8_t)blk[192 + g] * (s[i] - 32 * z[i]);
-        }
-        isum = group8_sum(isum);
-        const uint32_t dbits = (uint32_t)blk[208] | ((uint32_t)blk[209] << 8);
-        acc = acc + (half_bits_to_float(dbits) * xb.d) * (float)isum;
-    }
-    return acc;
-}
-
 // Q6_K rows whose start has the same 4-byte alignment (0 or 2) in every lane
 // of the wave: 210-byte blocks alternate between the two, so each block takes
 // one scalar branch to a body with a compile-time shift instead of per-lane

@@ -17,9 +17,6 @@ constexpr int kDppRowHalfMirror = 0x141;
 constexpr int kDppRowMirror = 0x140;
 constexpr int kDppRowRor4 = 0x124;   // lane i reads lane (i - 4) mod 16 of its row
 constexpr int kDppRowRor8 = 0x128;
-constexpr int kDppRowRor12 = 0x12C;  // lane i reads lane i + 4
-constexpr int kDppRowRor14 = 0x12E;  // lane i reads lane i + 2
-constexpr int kDppRowRor15 = 0x12F;  // lane i reads lane i + 1
 constexpr int kDppRowBcast15 = 0x142;  // lane 15 of each row to the next row (row_mask picks rows)
 constexpr int kDppRowBcast31 = 0x143;  // lane 31 to rows 2 and 3
 
@@ -42,7 +39,6 @@ __device__ __forceinline__ double dpp_d(double v) {
 // formed from it (LDS staging bases, row pointers) stay scalar instead of
 // being formed per lane.
 __device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
-__device__ __forceinline__ int readlane_i(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
 __device__ __forceinline__ float readlane_f(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
@@ -97,42 +93,6 @@ __device__ __forceinline__ float wave_max_f(float v) {
     return fmaxf(fmaxf(a, b), fmaxf(c, d));
 }
 
-// Wave-uniform argmax of (value, index): larger value first, lower index on
-// ties; lanes without a candidate pass idx = INT_MAX.  NaN never wins.
-__device__ __forceinline__ bool better(float av, int ai, float bv, int bi) {
-    if (bi == 0x7fffffff) return ai != 0x7fffffff;
-    if (ai == 0x7fffffff) return false;
-    return av > bv || (av == bv && ai < bi);
-}
-template <int CTRL>
-__device__ __forceinline__ void argmax_step(float &v, int &i) {
-    const float ov = dpp_f<CTRL>(v);
-    const int oi = dpp_i<CTRL>(i);
-    if (better(ov, oi, v, i)) {
-        v = ov;
-        i = oi;
-    }
-}
-__device__ __forceinline__ void wave_argmax(float &v, int &i) {
-    argmax_step<kDppQuadXor1>(v, i);
-    argmax_step<kDppQuadXor2>(v, i);
-    argmax_step<kDppRowHalfMirror>(v, i);
-    argmax_step<kDppRowMirror>(v, i);
-    float bv = readlane_f(v, 0);
-    int bi = readlane_i(i, 0);
-#pragma unroll
-    for (int r = 16; r < 64; r += 16) {
-        const float ov = readlane_f(v, r);
-        const int oi = readlane_i(i, r);
-        if (better(ov, oi, bv, bi)) {
-            bv = ov;
-            bi = oi;
-        }
-    }
-    v = bv;
-    i = bi;
-}
-
 // ggml's x86 f32 dot fold for one row held by 16 lanes, lane l owning the
 // partial sums of accumulators l and l+16 (already added in-lane as the first
 // fold step): then +8 lanes, +4 lanes, pairs, halves.  Exact in lane 0 of the
@@ -143,27 +103,6 @@ __device__ __forceinline__ float row16_ggml_fold(float a) {
     a = a + dpp_f<kDppQuadXor1>(a);
     a = a + dpp_f<kDppQuadXor2>(a);
     return a;
-}
-
-// The same fold for a row held by 8 lanes, lane m owning accumulators
-// 4m..4m+3 (elements 32i + 4m + c): +16 accumulators is 4 lanes up, +8 is 2,
-// +4 is 1; lane 0 of the group then adds its four in the (0+1)+(2+3) order.
-// row_ror:n makes lane i read lane (i - n) mod 16, so reading lane i + j is
-// row_ror:(16 - j).  Exact in lane 0 of each aligned 8-lane group.
-__device__ __forceinline__ float group8_ggml_fold(float a0, float a1, float a2, float a3) {
-    a0 = a0 + dpp_f<kDppRowRor12>(a0);
-    a1 = a1 + dpp_f<kDppRowRor12>(a1);
-    a2 = a2 + dpp_f<kDppRowRor12>(a2);
-    a3 = a3 + dpp_f<kDppRowRor12>(a3);
-    a0 = a0 + dpp_f<kDppRowRor14>(a0);
-    a1 = a1 + dpp_f<kDppRowRor14>(a1);
-    a2 = a2 + dpp_f<kDppRowRor14>(a2);
-    a3 = a3 + dpp_f<kDppRowRor14>(a3);
-    a0 = a0 + dpp_f<kDppRowRor15>(a0);
-    a1 = a1 + dpp_f<kDppRowRor15>(a1);
-    a2 = a2 + dpp_f<kDppRowRor15>(a2);
-    a3 = a3 + dpp_f<kDppRowRor15>(a3);
-    return (a0 + a1) + (a2 + a3);
 }
 
 }  // namespace hoard
