@@ -96,12 +96,13 @@ struct DotGateUp {
 
 // -- down: rows of the unit's expert, y to its (token, slot) place -------------
 // 32 kRowSets rows per workgroup of four waves: a wave's rows (kRowSets an 8-lane
-// group) go from memory to registers whole, all their blocks in flight at once, while the workgroup forms
-// Q8_K(h) of the unit's pairs in LDS from h (a launch of its own for that took
-// 4 to 5 us); then each pair's dots from the registers.  Bound by the weight
-// stream's latency: Qwen3-30B at 4 tokens 10.6 us a launch, 16.4 with the tile
-// in LDS, one wave a workgroup and Q8_K(h) in a launch before it; at 16 tokens
-// 23.7 against 35.3, Qwen3-Next 31.9 against 31.6.
+// group) go from memory to registers whole, all their blocks in flight at once,
+// while the workgroup forms Q8_K(h) of the unit's pairs in LDS from h (a launch
+// of its own for that takes 4 to 5 us); then each pair's dots from the registers.
+// Bound by the weight stream's latency at few tokens, by the dots and the forming
+// at 16 (waves ready but not issued for 54 % of their cycles): Qwen3-30B at 4
+// tokens 10.7 us a launch, 16.4 with the tile in LDS, one wave a workgroup and
+// Q8_K(h) in a launch before it; at 16 tokens 28.4 against 27.7 and 4.9.
 constexpr int kRowSets = 2;  // row sets of 8 a wave takes of the down rows (four of the shortest rows measured slower)
 template <int T, int NBH>
 __device__ __forceinline__ void down_dots(const BatchedArgs &a, const Unit &w, Q8L *q8h) {

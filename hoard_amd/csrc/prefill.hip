@@ -615,10 +615,11 @@ struct GateUp<kTypeQ3K> {
 // token chunks into LDS (one buffer ahead) while each wave holds the next
 // super-block of its rows in registers; the gate waves hand their values to the
 // up waves through LDS, which form h and store it to hbuf[sorted pair][row].
-// Bound by its vector and matrix instructions, which share a SIMD's issue, and
-// the weight stream together: Qwen3-30B at 512 tokens 89 us a launch (226 MB).
-// Q3_K rows took 174 us at 512 tokens of 64 experts with a tile in LDS and every
-// wave loading its tokens' blocks, 120 here.
+// Bound by its vector and matrix instructions, which share a SIMD's issue (53 of
+// 88 us a launch without any load, Qwen3-30B at 512 tokens, 226 MB), and by loads
+// that arrive later than one super-block ahead covers (the other 35).  Q3_K rows
+// took 174 us at 512 tokens of 64 experts with a tile in LDS and every wave
+// loading its tokens' blocks, 115 here.
 // LDS: xs, two buffers of the unit's Q8_K block b; gx, the gate values [row
 // tile][chunk][row i][lane].  CH: the 16-token chunks of a unit.  kInt: the blocks'
 // sums are int16 (a batch that runs dots too).

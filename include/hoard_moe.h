@@ -135,10 +135,9 @@ int hoard_moe_decode(hoard_moe *h, int layer_begin, int layer_end, float *x_dev,
    token routed independently: the counterpart of ggml_mul_mat_id over the
    experts with per-token ids and the weighted sum over them
    (src/run_specloop.cpp:126-139, src/run_m1.cpp:97-108).  The (token, slot)
-   pairs are grouped by expert so each selected expert's weights are read once
-   per call (per 64 pairs above 32 tokens, where the pairs are sorted by
-   expert into 64-pair units), and the expert products run on per-token int8
-   dots or int8 MFMA; each token's result is the single-token
+   pairs are sorted by expert into units of at most 64 pairs, each of which reads
+   its expert's weights once, and the expert products run on per-token int8 dots
+   (experts with few pairs) or int8 MFMA; each token's result is the single-token
    hoard_moe_layer's bit for bit.  M > 512 returns HOARD_ERR_INVALID.  fx_dev, res_dev, out_dev:
    [M][n_embd], 16-byte aligned (out may alias res); sel_dev / w_dev ([M][n_used]) receive the
    routing when non-NULL.  The call's per-expert token histogram and unique

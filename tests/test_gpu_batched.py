@@ -1,7 +1,8 @@
-"""Batched expert stage (M tokens, grouped by expert, int8 MFMA) through the C ABI.
+"""Batched expert stage (M tokens, grouped by expert; per-token dots or int8 MFMA by
+the group's size) through the C ABI.
 
-Each token's result must be the single-token path's bit for bit (the MFMA
-produces the same integer sub-block sums), and match the oracle's batched
+Each token's result must be the single-token path's bit for bit (both produce
+the same integer sub-block sums), and match the oracle's batched
 layer (ggml's mul_mat_id semantics: every token routed and computed
 independently) to the parity bar.  The per-expert histogram must count the
 (token, slot) pairs of the call.
@@ -54,11 +55,11 @@ def test_batched_matches_single_token_and_oracle(orc, stage, M):
     assert stats.last_unique == int((counts > 0).sum())
 
 
-@pytest.mark.parametrize("M", [11, 12, 16])
+@pytest.mark.parametrize("M", [7, 8, 11, 12, 16])
 def test_batched_large_expert_groups(orc, stage, M):
     """M copies of one token's fx (each with its own residual) put all M tokens
-    in each of its k expert groups: 11 runs the per-token dot path at its
-    largest group, 12 and 16 the MFMA path."""
+    in each of its k expert groups (and a shared expert's): 7 runs the per-token
+    dots at their largest group, 8 to 16 one MFMA unit each."""
     shape, hl, st = stage
     fx1, _ = _tokens(shape, 1, 700 + M)
     _, res = _tokens(shape, M, 800 + M)
@@ -250,8 +251,8 @@ def test_pooled_verify_step_above_256_ids(orc):
 @pytest.mark.parametrize("M", [17, 32])
 def test_qwen35_verify_sizes_above_16(orc, M):
     """Qwen3.5's Q5_K routed down rows beside its Q6_K shared down in one down
-    launch, for groups of more than 16 tokens (the shared group holds all M, so
-    its tile takes a second 16-column MFMA pass): every token the single-token
+    launch, the shared group, which holds all M, in two MFMA units of 16 beside
+    the routed rows' dot units: every token the single-token
     path's bits, and the batch against the oracle."""
     from hoard_amd.runtime import MoEStage
     shape = W.QWEN35

@@ -1,5 +1,6 @@
-"""Batches of 17..512 tokens: up to 32 the verify-sized path's expert groups (per-token
-dots, or int8 MFMA in 16-column passes), above 32 the sorted-pair expert GEMM on int8 MFMA.
+"""Batches of 17..512 tokens: up to 32 routed and grouped in one launch, above 32 by a tiled
+router GEMM and a pair sort; the expert products on per-token dots or on int8 MFMA units of
+16, 32 or 64 pairs by each expert's pairs.
 
 The counterpart of ggml_mul_mat_id over all T prompt tokens (src/run_m1.cpp:93-108).
 Each token's result must be the single-token path's bit for bit (the folded MFMA
@@ -75,8 +76,8 @@ def test_prefill_matches_single_token_and_oracle(orc, stage, M):
                          ids=["20x1", "30x2", "32x1", "200x1", "300x3"])
 def test_prefill_large_expert_groups(orc, stage, M, same):
     """Tokens sharing a few hiddens.  Up to 32 tokens the groups (15, 20 or 32
-    tokens) run on MFMA in one or two 16-column passes over each weight tile;
-    above, groups of 100-300 tokens are cut into several 64-pair units each."""
+    tokens) run on MFMA, in units of 16 (over 64 experts of 16 or 32); above,
+    groups of 100-300 tokens are cut into several units of 32 or 64 each."""
     shape, hl, st = stage
     fx, res = _tokens(shape, M, 3000 + M, same=same)
     print(f"prefill {shape.name} M={M}, {same} distinct hiddens", flush=True)
